@@ -38,6 +38,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "flash_sched.hpp"
 #include "kernels.hpp"
 #include "plan.hpp"
 
@@ -162,6 +163,7 @@ struct BwdArgs {
                        // (d columns dr .. D-1 load as zeros and are not stored)
     const int* cu_q;   // variable length (nullptr: dense), as in the forward
     const int* cu_k;
+    int B;             // batch entries (sequences)
     int H, Hkv;
     int total_q, total_k;
     // Grouped-query split of the dK/dV kernel (dense layout; gsplit = 1: none): part gp of
@@ -431,12 +433,16 @@ flash_bwd_dq_kernel(BwdArgs p) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, c32 = lane & 31;
-    const int bh = blockIdx.x;
-    const int qb_idx = CAUSAL ? (p.nqb - 1 - (int)blockIdx.y) : (int)blockIdx.y;
+    // Which query block of which (batch, head): see flash_sched.hpp.
+    int col;
+    const int64_t row = flash_split_id(flash_linear_id(), p.cu_q ? p.H : p.B * p.H, &col);
+    int b = col / p.H, qb_idx = CAUSAL ? p.nqb - 1 - (int)row : (int)row;
+    if (p.cu_q && !varlen_item<false, CAUSAL, FbGeom<D>::BLOCK_Q>(
+                      p.cu_q, p.cu_k, p.B, p.total_q, p.total_k, p.Sq, p.Sk, row, &b, &qb_idx))
+        return;
     const int q0 = qb_idx * FbGeom<D>::BLOCK_Q;
     const int qw = q0 + wave * FB_ROWS;
-    const SeqGeo G = seq_geo<D>(p, bh / p.H, bh % p.H);
-    if (q0 >= G.Sq) return;
+    const SeqGeo G = seq_geo<D>(p, b, col % p.H);
     const int Sq = G.Sq, Sk = G.Sk;
     const int qrow = qw + c32;
 
@@ -657,12 +663,21 @@ flash_bwd_dkdv_kernel(BwdArgs p) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, c32 = lane & 31;
-    const int bkv = blockIdx.x;
-    const int b = bkv / p.Hkv, j = bkv % p.Hkv;
-    const int k0 = (int)blockIdx.y * FbKv<D>::BLOCK;  // causal: lower key blocks are heavier, and first
+    // Which key block of which (batch, key/value head), and which of its column and group
+    // parts z: the parts of a block are neighbours, so that heavier blocks still go first
+    // (causal: lower key blocks are heavier); see flash_sched.hpp.
+    int col, z;
+    const int64_t row_z =
+        flash_split_id(flash_linear_id(), p.cu_q ? p.Hkv : p.B * p.Hkv, &col);
+    const int64_t row = flash_split_id(row_z, gridDim.z, &z);
+    int b = col / p.Hkv, kblk = (int)row;
+    if (p.cu_q && !varlen_item<true, CAUSAL, FbKv<D>::BLOCK>(
+                      p.cu_q, p.cu_k, p.B, p.total_q, p.total_k, p.Sq, p.Sk, row, &b, &kblk))
+        return;
+    const int j = col % p.Hkv;
+    const int k0 = kblk * FbKv<D>::BLOCK;
     const int kw = k0 + wave * FbKv<D>::ROWS;
     const SeqGeo G0 = seq_geo<D>(p, b, j * p.group);
-    if (k0 >= G0.Sk) return;
     const int Sq = G0.Sq, Sk = G0.Sk;
 
     f16x8 kf[FbKv<D>::KB][C::NDS], vf[FbKv<D>::KB][C::NDS];
@@ -678,7 +693,7 @@ flash_bwd_dkdv_kernel(BwdArgs p) {
     // (heads g_lo .. g_lo + ng - 1: the whole group, or one part of a grouped-query split).
     // Head gi's rows start at q_base0 + gi * qh (Q/dO elements) and r_base0 + gi * rh
     // (statistics).
-    const int gp = (int)blockIdx.z / FbKv<D>::DSPLIT;
+    const int gp = z / FbKv<D>::DSPLIT;
     const int g_lo = gp * p.gper;
     const int ng = max(0, min(p.group, g_lo + p.gper) - g_lo);
     const int Tq = (Sq + FB_T - 1) / FB_T;
@@ -701,7 +716,7 @@ flash_bwd_dkdv_kernel(BwdArgs p) {
 
     constexpr int NDBO = FbKv<D>::NDB_OUT;
     // first d block of this workgroup's dK, dV columns
-    const int db0 = ((int)blockIdx.z % FbKv<D>::DSPLIT) * NDBO;
+    const int db0 = (z % FbKv<D>::DSPLIT) * NDBO;
     f32x16 dk[FbKv<D>::KB][NDBO], dv[FbKv<D>::KB][NDBO];
 #pragma unroll
     for (int kb = 0; kb < FbKv<D>::KB; ++kb)
@@ -799,8 +814,11 @@ template <int D>
 void launch_bwd_d(BwdArgs a, int B, bool causal, hipStream_t stream) {
     a.nqb = ceil_div(a.Sq, FbGeom<D>::BLOCK_Q);
     const dim3 bq(FbGeom<D>::WQ * kWave), bk(FB_WAVES_KV * kWave);
-    const dim3 gq(B * a.H, a.nqb);
-    const dim3 gk(B * a.Hkv, ceil_div(a.Sk, FbKv<D>::BLOCK), FbKv<D>::DSPLIT * a.gsplit);
+    const dim3 gq(B * a.H, a.cu_q ? varlen_grid_y(B, a.total_q, a.Sq, FbGeom<D>::BLOCK_Q) : a.nqb);
+    const dim3 gk(B * a.Hkv,
+                  a.cu_q ? varlen_grid_y(B, a.total_k, a.Sk, FbKv<D>::BLOCK)
+                         : ceil_div(a.Sk, FbKv<D>::BLOCK),
+                  FbKv<D>::DSPLIT * a.gsplit);
     // The dQ kernel writes the row statistics the dK/dV kernel reads: same stream, in order.
     // An empty side (no query or no key rows) launches nothing for it; with no query rows
     // the dK/dV kernel still runs and stores zeros.
@@ -885,6 +903,7 @@ hipError_t launch_flash_bwd(const FlashBwdLaunch& f, hipStream_t stream) {
     a.dr = f.D;
     a.cu_q = f.cu_q;
     a.cu_k = f.cu_k;
+    a.B = f.B;
     a.H = f.H;
     a.Hkv = f.Hkv;
     a.total_q = f.total_q;

@@ -31,6 +31,7 @@
 //    zeros (no score or output contribution) and never stored.  D = 256 runs 4 waves of
 //    the whole register file each and a 2-deep ring (see FaCfg).
 #include "common.hpp"
+#include "flash_sched.hpp"
 #include "kernels.hpp"
 #include "plan.hpp"
 
@@ -55,6 +56,7 @@ struct FlashArgs {
     // cannot send a load or store outside the tensors.
     const int* cu_q;
     const int* cu_k;
+    int B;             // sequences
     int H, Hkv;
     int total_q, total_k;
     // Optional per-row log-sum-exp of the scaled scores (natural log; +inf for a row with
@@ -321,8 +323,20 @@ flash_fwd_kernel(FlashArgs p) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, c32 = lane & 31;
-    const int bh = blockIdx.x;
-    const int qb_idx = CAUSAL ? (p.nqb - 1 - (int)blockIdx.y) : (int)blockIdx.y;
+    // Which query block of which (batch, head): see flash_sched.hpp.
+    int bh = blockIdx.x, qb_idx = blockIdx.y;
+    if (p.cu_q) {
+        int b, head;
+        const int64_t item = flash_split_id(flash_linear_id(), p.H, &head);
+        if (!varlen_item<false, CAUSAL, C::BQ>(p.cu_q, p.cu_k, p.B, p.total_q, p.total_k, p.Sq, p.Sk,
+                                               item, &b, &qb_idx))
+            return;
+        bh = b * p.H + head;
+    } else if (CAUSAL && !p.kv_chunk) {
+        qb_idx = p.nqb - 1 - (int)flash_split_id(flash_linear_id(), gridDim.x, &bh);
+    } else if (CAUSAL) {
+        qb_idx = p.nqb - 1 - qb_idx;
+    }
     const int q0 = qb_idx * C::BQ;
     const int qw = q0 + wave * FA_WQ;
     const float c = p.scale_log2;
@@ -354,7 +368,6 @@ flash_fwd_kernel(FlashArgs p) {
         k_base = (int64_t)(bh / p.group) * Sk * p.dr;
         lse_base = (int64_t)bh * Sq;
     }
-    if (q0 >= Sq) return;  // a query block past this sequence (variable length): no work
     const f16* Qb = p.Q + q_base;
     const f16* Kb = p.K + k_base;
     const f16* Vb = p.V + k_base;
@@ -578,7 +591,8 @@ flash_combine_kernel(const float* o_part, const float* ml_part, int split, int64
 template <int D>
 void launch_d(FlashArgs a, int BH, bool causal, hipStream_t stream) {
     a.nqb = ceil_div(a.Sq, FaCfg<D>::BQ);
-    dim3 grid(BH, a.nqb, a.kv_chunk ? ceil_div(a.Sk, a.kv_chunk) : 1);
+    const int rows = a.cu_q ? varlen_grid_y(a.B, a.total_q, a.Sq, FaCfg<D>::BQ) : a.nqb;
+    dim3 grid(BH, rows, a.kv_chunk ? ceil_div(a.Sk, a.kv_chunk) : 1);
     const dim3 block(FaCfg<D>::WAVES * kWave);
     if (causal)
         hipLaunchKernelGGL((flash_fwd_kernel<D, true>), grid, block, 0, stream, a);
@@ -600,6 +614,7 @@ hipError_t launch_flash_fwd(const FlashLaunch& f, hipStream_t stream) {
     a.dr = f.D;
     a.cu_q = f.cu_q;
     a.cu_k = f.cu_k;
+    a.B = f.B;
     a.H = f.H;
     a.Hkv = f.Hkv;
     a.total_q = f.total_q;
