@@ -126,6 +126,22 @@ int wmma_gemm_f16f32(const void* A, int64_t lda, const void* B, int64_t ldb,
                      void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * wmma_gemm_f16f32 on operands as a row-major program's views hold them: trans_a non-zero
+ * says that A is stored [K][M] (A[m][k] at A[k * lda + m], lda >= M), trans_b that B is
+ * stored [N][K] (ldb >= K) -- a linear layer's weight, or the transposes of its backward.
+ * At most one of them.  The kernels read either storage order directly.  The workspace is
+ * sized for exactly these operands (their alignment decides what has to be copied); a
+ * transposed operand whose rows break 16-byte vectors needs it.  No counterpart in the
+ * reference, which copies a transposed input first (wmma_gemm.hip:1440).
+ */
+size_t wmma_gemm_view_workspace_size(const void* A, int64_t lda, int trans_a, const void* B,
+                                     int64_t ldb, int trans_b, int M, int N, int K, int tile_cfg);
+int wmma_gemm_f16f32_view(const void* A, int64_t lda, int trans_a, const void* B, int64_t ldb,
+                          int trans_b, const float* C_in, int64_t ldc_in, float* C_out, int64_t ldc,
+                          int M, int N, int K, float alpha, float beta, int tile_cfg,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Allocation-free variant of wmma_gemm_f16f32: the same computation and kernels, but no
  * workspace argument -- the split-K partial sums go to a device array inside this library
  * (wmma_gemm_noalloc_scratch_bytes() = 32 MiB per GPU, held until the process ends), so the

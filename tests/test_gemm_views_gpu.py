@@ -1,0 +1,96 @@
+"""GEMM operands read in the storage order of a view: transposes and column slices."""
+import pytest
+import torch
+
+from oracle import gemm as og
+from tests.conftest import report
+
+pytestmark = pytest.mark.gpu
+
+BAR = 1e-4  # max |got - ref| / max |ref|: fp32 sums on both sides
+
+
+def _close(got, ref):
+    err = (got.cpu() - ref).abs().max() / ref.abs().max().clamp_min(1e-30)
+    assert err <= BAR, float(err)
+
+
+def _inputs(m, n, k, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(m, k, generator=g).half(), torch.randn(k, n, generator=g).half()
+
+
+def _stored_transposed(x):
+    return x.t().contiguous().cuda().t()
+
+
+# Tile edges and remainders in each dimension; the skinny kernel's row blocks, column counts
+# and K rounds (8 x 128 per workgroup); rows that are not whole 16-byte vectors, which the
+# skinny kernel reads in place (odd K: rows start at odd elements) and the others copy.
+SHAPES = [
+    (1, 16, 8), (1, 77, 30), (3, 515, 1), (16, 4096, 1024), (16, 300, 1032), (5, 983, 589),
+    (17, 64, 2051), (31, 1000, 2050), (32, 2048, 4096), (33, 96, 72), (64, 64, 64), (65, 136, 200),
+    (127, 250, 333), (256, 256, 256), (257, 264, 520), (787, 983, 589), (1000, 4100, 1032),
+]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("which", ["a", "b", "ab"])
+def test_transposed_views(wo, m, n, k, which):
+    report("transposed_views", m=m, n=n, k=k, which=which)
+    A, B = _inputs(m, n, k)
+    a = _stored_transposed(A) if "a" in which else A.cuda()
+    b = _stored_transposed(B) if "b" in which else B.cuda()
+    ref = og.gemm_ref(A, B)
+    got = wo.matmul(a, b)
+    _close(got, ref)
+    assert torch.equal(got, wo.matmul(a, b))
+    C = torch.randn(m, n, generator=torch.Generator().manual_seed(3))
+    _close(wo.gemm(a, b, 2.0, 0.5, C.cuda()), og.gemm_ref(A, B, 2.0, 0.5, C))
+    Ci = C.cuda()
+    wo.gemm_inplace(a, b, Ci, 2.0, 0.5)
+    _close(Ci, og.gemm_ref(A, B, 2.0, 0.5, C))
+
+
+@pytest.mark.parametrize("tile", range(6))
+@pytest.mark.parametrize("which", ["a", "b"])
+def test_transposed_every_tile(wo, tile, which):
+    m, n, k = 520, 328, 136
+    report("transposed_every_tile", tile=tile, which=which)
+    A, B = _inputs(m, n, k, 1)
+    a = _stored_transposed(A) if which == "a" else A.cuda()
+    b = _stored_transposed(B) if which == "b" else B.cuda()
+    # the same products in the same order as on contiguous copies
+    assert torch.equal(wo.matmul_tiled(a, b, tile), wo.matmul_tiled(A.cuda(), B.cuda(), tile))
+    _close(wo.matmul_tiled(a, b, tile), og.gemm_ref(A, B))
+
+
+@pytest.mark.parametrize("off", [0, 1, 2, 3, 8])
+@pytest.mark.parametrize("m", [4, 20, 150])
+def test_sliced_views(wo, m, off):
+    # Slices keep their parent's stride: rows at any element offset, and a parent whose row
+    # length is odd, plain and transposed.
+    report("sliced_views", m=m, off=off)
+    g = torch.Generator().manual_seed(2)
+    X, W = torch.randn(m, 521, generator=g).half(), torch.randn(512, 331, generator=g).half()
+    Wt = torch.randn(300, 533, generator=g).half()
+    a, A = X.cuda()[:, off:off + 512], X[:, off:off + 512]
+    b, B = W.cuda()[:, off:off + 300], W[:, off:off + 300]
+    _close(wo.matmul(a, b), og.gemm_ref(A, B))
+    bt, Bt = Wt.cuda()[:, off:off + 512].t(), Wt[:, off:off + 512].t()
+    _close(wo.matmul(a, bt), og.gemm_ref(A, Bt))
+
+
+def test_other_strides_are_copied(wo):
+    # Steps, expanded rows and strides past the kernels' 32-bit offsets.
+    A, B = _inputs(48, 40, 64, 4)
+    ref = og.gemm_ref(A, B)
+    wide = torch.zeros(48, 128, dtype=torch.half, device="cuda")
+    wide[:, ::2] = A.cuda()
+    _close(wo.matmul(wide[:, ::2], B.cuda()), ref)
+    row = torch.randn(1, 64).half()
+    _close(wo.matmul(row.cuda().expand(48, 64), B.cuda()), og.gemm_ref(row.expand(48, 64), B))
+    far = torch.empty(2 * 5000000, dtype=torch.half, device="cuda").as_strided((2, 64), (5000000, 1))
+    far.copy_(A[:2])
+    _close(wo.matmul(far, B.cuda()), ref[:2])
+    _close(wo.matmul(B.cuda().t(), far.t()), og.gemm_ref(B.t(), A[:2].t()))

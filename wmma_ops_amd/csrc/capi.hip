@@ -63,10 +63,13 @@ size_t round256(size_t x) { return (x + 255) & ~(size_t)255; }
 // Workspace bytes, behind the split-K partial sums, for zero-padded dense copies of the
 // operands whose rows break 16-byte vectors: A [M][K8] when `a`, B [K][N8] when `b` (K8, N8
 // rounded up to 8), each copy 256-byte aligned (256 bytes of slack align the first).
-size_t repack_bytes(int M, int N, int K, bool a, bool b) {
+size_t repack_bytes(int M, int N, int K, bool a, bool b, GemmLayout layout = GemmLayout::NN) {
     if ((!a && !b) || M <= 0 || N <= 0 || K <= 0) return 0;
-    const size_t K8 = ((size_t)K + 7) & ~(size_t)7, N8 = ((size_t)N + 7) & ~(size_t)7;
-    return 256 + (a ? round256((size_t)M * K8 * 2) : 0) + (b ? round256((size_t)K * N8 * 2) : 0);
+    const size_t M8 = ((size_t)M + 7) & ~(size_t)7, K8 = ((size_t)K + 7) & ~(size_t)7,
+                 N8 = ((size_t)N + 7) & ~(size_t)7;
+    const size_t ab = layout == GemmLayout::TN ? (size_t)K * M8 : (size_t)M * K8;
+    const size_t bb = layout == GemmLayout::NT ? (size_t)N * K8 : (size_t)K * N8;
+    return 256 + (a ? round256(ab * 2) : 0) + (b ? round256(bb * 2) : 0);
 }
 
 }  // namespace
@@ -192,15 +195,53 @@ size_t wmma_gemm_workspace_size(int M, int N, int K, int tile_cfg) {
            repack_bytes(M, N, K, K % 8 != 0, N % 8 != 0 && p.kernel != WMMA_KERNEL_SKINNY);
 }
 
+static GemmLayout layout_of(int trans_a, int trans_b) {
+    return trans_a ? GemmLayout::TN : (trans_b ? GemmLayout::NT : GemmLayout::NN);
+}
+
+// Which operands of a GEMM the kernel of `plan` can read only as a copy with 16-byte rows.
+// The stored rows are K long, or M of a transposed A and N of a B as it is.
+struct RowCheck {
+    bool a_vec, b_vec;    // whole 16-byte vectors, as they are
+    bool a_copy, b_copy;  // read from a copy
+};
+static RowCheck check_rows(const wmma_gemm_plan& plan, GemmLayout layout, const void* A, int64_t lda,
+                           const void* B, int64_t ldb, int M, int N, int K) {
+    RowCheck r;
+    r.a_vec = (layout == GemmLayout::TN ? M : K) % 8 == 0 && lda % 8 == 0 && aligned16(A);
+    r.b_vec = (layout == GemmLayout::NT ? K : N) % 8 == 0 && ldb % 8 == 0 && aligned16(B);
+    const bool skinny = plan.kernel == WMMA_KERNEL_SKINNY;
+    if (skinny && layout == GemmLayout::NT) {  // reads both in place at any alignment
+        r.a_copy = r.b_copy = false;
+        return r;
+    }
+    // The skinny kernel streams B once, so there a 4-byte-aligned B is read in place by
+    // dword-aligned 16-byte loads (a copy would triple its traffic).
+    r.a_copy = !r.a_vec;
+    r.b_copy = !r.b_vec && !(skinny && (reinterpret_cast<uintptr_t>(B) & 3u) == 0);
+    return r;
+}
+
+size_t wmma_gemm_view_workspace_size(const void* A, int64_t lda, int trans_a, const void* B,
+                                     int64_t ldb, int trans_b, int M, int N, int K, int tile_cfg) {
+    if (trans_a && trans_b) return 0;
+    const GemmLayout layout = layout_of(trans_a, trans_b);
+    wmma_gemm_plan p{};
+    if (make_layout_plan(layout, M, N, K, tile_cfg, current_cus(), SIZE_MAX, &p) != WMMA_OK)
+        return 0;
+    const RowCheck r = check_rows(p, layout, A, lda, B, ldb, M, N, K);
+    return p.workspace_bytes + repack_bytes(M, N, K, r.a_copy, r.b_copy, layout);
+}
+
 // Shared checks and launch of wmma_gemm_f16f32 / wmma_gemm_f16f32_plan /
-// wmma_gemm_f16f32_noalloc.  `plan` is NULL for the planner's own plan (tile_cfg), else an
+// wmma_gemm_f16f32_noalloc / wmma_gemm_f16f32_view.  `plan` is NULL for the planner's own plan (tile_cfg), else an
 // explicit plan for exactly this shape.  use_scratch: the split-K partials go to the
 // library's own scratch array (the caller passes no workspace).
 static int gemm_run(const void* A, int64_t lda, const void* B, int64_t ldb, const float* C_in,
                     int64_t ldc_in, float* C_out, int64_t ldc, int M, int N, int K, float alpha,
                     float beta, int tile_cfg, const wmma_gemm_plan* explicit_plan,
                     void* workspace, size_t workspace_bytes, void* stream,
-                    bool use_scratch = false) {
+                    bool use_scratch = false, GemmLayout layout = GemmLayout::NN) {
     if (M < 0 || N < 0 || K < 0) return fail(WMMA_ERR_INVALID_ARG, "negative GEMM dimension");
     if (tile_cfg < WMMA_TILE_AUTO || tile_cfg >= WMMA_TILE_COUNT)
         return fail(WMMA_ERR_INVALID_ARG,
@@ -214,11 +255,17 @@ static int gemm_run(const void* A, int64_t lda, const void* B, int64_t ldb, cons
         return fail(WMMA_ERR_INVALID_ARG, "ldc_in (%lld) < N (%d)", (long long)ldc_in, N);
     if (K > 0) {
         if (!A || !B) return fail(WMMA_ERR_INVALID_ARG, "A or B is NULL");
-        if (lda < K) return fail(WMMA_ERR_INVALID_ARG, "lda (%lld) < K (%d)", (long long)lda, K);
-        if (ldb < N) return fail(WMMA_ERR_INVALID_ARG, "ldb (%lld) < N (%d)", (long long)ldb, N);
-        // 32-bit buffer offsets: one 256-row A tile and one 64-row B stage must fit (also
-        // with the leading dimensions of repacked copies, at most 7 elements longer).
-        if ((256 + 1) * (lda + 7) * 2 > kMaxOffset || (64 + 1) * (ldb + 7) * 2 > kMaxOffset ||
+        const bool ta = layout == GemmLayout::TN, tb = layout == GemmLayout::NT;
+        if (lda < (ta ? M : K))
+            return fail(WMMA_ERR_INVALID_ARG, "lda (%lld) < %s (%d)", (long long)lda, ta ? "M" : "K",
+                        ta ? M : K);
+        if (ldb < (tb ? K : N))
+            return fail(WMMA_ERR_INVALID_ARG, "ldb (%lld) < %s (%d)", (long long)ldb, tb ? "K" : "N",
+                        tb ? K : N);
+        // 32-bit buffer offsets: one 256-row A tile and one 64-row B stage (a 256-row tile of
+        // a transposed B) must fit (also with the leading dimensions of repacked copies, at most 7 elements longer).
+        if ((256 + 1) * (lda + 7) * 2 > kMaxOffset ||
+            ((tb ? 256 : 64) + 1) * (ldb + 7) * 2 > kMaxOffset ||
             (int64_t)kSkinnyMaxMWide * (lda + 7) * 2 > kMaxOffset)
             return fail(WMMA_ERR_UNSUPPORTED, "leading dimension too large for 32-bit offsets");
     }
@@ -242,7 +289,7 @@ static int gemm_run(const void* A, int64_t lda, const void* B, int64_t ldb, cons
             return fail(WMMA_ERR_INVALID_ARG, "plan does not describe this shape (make it with "
                                               "wmma_gemm_plan_custom or wmma_gemm_plan_make)");
     } else {
-        int rc = make_plan_within(M, N, K, tile_cfg, current_cus(), plan_cap, &plan);
+        int rc = make_layout_plan(layout, M, N, K, tile_cfg, current_cus(), plan_cap, &plan);
         if (rc != WMMA_OK) return fail(rc, "planner rejected the shape");
     }
     int scratch_dev = -1;
@@ -271,48 +318,55 @@ static int gemm_run(const void* A, int64_t lda, const void* B, int64_t ldb, cons
         if ((reinterpret_cast<uintptr_t>(workspace) & 3u) != 0)
             return fail(WMMA_ERR_MISALIGNED, "workspace must be 4-byte aligned");
     }
-    // An operand whose rows break 16-byte vectors (K or N not a multiple of 8, a leading
-    // dimension that is not, or an address off 16 bytes) is copied into a zero-padded dense
+    // An operand whose stored rows break 16-byte vectors (a length or leading dimension that
+    // is not a multiple of 8, an address off 16 bytes) is copied into a zero-padded dense
     // buffer behind the partial sums when the workspace holds it, and the vector kernels
     // run on the copy; without that room (or from the allocation-free entry point) the
-    // element-wise kernels read it in place.  The skinny kernel streams B once, so there a
-    // 4-byte-aligned B is read in place by dword-aligned 16-byte loads instead (a copy
-    // would triple its traffic).  The padding is zero and every kernel masks rows and
-    // columns at M, N and K, so the result is the same either way.
-    bool a_vec = K % 8 == 0 && lda % 8 == 0 && aligned16(A);
-    bool b_vec = N % 8 == 0 && ldb % 8 == 0 && aligned16(B);
-    const bool skinny = plan.kernel == WMMA_KERNEL_SKINNY;
+    // element-wise kernels read it in place, except that they read no transposed operand.
+    // The padding is zero and every kernel masks rows and columns at M, N and K, so the
+    // result is the same either way.
+    RowCheck rows = check_rows(plan, layout, A, lda, B, ldb, M, N, K);
     const bool b_al4 = (reinterpret_cast<uintptr_t>(B) & 3u) == 0;
-    const bool b_copy = !b_vec && !(skinny && b_al4);
-    if (K > 0 && (!a_vec || b_copy) && !use_scratch && workspace &&
-        workspace_bytes >= plan.workspace_bytes + repack_bytes(M, N, K, !a_vec, b_copy)) {
+    if (K > 0 && (rows.a_copy || rows.b_copy)) {
+        const bool room =
+            !use_scratch && workspace &&
+            workspace_bytes >= plan.workspace_bytes +
+                                   repack_bytes(M, N, K, rows.a_copy, rows.b_copy, layout);
+        if (!room && layout != GemmLayout::NN)
+            return fail(WMMA_ERR_WORKSPACE,
+                        "a transposed GEMM whose rows break 16-byte vectors needs a workspace of "
+                        "wmma_gemm_view_workspace_size bytes");
         const hipStream_t st = static_cast<hipStream_t>(stream);
         unsigned char* dst = reinterpret_cast<unsigned char*>(
             round256(reinterpret_cast<uintptr_t>(workspace) + plan.workspace_bytes));
-        if (!a_vec) {
-            const int64_t K8 = ((int64_t)K + 7) & ~(int64_t)7;
-            if (int rc = hip_status(launch_gemm_repack(A, lda, M, K, dst, st), "gemm repack A"))
-                return rc;
-            A = dst;
-            lda = K8;
-            a_vec = true;
-            dst += round256((size_t)M * (size_t)K8 * 2);
+        // The copy of an operand stored as n rows of `len`; its new leading dimension in *ld.
+        auto copy = [&](const void*& src, int64_t* ld, int n, int len, const char* what) -> int {
+            const int64_t len8 = ((int64_t)len + 7) & ~(int64_t)7;
+            if (int rc = hip_status(launch_gemm_repack(src, *ld, n, len, dst, st), what)) return rc;
+            src = dst;
+            *ld = len8;
+            dst += round256((size_t)n * (size_t)len8 * 2);
+            return WMMA_OK;
+        };
+        if (room && rows.a_copy) {
+            const bool ta = layout == GemmLayout::TN;
+            if (int rc = copy(A, &lda, ta ? K : M, ta ? M : K, "gemm repack A")) return rc;
+            rows.a_vec = true;
         }
-        if (b_copy) {
-            const int64_t N8 = ((int64_t)N + 7) & ~(int64_t)7;
-            if (int rc = hip_status(launch_gemm_repack(B, ldb, K, N, dst, st), "gemm repack B"))
-                return rc;
-            B = dst;
-            ldb = N8;
-            b_vec = true;
+        if (room && rows.b_copy) {
+            const bool tb = layout == GemmLayout::NT;
+            if (int rc = copy(B, &ldb, tb ? N : K, tb ? K : N, "gemm repack B")) return rc;
+            rows.b_vec = true;
         }
     }
-    const bool vec = K > 0 && a_vec && b_vec;
+    const bool vec = K > 0 && rows.a_vec && rows.b_vec;
     // One launch of plan `pl` on the sub-GEMM whose output starts at row r0, column c0.
     auto launch_part = [&](const wmma_gemm_plan& pl, int r0, int c0, int Mp, int Np) {
         GemmLaunch g{};
-        g.A = static_cast<const uint16_t*>(A) + (int64_t)r0 * lda;
-        g.B = static_cast<const uint16_t*>(B) + c0;
+        g.trans_a = layout == GemmLayout::TN && K > 0;
+        g.trans_b = layout == GemmLayout::NT && K > 0;
+        g.A = static_cast<const uint16_t*>(A) + (g.trans_a ? r0 : (int64_t)r0 * lda);
+        g.B = static_cast<const uint16_t*>(B) + (g.trans_b ? (int64_t)c0 * ldb : c0);
         g.C_in = use_c ? C_in + (int64_t)r0 * ldc_in + c0 : nullptr;
         g.C_out = C_out + (int64_t)r0 * ldc + c0;
         g.workspace = workspace;
@@ -326,7 +380,7 @@ static int gemm_run(const void* A, int64_t lda, const void* B, int64_t ldb, cons
         g.alpha = alpha;
         g.beta = beta;
         g.vec = vec;
-        g.skinny_b = pl.kernel == WMMA_KERNEL_SKINNY && !vec && K > 0 && a_vec && b_al4
+        g.skinny_b = pl.kernel == WMMA_KERNEL_SKINNY && !vec && K > 0 && rows.a_vec && b_al4
                          ? (ldb % 2 == 0 ? 2 : 3)
                          : 0;
         g.plan = pl;
@@ -338,15 +392,15 @@ static int gemm_run(const void* A, int64_t lda, const void* B, int64_t ldb, cons
         // reuse the workspace): the bulk on whole waves of 256x256 tiles, then the edge with
         // the plan the planner gives its own shape.  Column offsets keep 16-byte alignment
         // (edge_at is a multiple of 256) and 4-byte alignment of B for the skinny kernel.
-        const bool rows = plan.edge_dim == WMMA_EDGE_ROWS;
+        const bool by_rows = plan.edge_dim == WMMA_EDGE_ROWS;
         const int at = plan.edge_at;
         wmma_gemm_plan edge{};
-        if (make_plan_within(rows ? M - at : M, rows ? N : N - at, K, WMMA_TILE_AUTO,
+        if (make_layout_plan(layout, by_rows ? M - at : M, by_rows ? N : N - at, K, WMMA_TILE_AUTO,
                              current_cus(), plan_cap, &edge) != WMMA_OK ||
             edge.edge_dim != WMMA_EDGE_NONE || edge.workspace_bytes > plan.workspace_bytes)
             return fail(WMMA_ERR_INVALID_ARG, "inconsistent two-part plan");
-        if (int rc = launch_part(plan, 0, 0, rows ? at : M, rows ? N : at)) return rc;
-        return rows ? launch_part(edge, at, 0, M - at, N) : launch_part(edge, 0, at, M, N - at);
+        if (int rc = launch_part(plan, 0, 0, by_rows ? at : M, by_rows ? N : at)) return rc;
+        return by_rows ? launch_part(edge, at, 0, M - at, N) : launch_part(edge, 0, at, M, N - at);
     };
     const int rc = launch_all();
     if (scratch_dev >= 0 && scratch_ordered) {
@@ -362,6 +416,16 @@ int wmma_gemm_f16f32(const void* A, int64_t lda, const void* B, int64_t ldb, con
                      void* stream) {
     return gemm_run(A, lda, B, ldb, C_in, ldc_in, C_out, ldc, M, N, K, alpha, beta, tile_cfg,
                     nullptr, workspace, workspace_bytes, stream);
+}
+
+int wmma_gemm_f16f32_view(const void* A, int64_t lda, int trans_a, const void* B, int64_t ldb,
+                          int trans_b, const float* C_in, int64_t ldc_in, float* C_out, int64_t ldc,
+                          int M, int N, int K, float alpha, float beta, int tile_cfg,
+                          void* workspace, size_t workspace_bytes, void* stream) {
+    if (trans_a && trans_b)
+        return fail(WMMA_ERR_UNSUPPORTED, "at most one of A and B may be transposed");
+    return gemm_run(A, lda, B, ldb, C_in, ldc_in, C_out, ldc, M, N, K, alpha, beta, tile_cfg,
+                    nullptr, workspace, workspace_bytes, stream, false, layout_of(trans_a, trans_b));
 }
 
 int wmma_gemm_f16f32_noalloc(const void* A, int64_t lda, const void* B, int64_t ldb,

@@ -13,6 +13,12 @@
 //                           read while the last MFMAs of this one run.  Workgroup ids are
 //                           re-mapped per XCD and walked in grouped order so each XCD's L2
 //                           sees neighbouring tiles.
+//                           Either operand may also be stored transposed (a linear layer's
+//                           [out, in] weight, the transposes of its backward): both storage
+//                           orders have a conflict-free LDS layout and read, so no copy is
+//                           made.  2048 x 4096 x 4096, y = x W^T, dx = dy W, dW = dy^T x:
+//                           350 us with the transposes copied first, 240 us read in place;
+//                           4096^3 takes 124 us in every layout.
 //  * gemm_tiled_kernel   -- generic path for unaligned shapes (any M, N, K): element-wise
 //                           masked loads, B transposed in registers (8x8 blocks, v_perm) on
 //                           its way into a double-buffered LDS stage.
@@ -20,6 +26,10 @@
 //                           loads, computes C^T = B^T A^T with MFMA 16x16x32 so the wide
 //                           N dimension fills the matrix rows, reduces its four waves'
 //                           K slices in LDS.
+//  * gemm_skinny_nt_kernel- M <= 32 with B stored [N][K]: K-contiguous rows of both operands
+//                           straight into MFMA operands, usually without a K split
+//                           (M = 1, N = K = 4096: 9.4 us with the weight in HBM, 5.1 TB/s
+//                           past the launch; a copy and gemm_skinny_kernel took 45 us).
 //  * splitk_reduce_kernel-- sums split-K partials in a fixed order and applies the
 //                           alpha/beta epilogue (reading C_in once).
 //
@@ -54,7 +64,7 @@ struct GemmArgs {
 };
 
 // ------------------------------------------------------------------------------------
-// LDS-DMA MFMA kernel (A and B 16-byte aligned, K and N multiples of 8)
+// LDS-DMA MFMA kernel (A and B 16-byte aligned, their stored rows whole 16-byte vectors)
 //
 // One workgroup owns a BMxBN output tile and walks its K range in BK-deep stages held in
 // an NS-deep LDS ring.  Every 16-byte chunk of a stage travels global -> LDS by
@@ -62,12 +72,11 @@ struct GemmArgs {
 // instruction write 1 KB of LDS contiguously, so the swizzled LDS layout is produced by
 // choosing which global chunk each lane fetches.  Out-of-range chunks (M, N and K tails)
 // come back as zeros from the buffer range check.
-//   A stage: [BM][BK] fp16, rows of KCH 16-byte chunks, chunk c of row r stored at
-//            c ^ swz_a(r).  Fragments: ds_read_b128 (row = lane%32, K half = lane/32).
-//   B stage: [BK][BN] fp16 (row-major as in memory), chunk c of row k stored at
-//            c ^ swz_b(k).  Fragments: two ds_read_b64_tr_b16 per 32x32x16 operand, which
-//            deliver column lane%32 with four consecutive K values each.
-// Both operands therefore present K-contiguous MFMA fragments with the same K order.
+//   K-major operand (A as stored): [rows][BK] fp16, chunk c of row r stored at c ^ swz_a(r).
+//            Fragments: ds_read_b128 (row = lane%32, K half = lane/32).
+//   Other order (B as stored): [BK][cols], chunk c of row k stored at c ^ swz_b(k).
+//            Fragments: two ds_read_b64_tr_b16 per 32x32x16 operand, which deliver column
+//            lane%32 with four consecutive K values each.
 // Wave (wm, wn) owns a TMxTN sub-tile of (TM/32)x(TN/32) 32x32 accumulators.
 // ------------------------------------------------------------------------------------
 template <int KCH>
@@ -92,36 +101,89 @@ __device__ __forceinline__ int swz_b(int k) {
         return 2 * (k & 3);
 }
 
-// Per-lane constants of the LDS-DMA kernel.
-template <int A_DMA, int B_DMA, int FM, int FN>
-struct MfmaLane {
-    uint32_t a_off[A_DMA], b_off[B_DMA];  // DMA source offsets (kOobOffset when masked)
-    int a_k[A_DMA], b_k[B_DMA];           // K offset of each DMA chunk inside a stage
-    int a_addr[FM];                       // byte offset of the lane's A row in a stage
-    int a_sw[FM];                         // swizzle of that row
-    int b_addr[FN];                       // byte offset of the lane's first tr-read
-    int h;                                // lane / 32
-    int dma_a, dma_b;                     // this wave's DMA slice of a stage (uniform)
-};
+// One operand of the LDS-DMA kernel: R rows of the output side (rows of A, columns of B) by
+// BK of K per stage, in the order it has in memory.
+//   KMAJOR: [R][K], K contiguous (A as stored, or B given transposed): rows of BK/8 chunks,
+//           fragments by ds_read_b128.
+//   else:   [K][R], R contiguous (B as stored, or A given transposed): rows of R/8 chunks,
+//           fragments by two ds_read_b64_tr_b16.
+// Either way a fragment holds K 16 ks + 8 (lane/32) + 0..7 of row lane%32 of its 32-row
+// block, so any two operands multiply.
+template <bool KMAJOR, int R, int BK, int DMA, int F>
+struct MfmaOperand {
+    static constexpr int ROW = KMAJOR ? BK : R;  // elements per LDS row
+    static constexpr int CH = ROW / 8;           // 16-byte chunks per LDS row
+    static constexpr int READS = KMAJOR ? 1 : 2; // LDS reads per fragment
+    uint32_t off[DMA];   // DMA source offsets (kOobOffset when masked)
+    int k[DMA];          // K offset of each DMA chunk inside a stage
+    int addr[F];         // byte offset of the lane's (first) read of each 32-row block
+    int sw[F];           // KMAJOR: chunk swizzle of that row
+    int dst;             // this wave's DMA slice of the operand's stage (uniform)
 
-// Fragment reads of one 16-deep k-step of a stage (A via ds_read_b128, B via two
-// ds_read_b64_tr_b16 per 32x32x16 operand).
-template <int BN, int FM, int FN, class Lane>
-__device__ __forceinline__ void mfma_read(const WMMA_LDS unsigned char* s, const Lane& L, int ks,
-                                          f16x8 (&a)[FM], f16x8 (&b)[FN]) {
+    // r0: the operand's first row of the output tile, of `rows`; fragment blocks start at
+    // tile row f0.
+    __device__ __forceinline__ void init(int wave, int lane, int r0, int rows, int64_t ld, int f0) {
+        dst = wave * (DMA * 1024);
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-        const int c = (2 * ks + L.h) ^ L.a_sw[i];
-        a[i] = as_f16x8(*(const WMMA_LDS u32x4*)(s + L.a_addr[i] + (c << 4)));
-    }
+        for (int i = 0; i < DMA; ++i) {
+            const int P = 64 * (wave * DMA + i) + lane;
+            const int l = P / CH;  // LDS row
+            if constexpr (KMAJOR) {
+                const int c = (P % CH) ^ swz_a<CH>(l);
+                off[i] = r0 + l < rows ? (uint32_t)((l * ld + 8 * c) * 2) : kOobOffset;
+                k[i] = 8 * c;
+            } else {
+                const int c = (P % CH) ^ swz_b<CH>(l);
+                off[i] = r0 + 8 * c < rows ? (uint32_t)((l * ld + 8 * c) * 2) : kOobOffset;
+                k[i] = l;
+            }
+        }
+        if constexpr (KMAJOR) {
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-        const WMMA_LDS unsigned char* pb = s + L.b_addr[j] + ks * 16 * (BN * 2);
-        const f16x4 lo = lds_read_tr16(pb);
-        const f16x4 hi = lds_read_tr16(pb + 4 * (BN * 2));
-        b[j] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+            for (int f = 0; f < F; ++f) {
+                const int r = f0 + 32 * f + (lane & 31);
+                addr[f] = r * (BK * 2);
+                sw[f] = swz_a<CH>(r);
+            }
+        } else {
+            // tr-read source lane s = 4*jj + aa of 16-lane group g: K row 8*(g/2) + jj (+4
+            // for the upper half), columns 16*(g%2) + 4*aa .. +3 of the 32-column block.
+            const int g = lane >> 4, s16 = lane & 15, jj = s16 >> 2, aa = s16 & 3;
+            const int krow = 8 * (g >> 1) + jj;
+            const int swz = swz_b<CH>(jj);
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                const int n = f0 + 32 * f + 16 * (g & 1) + 4 * aa;
+                addr[f] = krow * (R * 2) + (((n >> 3) ^ swz) << 4) + ((n & 7) << 1);
+                sw[f] = 0;
+            }
+        }
     }
-}
+    // The DMA of one stage (kleft: K that is left from the stage's first on).
+    __device__ __forceinline__ void issue(WMMA_LDS unsigned char* stage, __amdgpu_buffer_rsrc_t r,
+                                          int kleft) const {
+        const bool full = kleft >= BK;
+#pragma unroll
+        for (int i = 0; i < DMA; ++i)
+            lds_dma16(r, (full || k[i] < kleft) ? off[i] : kOobOffset, stage + dst + i * 1024);
+    }
+    // Fragments of the 16-deep k-step ks; h = lane / 32.
+    __device__ __forceinline__ void read(const WMMA_LDS unsigned char* stage, int ks, int h,
+                                         f16x8 (&frag)[F]) const {
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            if constexpr (KMAJOR) {
+                const int c = (2 * ks + h) ^ sw[f];
+                frag[f] = as_f16x8(*(const WMMA_LDS u32x4*)(stage + addr[f] + (c << 4)));
+            } else {
+                const WMMA_LDS unsigned char* pb = stage + addr[f] + ks * 16 * (R * 2);
+                const f16x4 lo = lds_read_tr16(pb);
+                const f16x4 hi = lds_read_tr16(pb + 4 * (R * 2));
+                frag[f] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+            }
+        }
+    }
+};
 
 template <int FM, int FN>
 __device__ __forceinline__ void mfma_block(const f16x8 (&a)[FM], const f16x8 (&b)[FN],
@@ -158,23 +220,23 @@ __device__ __forceinline__ void mfma_sched() {
 // The three buffers are distinct (NS >= 3), so they are passed as __restrict__
 // pointers: that lets the compiler keep the DMA in flight across the reads.  Ordering
 // between a DMA and later reads of the same buffer is the vmcnt wait + barrier of (b).
-template <int BM, int BN, int BK, int WM, int WN, int NS, int A_DMA, int B_DMA, class Lane>
+template <int BK, int NS, int A_DMA, int B_DMA, int A_BYTES, class OpA, class OpB, int FM, int FN>
 __device__ __forceinline__ void mfma_iter(const WMMA_LDS unsigned char* __restrict__ cur,
                                           const WMMA_LDS unsigned char* __restrict__ nxt,
                                           WMMA_LDS unsigned char* __restrict__ dma_dst,
-                                          const Lane& L, __amdgpu_buffer_rsrc_t ra,
-                                          __amdgpu_buffer_rsrc_t rb, int kleft,
-                                          f16x8 (&af)[2][BM / WM / 32], f16x8 (&bf)[2][BN / WN / 32],
-                                          f32x16 (&acc)[BM / WM / 32][BN / WN / 32]) {
-    constexpr int FM = BM / WM / 32, FN = BN / WN / 32;
+                                          const OpA& oa, const OpB& ob, int h,
+                                          __amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb,
+                                          int kleft, f16x8 (&af)[2][FM], f16x8 (&bf)[2][FN],
+                                          f32x16 (&acc)[FM][FN]) {
     constexpr int KS = BK / 16;
     constexpr int PER_STAGE = A_DMA + B_DMA;
-    constexpr int RD = FM + 2 * FN, MF = FM * FN;
+    constexpr int RD = FM * OpA::READS + FN * OpB::READS, MF = FM * FN;
     static_assert(KS % 2 == 0, "fragment double buffer assumes an even k-step count");
     // (a)
 #pragma unroll
     for (int ks = 0; ks + 1 < KS; ++ks) {
-        mfma_read<BN>(cur, L, ks + 1, af[(ks + 1) & 1], bf[(ks + 1) & 1]);
+        oa.read(cur, ks + 1, h, af[(ks + 1) & 1]);
+        ob.read(cur + A_BYTES, ks + 1, h, bf[(ks + 1) & 1]);
         mfma_block(af[ks & 1], bf[ks & 1], acc);
         mfma_sched<MF, RD, 0>();
     }
@@ -184,29 +246,24 @@ __device__ __forceinline__ void mfma_iter(const WMMA_LDS unsigned char* __restri
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     // (c)
-    const bool full = kleft >= BK;
-#pragma unroll
-    for (int i = 0; i < A_DMA; ++i)
-        lds_dma16(ra, (full || L.a_k[i] < kleft) ? L.a_off[i] : kOobOffset,
-                  dma_dst + L.dma_a + i * 1024);
-#pragma unroll
-    for (int i = 0; i < B_DMA; ++i)
-        lds_dma16(rb, (full || L.b_k[i] < kleft) ? L.b_off[i] : kOobOffset,
-                  dma_dst + L.dma_b + i * 1024);
+    oa.issue(dma_dst, ra, kleft);
+    ob.issue(dma_dst + A_BYTES, rb, kleft);
     // (d)
-    mfma_read<BN>(nxt, L, 0, af[0], bf[0]);
+    oa.read(nxt, 0, h, af[0]);
+    ob.read(nxt + A_BYTES, 0, h, bf[0]);
     mfma_block(af[1], bf[1], acc);
     mfma_sched<MF, RD, PER_STAGE>();
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int NS>
+// TA / TB: A is stored [K][M] / B is stored [N][K] (a transposed view; ld is then the stride of
+// a stored row).
+template <int BM, int BN, int BK, int WM, int WN, int NS, bool TA = false, bool TB = false>
 __global__ void __launch_bounds__(WM * WN * kWave)
 __attribute__((amdgpu_waves_per_eu(WM * WN / 4, WM * WN / 4)))
 gemm_mfma_kernel(GemmArgs p) {
     constexpr int NW = WM * WN;
     constexpr int TM = BM / WM, TN = BN / WN;
     constexpr int FM = TM / 32, FN = TN / 32;
-    constexpr int KCH = BK / 8, BNC = BN / 8;
     constexpr int A_BYTES = BM * BK * 2, B_BYTES = BK * BN * 2;
     constexpr int STAGE = A_BYTES + B_BYTES;
     constexpr int A_DMA = A_BYTES / (1024 * NW);  // 1 KB DMA instructions per wave
@@ -233,42 +290,11 @@ gemm_mfma_kernel(GemmArgs p) {
     const int M = p.M, N = p.N;
     const int64_t lda = p.lda, ldb = p.ldb;
 
-    MfmaLane<A_DMA, B_DMA, FM, FN> L;
-#pragma unroll
-    for (int i = 0; i < A_DMA; ++i) {
-        const int P = 64 * (wave * A_DMA + i) + lane;
-        const int r = P / KCH, c = (P % KCH) ^ swz_a<KCH>(r);
-        L.a_off[i] = m0 + r < M ? (uint32_t)((r * lda + 8 * c) * 2) : kOobOffset;
-        L.a_k[i] = 8 * c;
-    }
-#pragma unroll
-    for (int i = 0; i < B_DMA; ++i) {
-        const int P = 64 * (wave * B_DMA + i) + lane;
-        const int k = P / BNC, c = (P % BNC) ^ swz_b<BNC>(k);
-        L.b_off[i] = n0 + 8 * c < N ? (uint32_t)((k * ldb + 8 * c) * 2) : kOobOffset;
-        L.b_k[i] = k;
-    }
-    L.h = lane >> 5;
-    L.dma_a = wave * (A_DMA * 1024);
-    L.dma_b = A_BYTES + wave * (B_DMA * 1024);
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-        const int r = wm * TM + i * 32 + (lane & 31);
-        L.a_addr[i] = r * (BK * 2);
-        L.a_sw[i] = swz_a<KCH>(r);
-    }
-    {
-        // tr-read source lane s = 4*jj + aa of 16-lane group g: row 8*(g/2) + jj (+4 for
-        // the upper half), columns 16*(g%2) + 4*aa .. +3 of the wave's 32-column tile.
-        const int g = lane >> 4, s16 = lane & 15, jj = s16 >> 2, aa = s16 & 3;
-        const int krow = 8 * (g >> 1) + jj;
-        const int sw = swz_b<BNC>(jj);
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            const int n = wn * TN + j * 32 + 16 * (g & 1) + 4 * aa;
-            L.b_addr[j] = A_BYTES + krow * (BN * 2) + (((n >> 3) ^ sw) << 4) + ((n & 7) << 1);
-        }
-    }
+    const int h = lane >> 5;
+    MfmaOperand<!TA, BM, BK, A_DMA, FM> oa;
+    MfmaOperand<TB, BN, BK, B_DMA, FN> ob;
+    oa.init(wave, lane, m0, M, lda, wm * TM);
+    ob.init(wave, lane, n0, N, ldb, wn * TN);
 
     f32x16 acc[FM][FN];
 #pragma unroll
@@ -276,12 +302,12 @@ gemm_mfma_kernel(GemmArgs p) {
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
 
-    const f16* Ablk = p.A + (int64_t)m0 * lda;
-    const f16* Bblk = p.B + n0;
-    auto rsrc_a = [&](int kt) { return make_rsrc(Ablk + kbeg + (int64_t)min(kt, nk - 1) * BK); };
-    auto rsrc_b = [&](int kt) {
-        return make_rsrc(Bblk + (int64_t)(kbeg + (int64_t)min(kt, nk - 1) * BK) * ldb);
-    };
+    // First element of each operand's tile, and the elements one stage of K moves it by.
+    const f16* Ablk = TA ? p.A + (int64_t)kbeg * lda + m0 : p.A + (int64_t)m0 * lda + kbeg;
+    const f16* Bblk = TB ? p.B + (int64_t)n0 * ldb + kbeg : p.B + (int64_t)kbeg * ldb + n0;
+    const int64_t a_step = TA ? BK * lda : BK, b_step = TB ? BK : BK * ldb;
+    auto rsrc_a = [&](int kt) { return make_rsrc(Ablk + min(kt, nk - 1) * a_step); };
+    auto rsrc_b = [&](int kt) { return make_rsrc(Bblk + min(kt, nk - 1) * b_step); };
     auto kleft = [&](int kt) { return kt < nk ? kend - (kbeg + kt * BK) : 0; };
 
     if (nk > 0) {
@@ -289,30 +315,21 @@ gemm_mfma_kernel(GemmArgs p) {
         // landed and visible, the first k-step of stage 0 read.
 #pragma unroll
         for (int s = 0; s < NS - 1; ++s) {
-            WMMA_LDS unsigned char* dst = lds + s * STAGE;
-            const int kl = kleft(s);
-            const bool full = kl >= BK;
-            const __amdgpu_buffer_rsrc_t ra = rsrc_a(s), rb = rsrc_b(s);
-#pragma unroll
-            for (int i = 0; i < A_DMA; ++i)
-                lds_dma16(ra, (full || L.a_k[i] < kl) ? L.a_off[i] : kOobOffset,
-                          dst + L.dma_a + i * 1024);
-#pragma unroll
-            for (int i = 0; i < B_DMA; ++i)
-                lds_dma16(rb, (full || L.b_k[i] < kl) ? L.b_off[i] : kOobOffset,
-                          dst + L.dma_b + i * 1024);
+            oa.issue(lds + s * STAGE, rsrc_a(s), kleft(s));
+            ob.issue(lds + s * STAGE + A_BYTES, rsrc_b(s), kleft(s));
         }
         wait_vmcnt<(NS - 2) * PER_STAGE>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         f16x8 af[2][FM], bf[2][FN];
-        mfma_read<BN>(lds, L, 0, af[0], bf[0]);
+        oa.read(lds, 0, h, af[0]);
+        ob.read(lds + A_BYTES, 0, h, bf[0]);
 
         for (int t = 0; t < nk; ++t) {
             const int tf = t + NS - 1;  // stage whose DMA is issued in this iteration
-            mfma_iter<BM, BN, BK, WM, WN, NS, A_DMA, B_DMA>(
-                lds + (t % NS) * STAGE, lds + ((t + 1) % NS) * STAGE, lds + (tf % NS) * STAGE, L,
-                rsrc_a(tf), rsrc_b(tf), kleft(tf), af, bf, acc);
+            mfma_iter<BK, NS, A_DMA, B_DMA, A_BYTES>(
+                lds + (t % NS) * STAGE, lds + ((t + 1) % NS) * STAGE, lds + (tf % NS) * STAGE, oa,
+                ob, h, rsrc_a(tf), rsrc_b(tf), kleft(tf), af, bf, acc);
         }
         wait_vmcnt<0>();
     }
@@ -323,7 +340,6 @@ gemm_mfma_kernel(GemmArgs p) {
     const int64_t ldo = partial ? (int64_t)N : p.ldc;
     const float alpha = partial ? 1.0f : p.alpha;
     const bool use_c = !partial && p.beta != 0.0f && p.Cin != nullptr;
-    const int h = lane >> 5;
     const int row0 = m0 + wm * TM + 4 * h, col0 = n0 + wn * TN + (lane & 31);
     const bool full_tile = m0 + BM <= M && n0 + BN <= N;
     // Full tiles whose rows take 16-byte vectors (output, and C_in when it is read) go
@@ -821,6 +837,133 @@ gemm_skinny_kernel(GemmArgs p) {
 }
 
 // ------------------------------------------------------------------------------------
+// Skinny kernel for B stored [N][K] (M <= 16 MB): a workgroup owns 16 NB rows of the stored B
+// (output columns) over its K range, its 8 waves taking 128-deep K steps in turn.  K is
+// contiguous in both operands, so every load is an MFMA operand as it arrives (16 bytes per
+// lane: row lane%16, K quarter lane/16; four loads of a row block cover its 256 bytes) and
+// nothing is transposed; the waves' sums meet in LDS once.  The next step's loads are in
+// flight while a step is multiplied.  A workgroup can cover all of K, so most shapes need
+// no K split and no reduction launch.  ALIGNED: stored rows are whole 16-byte vectors; else
+// rows start at any element: a dword-aligned 16-byte load plus the next dword, shifted by
+// v_alignbyte, and the K tail element-wise.
+// ------------------------------------------------------------------------------------
+constexpr int SKT_WAVES = 8;
+constexpr int SKT_STEP = 128;
+
+template <bool ALIGNED>
+struct SkinnyRows {
+    __amdgpu_buffer_rsrc_t rs;
+    uint32_t odd;  // bytes (0 or 2) from the descriptor's base to the first element
+    __device__ __forceinline__ explicit SkinnyRows(const f16* base) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(base);
+        odd = ALIGNED ? 0 : (uint32_t)(a & 2);
+        rs = make_rsrc(reinterpret_cast<const void*>(a - odd));
+    }
+    // Eight elements from k on of the row at element offset `row` (zeros past kend).
+    __device__ __forceinline__ u32x4 load(bool ok, int64_t row, int k, int kend) const {
+        const uint32_t at = (uint32_t)((row + k) * 2) + odd;
+        if constexpr (ALIGNED) return buf_load16(rs, ok && k < kend ? at : kOobOffset);
+        const bool whole = ok && k + 8 <= kend;
+        const uint32_t sh = at & 2;
+        const u32x4 x = buf_load16(rs, whole ? at - sh : kOobOffset);
+        // the dword at at - sh + 16 holds the chunk's last element when sh is 2
+        const uint32_t y = buf_load4(rs, whole && sh ? at + 14 : kOobOffset);
+        u32x4 v{__builtin_amdgcn_alignbyte(x[1], x[0], sh), __builtin_amdgcn_alignbyte(x[2], x[1], sh),
+                __builtin_amdgcn_alignbyte(x[3], x[2], sh), __builtin_amdgcn_alignbyte(y, x[3], sh)};
+        if (ok && k < kend && k + 8 > kend) {
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                const uint32_t lo = buf_load2(rs, k + e < kend ? at + 2 * e : kOobOffset);
+                const uint32_t hi = buf_load2(rs, k + e + 1 < kend ? at + 2 * e + 2 : kOobOffset);
+                v[e >> 1] = lo | (hi << 16);
+            }
+        }
+        return v;
+    }
+};
+
+template <int MB, int NB, bool ALIGNED>
+__global__ void __launch_bounds__(SKT_WAVES * kWave)
+gemm_skinny_nt_kernel(GemmArgs p) {
+    constexpr int COLS = 16 * NB, ROWS = 16 * MB;
+    __shared__ __attribute__((aligned(16))) float red[SKT_WAVES][ROWS][COLS + 4];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, r16 = lane & 15;
+    const int n0 = blockIdx.x * COLS;
+    const int kbeg = blockIdx.y * p.k_per_split;
+    const int kend = min(p.K, kbeg + p.k_per_split);
+    const int M = p.M, N = p.N;
+
+    f32x4 acc[NB][MB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = f32x4{};
+
+    const SkinnyRows<ALIGNED> ra(p.A), rb(p.B + (int64_t)n0 * p.ldb);
+    struct Step {
+        u32x4 b[NB][4], a[MB][4];
+    };
+    auto load = [&](int i, Step& S) {
+        const int k0 = kbeg + (wave + i * SKT_WAVES) * SKT_STEP + 8 * q;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                S.b[nb][u] = rb.load(n0 + 16 * nb + r16 < N, (16 * nb + r16) * p.ldb, k0 + 32 * u, kend);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                S.a[mb][u] = ra.load(16 * mb + r16 < M, (16 * mb + r16) * p.lda, k0 + 32 * u, kend);
+    };
+    auto compute = [&](const Step& S) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+                    acc[nb][mb] = mfma16(as_f16x8(S.b[nb][u]), as_f16x8(S.a[mb][u]), acc[nb][mb]);
+    };
+    const int steps = (kend - kbeg + SKT_WAVES * SKT_STEP - 1) / (SKT_WAVES * SKT_STEP);
+    Step S0, S1;
+    load(0, S0);
+    for (int i = 0; i < steps; i += 2) {
+        load(i + 1, S1);
+        compute(S0);
+        load(i + 2, S0);
+        compute(S1);
+    }
+
+    // D: lane holds column m = lane%16 of A's block, elements 4 (lane/16) + 0..3 of B's rows.
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+            *reinterpret_cast<f32x4*>(&red[wave][16 * mb + r16][16 * nb + 4 * q]) = acc[nb][mb];
+    __syncthreads();
+    const bool use_c = p.beta != 0.0f && p.Cin != nullptr;
+    float* part = p.split > 1 ? p.ws + (size_t)blockIdx.y * (size_t)M * (size_t)N : nullptr;
+    for (int e = tid; e < ROWS * COLS; e += SKT_WAVES * kWave) {
+        const int m = e / COLS, n = e % COLS;
+        if (m >= M || n0 + n >= N) continue;
+        float v = red[0][m][n];
+#pragma unroll
+        for (int w = 1; w < SKT_WAVES; ++w) v += red[w][m][n];
+        if (part) {
+            part[(int64_t)m * N + n0 + n] = v;
+        } else {
+            v = p.alpha * v;
+            if (use_c) v += p.beta * p.Cin[(int64_t)m * p.ldcin + n0 + n];
+            p.Cout[(int64_t)m * p.ldc + n0 + n] = v;
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------
 // Split-K reduction + epilogue: out = alpha * sum_s ws[s] (+ beta * C_in).  One thread per
 // W columns of a row (W = 4 when N is a multiple of 4 and the workspace 16-byte aligned).
 // ------------------------------------------------------------------------------------
@@ -917,12 +1060,12 @@ struct MfmaStages {
 constexpr MfmaStages kMfmaStages[WMMA_TILE_COUNT] = {
     {64, 4}, {64, 4}, {64, 3}, {64, 4}, {64, 3}, {32, 4}};
 
-template <int CFG>
+template <int CFG, bool TA, bool TB>
 void launch_mfma(const GemmArgs& a, hipStream_t stream) {
     constexpr TileShape t = kTiles[CFG];
     constexpr MfmaStages st = kMfmaStages[CFG];
     dim3 grid(a.tiles_m * a.tiles_n, a.split);
-    hipLaunchKernelGGL((gemm_mfma_kernel<t.bm, t.bn, st.bk, t.wm, t.wn, st.ns>), grid,
+    hipLaunchKernelGGL((gemm_mfma_kernel<t.bm, t.bn, st.bk, t.wm, t.wn, st.ns, TA, TB>), grid,
                        dim3(t.wm * t.wn * kWave), 0, stream, a);
 }
 
@@ -940,14 +1083,34 @@ void launch_skinny(int bmode, const GemmArgs& a, hipStream_t stream) {
     }
 }
 
+// Skinny kernel for B stored [N][K]: plan.tile_m = 16 MB rows, plan.tile_n = 16 NB columns.
+template <int MB, int NB>
+void launch_skinny_nt(bool aligned, const GemmArgs& a, hipStream_t stream) {
+    const dim3 grid(ceil_div(a.N, 16 * NB), a.split), block(SKT_WAVES * kWave);
+    if (aligned)
+        hipLaunchKernelGGL((gemm_skinny_nt_kernel<MB, NB, true>), grid, block, 0, stream, a);
+    else
+        hipLaunchKernelGGL((gemm_skinny_nt_kernel<MB, NB, false>), grid, block, 0, stream, a);
+}
+
+template <int MB>
+void launch_skinny_nt_cols(int cols, bool aligned, const GemmArgs& a, hipStream_t stream) {
+    switch (cols) {
+        case 16: launch_skinny_nt<MB, 1>(aligned, a, stream); break;
+        case 32: launch_skinny_nt<MB, 2>(aligned, a, stream); break;
+        default: launch_skinny_nt<MB, 4>(aligned, a, stream); break;
+    }
+}
+
+template <bool TA, bool TB>
 void launch_mfma_cfg(int cfg, const GemmArgs& a, hipStream_t stream) {
     switch (cfg) {
-        case 0: launch_mfma<0>(a, stream); break;
-        case 1: launch_mfma<1>(a, stream); break;
-        case 2: launch_mfma<2>(a, stream); break;
-        case 3: launch_mfma<3>(a, stream); break;
-        case 4: launch_mfma<4>(a, stream); break;
-        default: launch_mfma<5>(a, stream); break;
+        case 0: launch_mfma<0, TA, TB>(a, stream); break;
+        case 1: launch_mfma<1, TA, TB>(a, stream); break;
+        case 2: launch_mfma<2, TA, TB>(a, stream); break;
+        case 3: launch_mfma<3, TA, TB>(a, stream); break;
+        case 4: launch_mfma<4, TA, TB>(a, stream); break;
+        default: launch_mfma<5, TA, TB>(a, stream); break;
     }
 }
 
@@ -985,7 +1148,12 @@ hipError_t launch_gemm(const GemmLaunch& g, hipStream_t stream) {
     a.tiles_m = ceil_div(g.M, pl.tile_m);
     a.tiles_n = ceil_div(g.N, pl.tile_n);
 
-    if (pl.kernel == WMMA_KERNEL_SKINNY) {
+    if (pl.kernel == WMMA_KERNEL_SKINNY && g.trans_b) {
+        if (g.M <= 16)
+            launch_skinny_nt_cols<1>(pl.tile_n, g.vec, a, stream);
+        else
+            launch_skinny_nt_cols<2>(pl.tile_n, g.vec, a, stream);
+    } else if (pl.kernel == WMMA_KERNEL_SKINNY) {
         const int bmode = g.vec ? (int)SKB_VEC : g.skinny_b;
         if (g.M <= 16)
             launch_skinny<1>(bmode, a, stream);
@@ -994,8 +1162,12 @@ hipError_t launch_gemm(const GemmLaunch& g, hipStream_t stream) {
         else
             launch_skinny<4>(bmode, a, stream);
     } else {
-        if (g.vec)
-            launch_mfma_cfg(pl.tile_cfg, a, stream);
+        if (g.vec && g.trans_a)
+            launch_mfma_cfg<true, false>(pl.tile_cfg, a, stream);
+        else if (g.vec && g.trans_b)
+            launch_mfma_cfg<false, true>(pl.tile_cfg, a, stream);
+        else if (g.vec)
+            launch_mfma_cfg<false, false>(pl.tile_cfg, a, stream);
         else
             launch_tiled_cfg<false>(pl.tile_cfg, a, stream);
     }

@@ -19,7 +19,11 @@ struct GemmLaunch {
     int64_t lda, ldb, ldc_in, ldc;
     int M, N, K;
     float alpha, beta;
-    bool vec;  // 16-byte vector path: K, N, lda, ldb multiples of 8, A and B 16-byte aligned
+    // A stored [K][M] / B stored [N][K] (at most one of them; vec only); lda / ldb is the
+    // stride of a stored row.
+    bool trans_a, trans_b;
+    bool vec;  // 16-byte vector path: stored rows of A and B whole 16-byte vectors, lda, ldb
+               // multiples of 8, A and B 16-byte aligned
     // Skinny kernel when !vec: 0 = element-wise; 2 / 3 = A in 16-byte vectors, B 4-byte
     // aligned with ldb even / odd (rows read in place by dword-aligned 16-byte loads)
     int skinny_b;

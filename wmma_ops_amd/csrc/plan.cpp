@@ -79,12 +79,34 @@ double model_time_us(const wmma_gemm_plan& p, int M, int N, int K, int num_cus) 
     return t;
 }
 
+// Modelled time of a skinny plan for B stored [N][K], read off a sweep of 16, 32 and 64
+// columns x splits 1-8 at 44 shapes (M = 1-32, N = 256-14336, K = 1024-14336): a workgroup
+// streams its operand bytes at 27 KB/us, all of them together at 5.1 TB/s from HBM and
+// 7.3 TB/s from L2 (every workgroup reads all of A's K range again), and past one wave the
+// busiest CU sets the pace (N = 11008: 344 workgroups of 32 columns 29 us, 688 of 16 21 us).
+// A K split adds its reduction.  Its choices take 3% more time than the fastest of each
+// shape.
+static double skinny_nt_time_us(const wmma_gemm_plan& p, int M, int N, int K, int num_cus) {
+    const int split = std::max(p.split_k, 1);
+    const double kk = split > 1 ? p.k_per_split : K;
+    const int64_t wgs = (int64_t)ceil_div(N, p.tile_n) * split;
+    const int64_t waves = ceil_div64(wgs, num_cus);
+    const double kb = (p.tile_n + std::min(M, p.tile_m)) * kk * 2.0 / 1000.0;
+    const double uneven = wgs > num_cus ? (double)(waves * num_cus) / (double)wgs : 1.0;
+    const double hbm_mb = (2.0 * M * K + 2.0 * K * N + 4.0 * M * N) / 1e6;
+    double t = 2.0 + std::max(waves * kb / 27.0,
+                              uneven * std::max(hbm_mb / 5.1, wgs * kb / 1000.0 / 7.3));
+    if (split > 1) t += 3.0 + 0.5 * (split + 1) * 4.0 * M * N / 1e6;
+    return t;
+}
+
 // The plan with the shortest modelled time: every tile with K splits 1, 2, 4, 8, 16 (a
 // split only from K = 2048, at least 256 of K per part, and only while the workgroups fit
 // one wave of the CUs), and for M <= 32 the streaming kernel with splits up to K / 256.
 // Over the fitted shapes the choice costs 0.65% more time than the fastest plan of each
 // shape (the previous heuristics: 14%), and 0.8% on a second sweep of 63 shapes.
-static wmma_gemm_plan model_plan(int M, int N, int K, int num_cus, size_t max_ws) {
+static wmma_gemm_plan model_plan(int M, int N, int K, int num_cus, size_t max_ws,
+                                 bool skinny = true) {
     wmma_gemm_plan best{};
     double best_t = 1e300;
     for (int cfg = 0; cfg < WMMA_TILE_COUNT; ++cfg) {
@@ -103,7 +125,7 @@ static wmma_gemm_plan model_plan(int M, int N, int K, int num_cus, size_t max_ws
             }
         }
     }
-    if (M <= 32) {
+    if (skinny && M <= 32) {
         for (int sp : {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32}) {
             if (sp > std::max(1, K / 256)) break;
             wmma_gemm_plan c{};
@@ -300,6 +322,46 @@ int make_plan_within(int M, int N, int K, int tile_cfg, int num_cus, size_t max_
     if (tile_cfg == WMMA_TILE_AUTO && p.split_k == 1) two_part(M, N, K, num_cus, max_ws, &p);
     *out = p;
     return WMMA_OK;
+}
+
+// The skinny kernel for B stored [N][K]: columns per workgroup and K split.
+static wmma_gemm_plan skinny_nt_plan(int M, int N, int K, int num_cus, size_t max_ws) {
+    wmma_gemm_plan best{};
+    double best_t = 1e300;
+    const int mb = M <= 16 ? 1 : 2;
+    for (int cols : {16, 32, 64}) {
+        const int tiles = ceil_div(N, cols);
+        for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
+            if (sp > 1 && (K < sp * kSkinnyNtRound || (int64_t)tiles * sp > 4 * (int64_t)num_cus)) break;
+            wmma_gemm_plan c{};
+            c.kernel = WMMA_KERNEL_SKINNY;
+            c.tile_cfg = -1;
+            c.tile_m = 16 * mb;
+            c.tile_n = cols;
+            finish_split(M, N, K, tiles, sp, &c);
+            if (c.workspace_bytes > max_ws) continue;
+            const double t = skinny_nt_time_us(c, M, N, K, num_cus);
+            if (t < best_t * 0.999) {
+                best_t = t;
+                best = c;
+            }
+        }
+    }
+    return best;
+}
+
+int make_layout_plan(GemmLayout layout, int M, int N, int K, int tile_cfg, int num_cus,
+                     size_t max_ws, wmma_gemm_plan* out) {
+    if (num_cus <= 0) num_cus = 256;
+    const bool some = M > 0 && N > 0 && K > 0 && tile_cfg == WMMA_TILE_AUTO;
+    if (some && layout == GemmLayout::NT && M <= kSkinnyNtMaxM) {
+        *out = skinny_nt_plan(M, N, K, num_cus, max_ws);
+        return WMMA_OK;
+    }
+    int rc = make_plan_within(M, N, K, tile_cfg, num_cus, max_ws, out);
+    if (rc == WMMA_OK && layout != GemmLayout::NN && out->kernel == WMMA_KERNEL_SKINNY)
+        *out = model_plan(M, N, K, num_cus, max_ws, /*skinny=*/false);
+    return rc;
 }
 
 }  // namespace wmma_amd

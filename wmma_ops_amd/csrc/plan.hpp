@@ -87,6 +87,22 @@ constexpr double kEdgeGain = 0.93;
 // plan.cpp, which may split it into a bulk and an edge GEMM (out->edge_dim).
 int make_plan(int M, int N, int K, int tile_cfg, int num_cus, wmma_gemm_plan* out);
 
+// A GEMM whose A or B is given transposed (A stored [K][M], or B stored [N][K]; at most one).
+enum class GemmLayout { NN, TN, NT };
+
+// Skinny kernel for B stored [N][K] (gemm_skinny_nt_kernel): its rows, column counts per
+// workgroup and 8 x 128 of K that the waves of a workgroup take per round.
+constexpr int kSkinnyNtMaxM = 32;
+constexpr int kSkinnyNtRound = 1024;
+
+// make_plan_within for a transposed operand.  The tiled kernel takes either operand in
+// either layout and keeps the plan of the plain layout (its tiles read whole 64-byte or
+// longer runs of every operand in each of them); the streaming kernel reads B row-major
+// only: TN takes a tiled plan instead, NT at M <= kSkinnyNtMaxM a plan of its own kernel
+// (tile_m 16 or 32, tile_n 16, 32 or 64 columns per workgroup).
+int make_layout_plan(GemmLayout layout, int M, int N, int K, int tile_cfg, int num_cus,
+                     size_t max_ws, wmma_gemm_plan* out);
+
 // make_plan among the plans whose split-K partial sums fit max_ws bytes: a tuned-table
 // entry or a split that needs more is passed over for the next choice (a plan without a
 // split needs none, so there always is one).

@@ -3,7 +3,7 @@
 // Mirrors the pybind module of the reference (wmma_gemm.hip:2120-2157): the same
 // function names, argument meaning, defaults and TORCH_CHECK messages
 // (wmma_gemm.hip:1197-1263, 1432-1528, 1891-2078).  Tensors are validated here, made
-// contiguous, outputs come from the caching allocator, and the work is enqueued on the
+// contiguous where the kernels do not read them as they are, outputs come from the caching allocator, and the work is enqueued on the
 // current HIP stream of A's device through the C-ABI in include/wmma_ops_amd.h.  Unlike
 // the reference a device guard is taken, so the launch goes to the tensors' device.
 //
@@ -18,6 +18,7 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include <algorithm>
 #include <cmath>
 #include <string>
 
@@ -43,7 +44,10 @@ void check_ab(const torch::Tensor& A, const torch::Tensor& B, bool same_device_c
     TORCH_CHECK(A.size(1) == B.size(0), "Inner dimensions must match");
 }
 
+// The reference takes a contiguous input only at a 16-byte address; one that is not contiguous
+// it copies first, so a view at any address is accepted.
 void check_aligned(const torch::Tensor& t, const char* msg) {
+    if (!t.is_contiguous()) return;
     TORCH_CHECK((reinterpret_cast<uintptr_t>(t.data_ptr()) % 16) == 0, msg);
 }
 
@@ -52,20 +56,60 @@ torch::Tensor workspace_for(size_t bytes, const torch::Tensor& like) {
     return torch::empty({(int64_t)bytes}, torch::dtype(torch::kUInt8).device(like.device()));
 }
 
+// How the GEMM reads an operand: `t` itself, with the stride of a stored row, and whether it
+// is stored transposed.
+struct GemmOperand {
+    torch::Tensor t;
+    int64_t ld;
+    bool trans;
+};
+
+// Strides that the kernels' 32-bit offsets hold whatever the tile (257 rows of 2-byte elements).
+constexpr int64_t kMaxViewStride = 4000000;
+
+// A tensor that is not contiguous but keeps whole rows (a slice of columns) or whole columns
+// (a transpose) in order is read where it is; anything else (steps, expanded or overlapping
+// rows, longer strides) as a contiguous copy.
+GemmOperand gemm_operand(const torch::Tensor& t) {
+    const int64_t r = t.size(0), c = t.size(1);
+    if (t.is_contiguous()) return {t, t.stride(0), false};
+    if (r > 1 && c > 1 && std::max(t.stride(0), t.stride(1)) <= kMaxViewStride) {
+        if (t.stride(1) == 1 && t.stride(0) >= c) return {t, t.stride(0), false};
+        if (t.stride(0) == 1 && t.stride(1) >= r) return {t, t.stride(1), true};
+    }
+    torch::Tensor copy = t.contiguous();
+    return {copy, copy.stride(0), false};
+}
+
+// A and B as the GEMM reads them; of two transposed ones the smaller is copied.
+void gemm_operands(const torch::Tensor& A, const torch::Tensor& B, GemmOperand* a, GemmOperand* b) {
+    *a = gemm_operand(A);
+    *b = gemm_operand(B);
+    if (a->trans && b->trans) {
+        GemmOperand* x = A.numel() <= B.numel() ? a : b;
+        x->t = x->t.contiguous();
+        x->ld = x->t.stride(0);
+        x->trans = false;
+    }
+}
+
 // One GEMM through the C-ABI.  C_in may be undefined; C_out preallocated.
-void run_gemm(const torch::Tensor& A, const torch::Tensor& B, const torch::Tensor& C_in,
+void run_gemm(const GemmOperand& A, const GemmOperand& B, const torch::Tensor& C_in,
               torch::Tensor& C_out, double alpha, double beta, int tile_cfg) {
-    const int M = (int)A.size(0), K = (int)A.size(1), N = (int)B.size(1);
-    TORCH_CHECK(A.size(0) <= INT32_MAX && A.size(1) <= INT32_MAX && B.size(1) <= INT32_MAX,
+    TORCH_CHECK(A.t.size(0) <= INT32_MAX && A.t.size(1) <= INT32_MAX && B.t.size(1) <= INT32_MAX,
                 "dimensions exceed int32");
-    const size_t ws_bytes = wmma_gemm_workspace_size(M, N, K, tile_cfg);
-    torch::Tensor ws = workspace_for(ws_bytes, A);
+    const int M = (int)A.t.size(0), K = (int)A.t.size(1), N = (int)B.t.size(1);
+    const size_t ws_bytes =
+        wmma_gemm_view_workspace_size(A.t.data_ptr(), A.ld, A.trans, B.t.data_ptr(), B.ld, B.trans,
+                                      M, N, K, tile_cfg);
+    torch::Tensor ws = workspace_for(ws_bytes, A.t);
     const float* cin = C_in.defined() ? C_in.data_ptr<float>() : nullptr;
     const int64_t ldcin = C_in.defined() ? C_in.stride(0) : N;
-    int rc = wmma_gemm_f16f32(A.data_ptr(), A.stride(0), B.data_ptr(), B.stride(0), cin, ldcin,
-                              C_out.data_ptr<float>(), C_out.stride(0), M, N, K,
-                              static_cast<float>(alpha), static_cast<float>(beta), tile_cfg,
-                              ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, current_stream(A));
+    int rc = wmma_gemm_f16f32_view(A.t.data_ptr(), A.ld, A.trans, B.t.data_ptr(), B.ld, B.trans, cin,
+                                   ldcin, C_out.data_ptr<float>(), C_out.stride(0), M, N, K,
+                                   static_cast<float>(alpha), static_cast<float>(beta), tile_cfg,
+                                   ws.defined() ? ws.data_ptr() : nullptr, ws_bytes,
+                                   current_stream(A.t));
     check_status(rc, "wmma_gemm_f16f32");
 }
 
@@ -76,14 +120,14 @@ torch::Tensor matmul_impl(torch::Tensor A, torch::Tensor B, int tile_cfg, bool s
                           bool vec_text) {
     check_ab(A, B, same_device);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(A.device());
-    A = A.contiguous();
-    B = B.contiguous();
     check_aligned(A, vec_text ? "A must be 16-byte aligned for vectorized loads"
                               : "A must be 16-byte aligned");
     check_aligned(B, vec_text ? "B must be 16-byte aligned for vectorized loads"
                               : "B must be 16-byte aligned");
+    GemmOperand a, b;
+    gemm_operands(A, B, &a, &b);
     auto C = torch::empty({A.size(0), B.size(1)}, torch::dtype(torch::kFloat32).device(A.device()));
-    run_gemm(A, B, torch::Tensor(), C, 1.0, 0.0, tile_cfg);
+    run_gemm(a, b, torch::Tensor(), C, 1.0, 0.0, tile_cfg);
     return C;
 }
 
@@ -116,10 +160,10 @@ torch::Tensor gemm_impl(torch::Tensor A, torch::Tensor B, double alpha, double b
                         c10::optional<torch::Tensor> C_opt) {
     check_ab(A, B, true);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(A.device());
-    A = A.contiguous();
-    B = B.contiguous();
     check_aligned(A, "A must be 16-byte aligned");
     check_aligned(B, "B must be 16-byte aligned");
+    GemmOperand a, b;
+    gemm_operands(A, B, &a, &b);
     const int64_t M = A.size(0), N = B.size(1);
     torch::Tensor C_in;
     if (beta != 0.0 && C_opt.has_value() && C_opt->defined()) {
@@ -132,7 +176,7 @@ torch::Tensor gemm_impl(torch::Tensor A, torch::Tensor B, double alpha, double b
         C_in = C_in.contiguous();
     }
     auto C_out = torch::empty({M, N}, torch::dtype(torch::kFloat32).device(A.device()));
-    run_gemm(A, B, C_in, C_out, alpha, beta, WMMA_TILE_AUTO);
+    run_gemm(a, b, C_in, C_out, alpha, beta, WMMA_TILE_AUTO);
     return C_out;
 }
 
@@ -162,11 +206,11 @@ void gemm_inplace(torch::Tensor A, torch::Tensor B, torch::Tensor C, double alph
                 "C dimensions must match output (M×N)");
     TORCH_CHECK(C.is_contiguous(), "C must be contiguous for in-place update");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(A.device());
-    A = A.contiguous();
-    B = B.contiguous();
     check_aligned(A, "A must be 16-byte aligned");
     check_aligned(B, "B must be 16-byte aligned");
-    run_gemm(A, B, C, C, alpha, beta, WMMA_TILE_AUTO);
+    GemmOperand a, b;
+    gemm_operands(A, B, &a, &b);
+    run_gemm(a, b, C, C, alpha, beta, WMMA_TILE_AUTO);
 }
 
 // Checks of the dense attention inputs Q [B,H,Sq,D], K/V [B,Hkv,Sk,D] (flash_attention and
