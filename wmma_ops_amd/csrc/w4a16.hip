@@ -618,9 +618,10 @@ w4a16_decode_kernel(W4Args p) {
     load_round(0, R0);
 
     // Stage activations and per-run sums.  Thread i owns chunk i (8 values); the four
-    // chunks of a 32-value run sit in four consecutive lanes.
+    // chunks of a 32-value run sit in four consecutive lanes.  Every lane takes part in the
+    // shuffles; a lane past the last chunk stores nothing (its slot is the run sums').
     auto stage_chunk = [&](int i, u32x4 v) {
-        reinterpret_cast<u32x4*>(sA)[i] = v;
+        if (i < nchunk) reinterpret_cast<u32x4*>(sA)[i] = v;
         const f16x8 a = as_f16x8(v);
         float s1 = (float)a[0] + (float)a[1] + (float)a[4] + (float)a[5];
         float s16 = (float)a[2] + (float)a[3] + (float)a[6] + (float)a[7];
@@ -628,7 +629,7 @@ w4a16_decode_kernel(W4Args p) {
         s16 += __shfl_xor(s16, 1);
         s1 += __shfl_xor(s1, 2);
         s16 += __shfl_xor(s16, 2);
-        if ((i & 3) == 0) sSum[i >> 2] = make_float2(s1, s16);
+        if ((i & 3) == 0 && i < nchunk) sSum[i >> 2] = make_float2(s1, s16);
     };
 #pragma unroll
     for (int j = 0; j < ABUF; ++j) {
