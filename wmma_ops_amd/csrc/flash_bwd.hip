@@ -434,8 +434,9 @@ flash_bwd_dq_kernel(BwdArgs p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, c32 = lane & 31;
     // Which query block of which (batch, head): see flash_sched.hpp.
-    int col;
-    const int64_t row = flash_split_id(flash_linear_id(), p.cu_q ? p.H : p.B * p.H, &col);
+    int col = blockIdx.x;
+    int64_t row = blockIdx.y;
+    if (CAUSAL || p.cu_q) row = flash_split_id(flash_linear_id(), p.cu_q ? p.H : p.B * p.H, &col);
     int b = col / p.H, qb_idx = CAUSAL ? p.nqb - 1 - (int)row : (int)row;
     if (p.cu_q && !varlen_item<false, CAUSAL, FbGeom<D>::BLOCK_Q>(
                       p.cu_q, p.cu_k, p.B, p.total_q, p.total_k, p.Sq, p.Sk, row, &b, &qb_idx))
@@ -664,12 +665,15 @@ flash_bwd_dkdv_kernel(BwdArgs p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, c32 = lane & 31;
     // Which key block of which (batch, key/value head), and which of its column and group
-    // parts z: the parts of a block are neighbours, so that heavier blocks still go first
-    // (causal: lower key blocks are heavier); see flash_sched.hpp.
-    int col, z;
-    const int64_t row_z =
-        flash_split_id(flash_linear_id(), p.cu_q ? p.Hkv : p.B * p.Hkv, &col);
-    const int64_t row = flash_split_id(row_z, gridDim.z, &z);
+    // parts z; see flash_sched.hpp.  Where blocks weigh differently (causal: lower key blocks
+    // are heavier) the parts of a block are neighbours, so that heavier blocks still go
+    // first; where they do not, the parts stay apart (6 x 16 / 2 heads, 2089 tokens, 3 group
+    // parts, not causal: 717 us against 725 -- workgroups at one time share their Q and dO).
+    int col = blockIdx.x, z = blockIdx.z;
+    int64_t row = blockIdx.y;
+    if (CAUSAL || p.cu_q)
+        row = flash_split_id(flash_split_id(flash_linear_id(), p.cu_q ? p.Hkv : p.B * p.Hkv, &col),
+                             gridDim.z, &z);
     int b = col / p.Hkv, kblk = (int)row;
     if (p.cu_q && !varlen_item<true, CAUSAL, FbKv<D>::BLOCK>(
                       p.cu_q, p.cu_k, p.B, p.total_q, p.total_k, p.Sq, p.Sk, row, &b, &kblk))
