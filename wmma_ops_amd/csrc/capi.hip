@@ -796,6 +796,18 @@ static void flash_pack_groups(int causal, int* H, int Hkv, int* Sq) {
     *H = Hkv;
 }
 
+// Key-range split of a dense forward after flash_pack_groups, and its partial sums' bytes.
+static size_t flash_fwd_split(int B, int H, int Hkv, int Sq, int Sk, int D, bool decode, int* split) {
+    const int cus = current_cus();
+    if (decode) {
+        const int64_t units = (int64_t)B * H;
+        *split = flash_decode_split(units, Sq, Sk, D, cus);
+        return flash_decode_workspace_bytes(units, Sq, Sk, D, *split);
+    }
+    *split = flash_kv_split(B, H, Hkv, Sq, Sk, D, cus);
+    return flash_fwd_workspace_bytes(B, H, Sq, Sk, D, *split);
+}
+
 // Dense forward; `workspace` (may be NULL) enables the key-range split when it holds the
 // split's partial sums.
 static int flash_fwd_run(const void* Q, const void* K, const void* V, void* O, float* lse, int B,
@@ -823,9 +835,10 @@ static int flash_fwd_run(const void* Q, const void* K, const void* V, void* O, f
     f.causal = causal != 0;
     f.lse = lse;
     flash_pack_groups(causal, &f.H, f.Hkv, &f.Sq);
+    const bool decode = flash_decode_takes(f.Sq, causal != 0);
     if (workspace) {
-        const int split = flash_kv_split(B, f.H, Hkv, f.Sq, Sk, D, current_cus());
-        const size_t need = flash_fwd_workspace_bytes(B, f.H, f.Sq, Sk, D, split);
+        int split;
+        const size_t need = flash_fwd_split(B, f.H, Hkv, f.Sq, Sk, D, decode, &split);
         if (split > 1 && workspace_bytes >= need) {
             if (!aligned16(workspace))
                 return fail(WMMA_ERR_MISALIGNED, "workspace must be 16-byte aligned");
@@ -833,6 +846,8 @@ static int flash_fwd_run(const void* Q, const void* K, const void* V, void* O, f
             f.workspace = workspace;
         }
     }
+    if (decode)
+        return hip_status(launch_flash_decode(f, static_cast<hipStream_t>(stream)), "flash launch");
     return hip_status(launch_flash_fwd(f, static_cast<hipStream_t>(stream)), "flash launch");
 }
 
@@ -848,8 +863,8 @@ size_t wmma_flash_attn_fwd_workspace_size(int B, int H, int Hkv, int Sq, int Sk,
         D % 8 != 0 || D > kFlashMaxDFwd)
         return 0;
     flash_pack_groups(causal, &H, Hkv, &Sq);
-    return flash_fwd_workspace_bytes(B, H, Sq, Sk, D,
-                                     flash_kv_split(B, H, Hkv, Sq, Sk, D, current_cus()));
+    int split;
+    return flash_fwd_split(B, H, Hkv, Sq, Sk, D, flash_decode_takes(Sq, causal != 0), &split);
 }
 
 int wmma_flash_attn_fwd_ws(const void* Q, const void* K, const void* V, void* O, float* lse,

@@ -639,13 +639,18 @@ hipError_t launch_flash_fwd(const FlashLaunch& f, hipStream_t stream) {
         launch_d<128>(a, BH, f.causal, stream);
     else
         launch_d<64>(a, BH, f.causal, stream);
-    if (a.kv_chunk == 0) return hipGetLastError();
-    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    const int64_t rows = (int64_t)BH * f.Sq;
-    const int64_t threads = rows * (f.D / 4);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || a.kv_chunk == 0) return e;
+    return launch_flash_combine(a.o_part, a.ml_part, ceil_div(f.Sk, a.kv_chunk), (int64_t)BH * f.Sq,
+                                f.D, f.O, f.lse, stream);
+}
+
+hipError_t launch_flash_combine(const float* o_part, const float* ml_part, int split, int64_t rows,
+                                int D, void* O, float* lse, hipStream_t stream) {
+    const int64_t threads = rows * (D / 4);
     const int grid = (int)std::min<int64_t>(ceil_div64(threads, 256), 8192);
-    hipLaunchKernelGGL(flash_combine_kernel, dim3(grid), dim3(256), 0, stream, a.o_part, a.ml_part,
-                       ceil_div(f.Sk, a.kv_chunk), rows, f.D, a.O, f.lse);
+    hipLaunchKernelGGL(flash_combine_kernel, dim3(grid), dim3(256), 0, stream, o_part, ml_part,
+                       split, rows, D, static_cast<f16*>(O), lse);
     return hipGetLastError();
 }
 

@@ -147,6 +147,19 @@ int flash_kv_split(int B, int H, int Hkv, int Sq, int Sk, int D, int num_cus);
 // Workspace bytes of a split (0 for split <= 1); D is the head dim passed to the kernels.
 size_t flash_fwd_workspace_bytes(int B, int H, int Sq, int Sk, int D, int split);
 
+// Merges `split` chunks of a split key range (flash_fwd.hip): o_part [split][rows][D], ml_part
+// [split][rows][2] -> O [rows][D], lse [rows] (may be NULL).
+hipError_t launch_flash_combine(const float* o_part, const float* ml_part, int split, int64_t rows,
+                                int D, void* O, float* lse, hipStream_t stream);
+
+// Decoding shapes (flash_decode.hip): dense, not causal, at most 32 query rows per key/value
+// head after the query heads of a group are packed (f.H key/value heads of f.Sq rows).
+// kv_split / workspace as for launch_flash_fwd, sized by flash_decode_workspace_bytes.
+bool flash_decode_takes(int Sq, bool causal);
+int flash_decode_split(int64_t units, int Sq, int Sk, int D, int num_cus);
+size_t flash_decode_workspace_bytes(int64_t units, int Sq, int Sk, int D, int split);
+hipError_t launch_flash_decode(const FlashLaunch& f, hipStream_t stream);
+
 // Flash-attention backward: dQ, dK, dV (fp16, the layouts of Q, K, V) from dO, Q, K, V, O
 // and the forward's log-sum-exp.  ws: fp32 workspace of 2 * flash_bwd_workspace_rows().
 struct FlashBwdLaunch {
