@@ -419,6 +419,49 @@ int wmma_flash_attn_varlen_fwd_lse(const void* Q, const void* K, const void* V, 
                                    int D, float scale, int causal, void* stream);
 
 /*
+ * Attention on tensors as a program's views hold them -- heads split off a projection's
+ * [B,S,H,D] output, or slices of a fused one.  Elements from one batch entry, head and row
+ * to the next (`batch` is not used by the packed entry points); the D elements of a row are
+ * contiguous.  All multiples of 8, K and V with equal row strides, and in the backward pass
+ * Q and dO too; the rows of one head within 2^31 bytes.  O, lse and the gradients are
+ * contiguous as in the entry points above, whose results these return.  No counterpart in
+ * the reference.
+ */
+typedef struct wmma_attn_strides {
+    int64_t batch, head, row;
+} wmma_attn_strides;
+
+size_t wmma_flash_attn_fwd_strided_workspace_size(wmma_attn_strides q, int B, int H, int Hkv, int Sq,
+                                                  int Sk, int D, int causal);
+int wmma_flash_attn_fwd_strided(const void* Q, wmma_attn_strides q, const void* K,
+                                wmma_attn_strides k, const void* V, wmma_attn_strides v, void* O,
+                                float* lse, int B, int H, int Hkv, int Sq, int Sk, int D,
+                                float scale, int causal, void* workspace, size_t workspace_bytes,
+                                void* stream);
+int wmma_flash_attn_varlen_fwd_strided(const void* Q, wmma_attn_strides q, const void* K,
+                                       wmma_attn_strides k, const void* V, wmma_attn_strides v,
+                                       void* O, float* lse, const int32_t* cu_seqlens_q,
+                                       const int32_t* cu_seqlens_k, int B, int H, int Hkv,
+                                       int total_q, int total_k, int max_seqlen_q,
+                                       int max_seqlen_k, int D, float scale, int causal,
+                                       void* stream);
+int wmma_flash_attn_bwd_strided(const void* dO, wmma_attn_strides dout, const void* Q,
+                                wmma_attn_strides q, const void* K, wmma_attn_strides k,
+                                const void* V, wmma_attn_strides v, const void* O, const float* lse,
+                                void* dQ, void* dK, void* dV, void* workspace,
+                                size_t workspace_bytes, int B, int H, int Hkv, int Sq, int Sk,
+                                int D, float scale, int causal, void* stream);
+int wmma_flash_attn_varlen_bwd_strided(const void* dO, wmma_attn_strides dout, const void* Q,
+                                       wmma_attn_strides q, const void* K, wmma_attn_strides k,
+                                       const void* V, wmma_attn_strides v, const void* O,
+                                       const float* lse, void* dQ, void* dK, void* dV,
+                                       const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                       void* workspace, size_t workspace_bytes, int B, int H,
+                                       int Hkv, int total_q, int total_k, int max_seqlen_q,
+                                       int max_seqlen_k, int D, float scale, int causal,
+                                       void* stream);
+
+/*
  * Bytes of fp32 workspace wmma_flash_attn_bwd needs: 2 * 4 * B * H * Sq (two row
  * statistics per query row).  For the variable-length backward pass B = 1, Sq = total_q.
  */

@@ -790,10 +790,35 @@ bool aligned4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0
 // exactly as before, and each K/V tile is read once per group instead of once per query
 // head (for decoding, H/Hkv times fewer bytes).  A causal mask depends on the row's position
 // in its own head's sequence, so causal shapes keep one sequence per query head.
-static void flash_pack_groups(int causal, int* H, int Hkv, int* Sq) {
+static void flash_pack_groups(int causal, int* H, int Hkv, int* Sq, AttnStrides* q) {
     if (causal || Hkv <= 0 || *H <= Hkv || (int64_t)*Sq * (*H / Hkv) > INT32_MAX) return;
+    // the rows of a group's heads must be one run of rows (a single query per head: its heads)
+    if (*Sq == 1)
+        q->row = q->head;
+    else if (q->head != *Sq * q->row)
+        return;
+    // 32-bit offsets inside the run
+    if ((int64_t)*Sq * (*H / Hkv) * q->row * 2 > kMaxOffset) return;
+    q->head *= *H / Hkv;
     *Sq *= *H / Hkv;
     *H = Hkv;
+}
+
+// Strides of the query and key sides of an attention call: 16-byte vectors everywhere, one
+// row stride per side, and a head's rows within 32-bit offsets.
+static int flash_stride_check(const AttnStrides* tensors, int n, int64_t rows, const char* what) {
+    for (int i = 0; i < n; ++i) {
+        const AttnStrides& t = tensors[i];
+        if (t.batch < 0 || t.head < 0 || t.row < 0 || t.batch % 8 || t.head % 8 || t.row % 8)
+            return fail(WMMA_ERR_MISALIGNED, "%s strides must be multiples of 8", what);
+        if (t.head / 8 > (int64_t)UINT32_MAX)
+            return fail(WMMA_ERR_UNSUPPORTED, "%s head stride too large", what);
+        if (t.row != tensors[0].row)
+            return fail(WMMA_ERR_UNSUPPORTED, "%s must have one row stride", what);
+        if (std::max<int64_t>(rows, 64) * t.row * 2 > kMaxOffset)
+            return fail(WMMA_ERR_UNSUPPORTED, "sequence too long for 32-bit offsets");
+    }
+    return WMMA_OK;
 }
 
 // Key-range split of a dense forward after flash_pack_groups, and its partial sums' bytes.
@@ -810,9 +835,10 @@ static size_t flash_fwd_split(int B, int H, int Hkv, int Sq, int Sk, int D, bool
 
 // Dense forward; `workspace` (may be NULL) enables the key-range split when it holds the
 // split's partial sums.
-static int flash_fwd_run(const void* Q, const void* K, const void* V, void* O, float* lse, int B,
-                         int H, int Hkv, int Sq, int Sk, int D, float scale, int causal,
-                         void* workspace, size_t workspace_bytes, void* stream) {
+static int flash_fwd_run(const void* Q, AttnStrides q, const void* K, AttnStrides k, const void* V,
+                         AttnStrides v, void* O, float* lse, int B, int H, int Hkv, int Sq, int Sk,
+                         int D, float scale, int causal, void* workspace, size_t workspace_bytes,
+                         void* stream) {
     if (int rc = flash_dense_check(B, H, Hkv, Sq, Sk, D, scale, kFlashMaxDFwd)) return rc;
     if (B == 0 || H == 0 || Sq == 0) return ok();
     if (Sk == 0) return fail(WMMA_ERR_INVALID_ARG, "Sk must be positive when Sq > 0");
@@ -834,8 +860,11 @@ static int flash_fwd_run(const void* Q, const void* K, const void* V, void* O, f
     f.scale = scale;
     f.causal = causal != 0;
     f.lse = lse;
-    flash_pack_groups(causal, &f.H, f.Hkv, &f.Sq);
-    const bool decode = flash_decode_takes(f.Sq, causal != 0);
+    f.q = q;
+    f.k = k;
+    f.v = v;
+    flash_pack_groups(causal, &f.H, f.Hkv, &f.Sq, &f.q);
+    const bool decode = f.H == f.Hkv && flash_decode_takes(f.Sq, causal != 0);
     if (workspace) {
         int split;
         const size_t need = flash_fwd_split(B, f.H, Hkv, f.Sq, Sk, D, decode, &split);
@@ -851,10 +880,27 @@ static int flash_fwd_run(const void* Q, const void* K, const void* V, void* O, f
     return hip_status(launch_flash_fwd(f, static_cast<hipStream_t>(stream)), "flash launch");
 }
 
+// The same on contiguous tensors.
+static int flash_fwd_dense(const void* Q, const void* K, const void* V, void* O, float* lse, int B,
+                           int H, int Hkv, int Sq, int Sk, int D, float scale, int causal,
+                           void* workspace, size_t workspace_bytes, void* stream) {
+    const AttnStrides kv = dense_strides(Hkv, Sk, D);
+    return flash_fwd_run(Q, dense_strides(H, Sq, D), K, kv, V, kv, O, lse, B, H, Hkv, Sq, Sk, D,
+                         scale, causal, workspace, workspace_bytes, stream);
+}
+
 int wmma_flash_attn_fwd_lse(const void* Q, const void* K, const void* V, void* O, float* lse,
                             int B, int H, int Hkv, int Sq, int Sk, int D, float scale, int causal,
                             void* stream) {
-    return flash_fwd_run(Q, K, V, O, lse, B, H, Hkv, Sq, Sk, D, scale, causal, nullptr, 0, stream);
+    return flash_fwd_dense(Q, K, V, O, lse, B, H, Hkv, Sq, Sk, D, scale, causal, nullptr, 0, stream);
+}
+
+static size_t flash_fwd_strided_workspace(AttnStrides q, int B, int H, int Hkv, int Sq, int Sk, int D,
+                                          int causal) {
+    flash_pack_groups(causal, &H, Hkv, &Sq, &q);
+    int split;
+    return flash_fwd_split(B, H, Hkv, Sq, Sk, D, H == Hkv && flash_decode_takes(Sq, causal != 0),
+                           &split);
 }
 
 size_t wmma_flash_attn_fwd_workspace_size(int B, int H, int Hkv, int Sq, int Sk, int D,
@@ -862,15 +908,33 @@ size_t wmma_flash_attn_fwd_workspace_size(int B, int H, int Hkv, int Sq, int Sk,
     if (B <= 0 || H <= 0 || Hkv <= 0 || H % Hkv != 0 || Sq <= 0 || Sk <= 0 || D <= 0 ||
         D % 8 != 0 || D > kFlashMaxDFwd)
         return 0;
-    flash_pack_groups(causal, &H, Hkv, &Sq);
-    int split;
-    return flash_fwd_split(B, H, Hkv, Sq, Sk, D, flash_decode_takes(Sq, causal != 0), &split);
+    return flash_fwd_strided_workspace(dense_strides(H, Sq, D), B, H, Hkv, Sq, Sk, D, causal);
+}
+
+size_t wmma_flash_attn_fwd_strided_workspace_size(wmma_attn_strides q, int B, int H, int Hkv, int Sq,
+                                                  int Sk, int D, int causal) {
+    if (B <= 0 || H <= 0 || Hkv <= 0 || H % Hkv != 0 || Sq <= 0 || Sk <= 0 || D <= 0 ||
+        D % 8 != 0 || D > kFlashMaxDFwd)
+        return 0;
+    return flash_fwd_strided_workspace(q, B, H, Hkv, Sq, Sk, D, causal);
+}
+
+int wmma_flash_attn_fwd_strided(const void* Q, wmma_attn_strides q, const void* K,
+                                wmma_attn_strides k, const void* V, wmma_attn_strides v, void* O,
+                                float* lse, int B, int H, int Hkv, int Sq, int Sk, int D,
+                                float scale, int causal, void* workspace, size_t workspace_bytes,
+                                void* stream) {
+    const AttnStrides kv[2] = {k, v};
+    if (int rc = flash_stride_check(&q, 1, Sq, "Q")) return rc;
+    if (int rc = flash_stride_check(kv, 2, Sk, "K and V")) return rc;
+    return flash_fwd_run(Q, q, K, k, V, v, O, lse, B, H, Hkv, Sq, Sk, D, scale, causal, workspace,
+                         workspace_bytes, stream);
 }
 
 int wmma_flash_attn_fwd_ws(const void* Q, const void* K, const void* V, void* O, float* lse,
                            int B, int H, int Hkv, int Sq, int Sk, int D, float scale, int causal,
                            void* workspace, size_t workspace_bytes, void* stream) {
-    return flash_fwd_run(Q, K, V, O, lse, B, H, Hkv, Sq, Sk, D, scale, causal, workspace,
+    return flash_fwd_dense(Q, K, V, O, lse, B, H, Hkv, Sq, Sk, D, scale, causal, workspace,
                          workspace_bytes, stream);
 }
 
@@ -879,11 +943,11 @@ int wmma_flash_attn_fwd_gqa(const void* Q, const void* K, const void* V, void* O
     return wmma_flash_attn_fwd_lse(Q, K, V, O, nullptr, B, H, Hkv, Sq, Sk, D, scale, causal, stream);
 }
 
-int wmma_flash_attn_varlen_fwd_lse(const void* Q, const void* K, const void* V, void* O,
-                                   float* lse, const int32_t* cu_seqlens_q,
-                                   const int32_t* cu_seqlens_k, int B, int H, int Hkv,
-                                   int total_q, int total_k, int max_seqlen_q, int max_seqlen_k,
-                                   int D, float scale, int causal, void* stream) {
+static int flash_varlen_fwd_run(const void* Q, AttnStrides q, const void* K, AttnStrides k,
+                                const void* V, AttnStrides v, void* O, float* lse,
+                                const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int B,
+                                int H, int Hkv, int total_q, int total_k, int max_seqlen_q,
+                                int max_seqlen_k, int D, float scale, int causal, void* stream) {
     if (int rc = flash_varlen_check(B, H, Hkv, total_q, total_k, max_seqlen_q, max_seqlen_k, D,
                                     scale, kFlashMaxDFwd))
         return rc;
@@ -913,7 +977,37 @@ int wmma_flash_attn_varlen_fwd_lse(const void* Q, const void* K, const void* V, 
     f.total_q = total_q;
     f.total_k = total_k;
     f.lse = lse;
+    f.q = q;
+    f.k = k;
+    f.v = v;
     return hip_status(launch_flash_fwd(f, static_cast<hipStream_t>(stream)), "flash launch");
+}
+
+int wmma_flash_attn_varlen_fwd_lse(const void* Q, const void* K, const void* V, void* O,
+                                   float* lse, const int32_t* cu_seqlens_q,
+                                   const int32_t* cu_seqlens_k, int B, int H, int Hkv,
+                                   int total_q, int total_k, int max_seqlen_q, int max_seqlen_k,
+                                   int D, float scale, int causal, void* stream) {
+    const AttnStrides kv = packed_strides(Hkv, D);
+    return flash_varlen_fwd_run(Q, packed_strides(H, D), K, kv, V, kv, O, lse, cu_seqlens_q,
+                                cu_seqlens_k, B, H, Hkv, total_q, total_k, max_seqlen_q,
+                                max_seqlen_k, D, scale, causal, stream);
+}
+
+int wmma_flash_attn_varlen_fwd_strided(const void* Q, wmma_attn_strides q, const void* K,
+                                       wmma_attn_strides k, const void* V, wmma_attn_strides v,
+                                       void* O, float* lse, const int32_t* cu_seqlens_q,
+                                       const int32_t* cu_seqlens_k, int B, int H, int Hkv,
+                                       int total_q, int total_k, int max_seqlen_q,
+                                       int max_seqlen_k, int D, float scale, int causal,
+                                       void* stream) {
+    q.batch = k.batch = v.batch = 0;
+    const AttnStrides kv[2] = {k, v};
+    if (int rc = flash_stride_check(&q, 1, max_seqlen_q, "Q")) return rc;
+    if (int rc = flash_stride_check(kv, 2, max_seqlen_k, "K and V")) return rc;
+    return flash_varlen_fwd_run(Q, q, K, k, V, v, O, lse, cu_seqlens_q, cu_seqlens_k, B, H, Hkv,
+                                total_q, total_k, max_seqlen_q, max_seqlen_k, D, scale, causal,
+                                stream);
 }
 
 int wmma_flash_attn_varlen_fwd(const void* Q, const void* K, const void* V, void* O,
@@ -981,10 +1075,11 @@ size_t wmma_flash_attn_bwd_split_workspace_size(int B, int H, int Hkv, int Sq, i
     return gs > 1 ? round256(need) + flash_bwd_split_bytes(B, Hkv, Sk, D, gs) : need;
 }
 
-int wmma_flash_attn_bwd(const void* dO, const void* Q, const void* K, const void* V, const void* O,
-                        const float* lse, void* dQ, void* dK, void* dV, void* workspace,
-                        size_t workspace_bytes, int B, int H, int Hkv, int Sq, int Sk, int D,
-                        float scale, int causal, void* stream) {
+static int flash_bwd_dense_run(const void* dO, AttnStrides dout, const void* Q, AttnStrides q,
+                               const void* K, AttnStrides k, const void* V, AttnStrides v,
+                               const void* O, const float* lse, void* dQ, void* dK, void* dV,
+                               void* workspace, size_t workspace_bytes, int B, int H, int Hkv,
+                               int Sq, int Sk, int D, float scale, int causal, void* stream) {
     if (int rc = flash_dense_check(B, H, Hkv, Sq, Sk, D, scale, kFlashMaxDBwd)) return rc;
     if (B == 0 || H == 0 || (Sq == 0 && Sk == 0)) return ok();
     if (Sk == 0) return fail(WMMA_ERR_INVALID_ARG, "Sk must be positive when Sq > 0");
@@ -1006,15 +1101,42 @@ int wmma_flash_attn_bwd(const void* dO, const void* Q, const void* K, const void
     f.D = D;
     f.scale = scale;
     f.causal = causal != 0;
+    f.q = q;
+    f.k = k;
+    f.v = v;
+    f.dout = dout;
     return flash_bwd_run(f, workspace, workspace_bytes, stream);
 }
 
-int wmma_flash_attn_varlen_bwd(const void* dO, const void* Q, const void* K, const void* V,
-                               const void* O, const float* lse, void* dQ, void* dK, void* dV,
-                               const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
-                               void* workspace, size_t workspace_bytes, int B, int H, int Hkv,
-                               int total_q, int total_k, int max_seqlen_q, int max_seqlen_k,
-                               int D, float scale, int causal, void* stream) {
+int wmma_flash_attn_bwd(const void* dO, const void* Q, const void* K, const void* V, const void* O,
+                        const float* lse, void* dQ, void* dK, void* dV, void* workspace,
+                        size_t workspace_bytes, int B, int H, int Hkv, int Sq, int Sk, int D,
+                        float scale, int causal, void* stream) {
+    const AttnStrides q = dense_strides(H, Sq, D), kv = dense_strides(Hkv, Sk, D);
+    return flash_bwd_dense_run(dO, q, Q, q, K, kv, V, kv, O, lse, dQ, dK, dV, workspace,
+                               workspace_bytes, B, H, Hkv, Sq, Sk, D, scale, causal, stream);
+}
+
+int wmma_flash_attn_bwd_strided(const void* dO, wmma_attn_strides dout, const void* Q,
+                                wmma_attn_strides q, const void* K, wmma_attn_strides k,
+                                const void* V, wmma_attn_strides v, const void* O, const float* lse,
+                                void* dQ, void* dK, void* dV, void* workspace,
+                                size_t workspace_bytes, int B, int H, int Hkv, int Sq, int Sk,
+                                int D, float scale, int causal, void* stream) {
+    const AttnStrides qd[2] = {q, dout}, kv[2] = {k, v};
+    if (int rc = flash_stride_check(qd, 2, Sq, "Q and dO")) return rc;
+    if (int rc = flash_stride_check(kv, 2, Sk, "K and V")) return rc;
+    return flash_bwd_dense_run(dO, dout, Q, q, K, k, V, v, O, lse, dQ, dK, dV, workspace,
+                               workspace_bytes, B, H, Hkv, Sq, Sk, D, scale, causal, stream);
+}
+
+static int flash_varlen_bwd_run(const void* dO, AttnStrides dout, const void* Q, AttnStrides q,
+                                const void* K, AttnStrides k, const void* V, AttnStrides v,
+                                const void* O, const float* lse, void* dQ, void* dK, void* dV,
+                                const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                void* workspace, size_t workspace_bytes, int B, int H, int Hkv,
+                                int total_q, int total_k, int max_seqlen_q, int max_seqlen_k,
+                                int D, float scale, int causal, void* stream) {
     if (int rc = flash_varlen_check(B, H, Hkv, total_q, total_k, max_seqlen_q, max_seqlen_k, D,
                                     scale, kFlashMaxDBwd))
         return rc;
@@ -1040,11 +1162,45 @@ int wmma_flash_attn_varlen_bwd(const void* dO, const void* Q, const void* K, con
     f.D = D;
     f.scale = scale;
     f.causal = causal != 0;
+    f.q = q;
+    f.k = k;
+    f.v = v;
+    f.dout = dout;
     f.cu_q = cu_seqlens_q;
     f.cu_k = cu_seqlens_k;
     f.total_q = total_q;
     f.total_k = total_k;
     return flash_bwd_run(f, workspace, workspace_bytes, stream);
+}
+
+int wmma_flash_attn_varlen_bwd(const void* dO, const void* Q, const void* K, const void* V,
+                               const void* O, const float* lse, void* dQ, void* dK, void* dV,
+                               const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                               void* workspace, size_t workspace_bytes, int B, int H, int Hkv,
+                               int total_q, int total_k, int max_seqlen_q, int max_seqlen_k,
+                               int D, float scale, int causal, void* stream) {
+    const AttnStrides q = packed_strides(H, D), kv = packed_strides(Hkv, D);
+    return flash_varlen_bwd_run(dO, q, Q, q, K, kv, V, kv, O, lse, dQ, dK, dV, cu_seqlens_q,
+                                cu_seqlens_k, workspace, workspace_bytes, B, H, Hkv, total_q,
+                                total_k, max_seqlen_q, max_seqlen_k, D, scale, causal, stream);
+}
+
+int wmma_flash_attn_varlen_bwd_strided(const void* dO, wmma_attn_strides dout, const void* Q,
+                                       wmma_attn_strides q, const void* K, wmma_attn_strides k,
+                                       const void* V, wmma_attn_strides v, const void* O,
+                                       const float* lse, void* dQ, void* dK, void* dV,
+                                       const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                       void* workspace, size_t workspace_bytes, int B, int H,
+                                       int Hkv, int total_q, int total_k, int max_seqlen_q,
+                                       int max_seqlen_k, int D, float scale, int causal,
+                                       void* stream) {
+    q.batch = k.batch = v.batch = dout.batch = 0;
+    const AttnStrides qd[2] = {q, dout}, kv[2] = {k, v};
+    if (int rc = flash_stride_check(qd, 2, max_seqlen_q, "Q and dO")) return rc;
+    if (int rc = flash_stride_check(kv, 2, max_seqlen_k, "K and V")) return rc;
+    return flash_varlen_bwd_run(dO, dout, Q, q, K, k, V, v, O, lse, dQ, dK, dV, cu_seqlens_q,
+                                cu_seqlens_k, workspace, workspace_bytes, B, H, Hkv, total_q,
+                                total_k, max_seqlen_q, max_seqlen_k, D, scale, causal, stream);
 }
 
 }  // extern "C"

@@ -156,6 +156,7 @@ struct BwdArgs {
     int64_t rows;      // query rows of lse: B*H*Sq dense, H*total_q variable length
     int Sq, Sk;
     int nqb;           // 256-query blocks (dQ kernel)
+    int grid_y;
     float c;           // scale * log2(e)
     float scale;
     int group;         // query heads per key/value head
@@ -163,9 +164,13 @@ struct BwdArgs {
                        // (d columns dr .. D-1 load as zeros and are not stored)
     const int* cu_q;   // variable length (nullptr: dense), as in the forward
     const int* cu_k;
+    bool ordered;      // variable length: items in the order of flash_sched.hpp
     int B;             // batch entries (sequences)
     int H, Hkv;
     int total_q, total_k;
+    ChunkStrides q, k, v, dout;  // q.row == dout.row, k.row == v.row
+    ChunkStrides o, dkv;         // contiguous: O and dQ; dK, dV and the group parts
+    FastDiv div_h, div_hkv, div_group, div_bh, div_bhkv, div_z;
     // Grouped-query split of the dK/dV kernel (dense layout; gsplit = 1: none): part gp of
     // blockIdx.z / DSPLIT takes query heads [gp gper, (gp + 1) gper) of the group and
     // writes fp32 partial dK, dV (scaled as the final ones) to kv_part[gp] and
@@ -177,34 +182,43 @@ struct BwdArgs {
 
 // Geometry of one (batch entry, query head): lengths, row strides (elements) and bases.
 struct SeqGeo {
-    int Sq, Sk, qs, ks;
-    int64_t q_base, k_base, r_base;  // Q/O/dO element base, K/V element base, lse row base
+    int Sq, Sk;
+    int qs, ks, os, dks;             // row strides of Q and dO, K and V, O and dQ, dK and dV
+    int64_t q_base, do_base, k_base, v_base;  // element bases
+    int64_t o_base, dk_base;
+    int64_t r_base;                  // lse row base
 };
 
-template <int D>
+template <int D, bool VARLEN>
 __device__ __forceinline__ SeqGeo seq_geo(const BwdArgs& p, int b, int hq) {
     SeqGeo g;
-    if (p.cu_q) {
+    int q_row = 0, k_row = 0;  // first query and key row
+    const int hk = div_by(p.div_group, hq);
+    if constexpr (VARLEN) {
         const int qa = min(max(p.cu_q[b], 0), p.total_q);
         const int qe = min(max(p.cu_q[b + 1], qa), p.total_q);
         const int ka = min(max(p.cu_k[b], 0), p.total_k);
         const int ke = min(max(p.cu_k[b + 1], ka), p.total_k);
         g.Sq = min(qe - qa, p.Sq);
         g.Sk = min(ke - ka, p.Sk);
-        g.qs = p.H * p.dr;
-        g.ks = p.Hkv * p.dr;
-        g.q_base = (int64_t)qa * g.qs + (int64_t)hq * p.dr;
-        g.k_base = (int64_t)ka * g.ks + (int64_t)(hq / p.group) * p.dr;
+        q_row = qa;
+        k_row = ka;
         g.r_base = (int64_t)hq * p.total_q + qa;
     } else {
         g.Sq = p.Sq;
         g.Sk = p.Sk;
-        g.qs = p.dr;
-        g.ks = p.dr;
-        g.q_base = ((int64_t)b * p.H + hq) * p.Sq * p.dr;
-        g.k_base = ((int64_t)b * p.Hkv + hq / p.group) * p.Sk * p.dr;
         g.r_base = ((int64_t)b * p.H + hq) * p.Sq;
     }
+    g.qs = p.q.row_elems();
+    g.ks = p.k.row_elems();
+    g.os = p.o.row_elems();
+    g.dks = p.dkv.row_elems();
+    g.q_base = p.q.at(b, hq, q_row);
+    g.do_base = p.dout.at(b, hq, q_row);
+    g.o_base = p.o.at(b, hq, q_row);
+    g.k_base = p.k.at(b, hk, k_row);
+    g.v_base = p.v.at(b, hk, k_row);
+    g.dk_base = p.dkv.at(b, hk, k_row);
     return g;
 }
 
@@ -421,7 +435,8 @@ __device__ __forceinline__ void fb_dq_iter(const WMMA_LDS unsigned char* __restr
     }
 }
 
-template <int D, bool CAUSAL>
+// VARLEN is a kernel of its own, as in the forward.
+template <int D, bool CAUSAL, bool VARLEN>
 __global__ void __launch_bounds__(FbGeom<D>::WQ * kWave)
 __attribute__((amdgpu_waves_per_eu(FbGeom<D>::WQ / 4, FbGeom<D>::WQ / 4)))
 flash_bwd_dq_kernel(BwdArgs p) {
@@ -436,25 +451,28 @@ flash_bwd_dq_kernel(BwdArgs p) {
     // Which query block of which (batch, head): see flash_sched.hpp.
     int col = blockIdx.x;
     int64_t row = blockIdx.y;
-    if (CAUSAL || p.cu_q) row = flash_split_id(flash_linear_id(), p.cu_q ? p.H : p.B * p.H, &col);
-    int b = col / p.H, qb_idx = CAUSAL ? p.nqb - 1 - (int)row : (int)row;
-    if (p.cu_q && !varlen_item<false, CAUSAL, FbGeom<D>::BLOCK_Q>(
+    const bool ordered = VARLEN && p.ordered;
+    if (ordered || CAUSAL)
+        row = flash_split_id(flash_linear_id(p.div_bh.d, p.grid_y), ordered ? p.div_h : p.div_bh, &col);
+    int b = div_by(p.div_h, col), qb_idx = CAUSAL ? p.nqb - 1 - (int)row : (int)row;
+    if (ordered && !varlen_item<false, CAUSAL, FbGeom<D>::BLOCK_Q>(
                       p.cu_q, p.cu_k, p.B, p.total_q, p.total_k, p.Sq, p.Sk, row, &b, &qb_idx))
         return;
     const int q0 = qb_idx * FbGeom<D>::BLOCK_Q;
     const int qw = q0 + wave * FB_ROWS;
-    const SeqGeo G = seq_geo<D>(p, b, col % p.H);
+    const SeqGeo G = seq_geo<D, VARLEN>(p, b, ordered ? col : col - b * p.H);
+    if (VARLEN && q0 >= G.Sq) return;
     const int Sq = G.Sq, Sk = G.Sk;
     const int qrow = qw + c32;
 
     f16x8 qf[C::NDS], dof[C::NDS];
     fb_load_frag<D>(p.Q + G.q_base, G.qs, p.dr, qrow, Sq, h, qf);
-    fb_load_frag<D>(p.dO + G.q_base, G.qs, p.dr, qrow, Sq, h, dof);
+    fb_load_frag<D>(p.dO + G.do_base, G.qs, p.dr, qrow, Sq, h, dof);
     // Delta = rowsum(dO o O): this lane's 64 d values, then the other half of the row.
     float delta;
     {
         f16x8 of[C::NDS];
-        fb_load_frag<D>(p.O + G.q_base, G.qs, p.dr, qrow, Sq, h, of);
+        fb_load_frag<D>(p.O + G.o_base, G.os, p.dr, qrow, Sq, h, of);
         float acc[2] = {0.0f, 0.0f};
 #pragma unroll
         for (int ds = 0; ds < C::NDS; ++ds)
@@ -479,7 +497,7 @@ flash_bwd_dq_kernel(BwdArgs p) {
     FbLane<D, FbGeom<D>::WQ> L;
     fb_lane_init<D>(L, wave, lane, G.ks, p.dr);
     const f16* Kb = p.K + G.k_base;
-    const f16* Vb = p.V + G.k_base;
+    const f16* Vb = p.V + G.v_base;
     const int kv_end = CAUSAL ? min(Sk, q0 + FbGeom<D>::BLOCK_Q) : Sk;
     const int T = (kv_end + FB_T - 1) / FB_T;
     const int Tw = CAUSAL ? min(T, (qw + FB_ROWS - 1) / FB_T + 1) : T;
@@ -509,7 +527,7 @@ flash_bwd_dq_kernel(BwdArgs p) {
         }
         wait_vmcnt<0>();
     }
-    fb_store_rows<C::NDB>(p.dQ + G.q_base, G.qs, p.dr, qrow, Sq, h, dq, p.scale);
+    fb_store_rows<C::NDB>(p.dQ + G.o_base, G.os, p.dr, qrow, Sq, h, dq, p.scale);
 }
 
 // ------------------------------------------------------------------------- dK/dV kernel --
@@ -652,7 +670,7 @@ __device__ __forceinline__ void fb_kv_iter(const WMMA_LDS unsigned char* __restr
     }
 }
 
-template <int D, bool CAUSAL>
+template <int D, bool CAUSAL, bool VARLEN>
 __global__ void __launch_bounds__(FB_WAVES_KV * kWave)
 __attribute__((amdgpu_waves_per_eu(FB_WAVES_KV / 4, FB_WAVES_KV / 4)))
 flash_bwd_dkdv_kernel(BwdArgs p) {
@@ -671,31 +689,34 @@ flash_bwd_dkdv_kernel(BwdArgs p) {
     // parts, not causal: 717 us against 725 -- workgroups at one time share their Q and dO).
     int col = blockIdx.x, z = blockIdx.z;
     int64_t row = blockIdx.y;
-    if (CAUSAL || p.cu_q)
-        row = flash_split_id(flash_split_id(flash_linear_id(), p.cu_q ? p.Hkv : p.B * p.Hkv, &col),
-                             gridDim.z, &z);
-    int b = col / p.Hkv, kblk = (int)row;
-    if (p.cu_q && !varlen_item<true, CAUSAL, FbKv<D>::BLOCK>(
+    const bool ordered = VARLEN && p.ordered;
+    if (ordered || CAUSAL)
+        row = flash_split_id(flash_split_id(flash_linear_id(p.div_bhkv.d, p.grid_y, p.div_z.d),
+                                            ordered ? p.div_hkv : p.div_bhkv, &col),
+                             p.div_z, &z);
+    int b = div_by(p.div_hkv, col), kblk = (int)row;
+    if (ordered && !varlen_item<true, CAUSAL, FbKv<D>::BLOCK>(
                       p.cu_q, p.cu_k, p.B, p.total_q, p.total_k, p.Sq, p.Sk, row, &b, &kblk))
         return;
-    const int j = col % p.Hkv;
+    const int j = ordered ? col : col - b * p.Hkv;
     const int k0 = kblk * FbKv<D>::BLOCK;
     const int kw = k0 + wave * FbKv<D>::ROWS;
-    const SeqGeo G0 = seq_geo<D>(p, b, j * p.group);
+    const SeqGeo G0 = seq_geo<D, VARLEN>(p, b, j * p.group);
+    if (VARLEN && k0 >= G0.Sk) return;
     const int Sq = G0.Sq, Sk = G0.Sk;
 
     f16x8 kf[FbKv<D>::KB][C::NDS], vf[FbKv<D>::KB][C::NDS];
 #pragma unroll
     for (int kb = 0; kb < FbKv<D>::KB; ++kb) {
         fb_load_frag<D>(p.K + G0.k_base, G0.ks, p.dr, kw + 32 * kb + c32, Sk, h, kf[kb]);
-        fb_load_frag<D>(p.V + G0.k_base, G0.ks, p.dr, kw + 32 * kb + c32, Sk, h, vf[kb]);
+        fb_load_frag<D>(p.V + G0.v_base, G0.ks, p.dr, kw + 32 * kb + c32, Sk, h, vf[kb]);
     }
 
     FbLane<D, FB_WAVES_KV> L;
     fb_lane_init<D>(L, wave, lane, G0.qs, p.dr);
     // Query tiles: t0 .. Tq-1 of each of this workgroup's query heads of the group in turn
     // (heads g_lo .. g_lo + ng - 1: the whole group, or one part of a grouped-query split).
-    // Head gi's rows start at q_base0 + gi * qh (Q/dO elements) and r_base0 + gi * rh
+    // Head gi's rows start gi heads further in Q and dO and at r_base0 + gi * rh
     // (statistics).
     const int gp = z / FbKv<D>::DSPLIT;
     const int g_lo = gp * p.gper;
@@ -704,12 +725,12 @@ flash_bwd_dkdv_kernel(BwdArgs p) {
     const int t0 = CAUSAL ? min(k0 / FB_T, Tq) : 0;
     const int nT = Tq - t0;
     const int U = ng * nT;
-    const int64_t qh = p.cu_q ? (int64_t)p.dr : (int64_t)Sq * p.dr;
-    const int64_t rh = p.cu_q ? (int64_t)p.total_q : (int64_t)Sq;
+    const int64_t rh = VARLEN ? (int64_t)p.total_q : (int64_t)Sq;
     const float* ws_lse = p.ws + p.rows;
     const float* ws_delta = p.ws;
     // Statistic slot source of this wave: wave 0 -L/scale, wave 1 -Delta, others nothing.
     const float* st_src = wave == 0 ? ws_lse : ws_delta;
+
     auto tile_of = [&](int u, int& gi, int& t) {
         const int uu = min(u, U - 1);
         const int gr = uu / nT;
@@ -732,13 +753,18 @@ flash_bwd_dkdv_kernel(BwdArgs p) {
     const float c = p.c;
 
     if (U > 0) {
+        auto q_rsrc = [&](int gi, int t) {
+            return make_rsrc(p.Q + G0.q_base + p.q.at(0, gi, t * FB_T));
+        };
+        auto do_rsrc = [&](int gi, int t) {
+            return make_rsrc(p.dO + G0.do_base + p.dout.at(0, gi, t * FB_T));
+        };
         auto issue = [&](WMMA_LDS unsigned char* dst, int u) {
             int gi, t;
             tile_of(u, gi, t);
-            const int64_t qoff = G0.q_base + gi * qh + (int64_t)t * FB_T * G0.qs;
             const int left = qleft(u, t);
-            fb_dma_tile<D>(dst, L, make_rsrc(p.Q + qoff), left);
-            fb_dma_tile<D>(dst + C::TILE, L, make_rsrc(p.dO + qoff), left);
+            fb_dma_tile<D>(dst, L, q_rsrc(gi, t), left);
+            fb_dma_tile<D>(dst + C::TILE, L, do_rsrc(gi, t), left);
             lds_dma4(make_rsrc(st_src + G0.r_base + gi * rh + (int64_t)t * FB_T),
                      wave < 2 && lane < left ? (uint32_t)(4 * lane) : kOobOffset,
                      dst + 2 * C::TILE + wave * C::STAT);
@@ -750,10 +776,9 @@ flash_bwd_dkdv_kernel(BwdArgs p) {
             int gi, t, gf, tf;
             tile_of(u, gi, t);
             tile_of(uf, gf, tf);
-            const int64_t qoff = G0.q_base + gf * qh + (int64_t)tf * FB_T * G0.qs;
             fb_kv_iter<D, decltype(mask_tag)::value>(
                 lds + (u % NS) * C::STAGE_KV, lds + (uf % NS) * C::STAGE_KV, L, wave,
-                make_rsrc(p.Q + qoff), make_rsrc(p.dO + qoff),
+                q_rsrc(gf, tf), do_rsrc(gf, tf),
                 make_rsrc(st_src + G0.r_base + gf * rh + (int64_t)tf * FB_T), qleft(uf, tf), kf, vf,
                 dk, dv, c, t * FB_T, kw + c32, db0);
         };
@@ -767,22 +792,22 @@ flash_bwd_dkdv_kernel(BwdArgs p) {
         wait_vmcnt<0>();
     }
     if (p.gsplit > 1) {
-        float* pk = p.kv_part + (int64_t)gp * p.kv_elems + G0.k_base;
-        float* pv = p.kv_part + (int64_t)(p.gsplit + gp) * p.kv_elems + G0.k_base;
+        float* pk = p.kv_part + (int64_t)gp * p.kv_elems + G0.dk_base;
+        float* pv = p.kv_part + (int64_t)(p.gsplit + gp) * p.kv_elems + G0.dk_base;
 #pragma unroll
         for (int kb = 0; kb < FbKv<D>::KB; ++kb) {
-            fb_store_rows_f32<NDBO>(pk, G0.ks, p.dr, kw + 32 * kb + c32, Sk, h, dk[kb], p.scale,
+            fb_store_rows_f32<NDBO>(pk, G0.dks, p.dr, kw + 32 * kb + c32, Sk, h, dk[kb], p.scale,
                                     32 * db0);
-            fb_store_rows_f32<NDBO>(pv, G0.ks, p.dr, kw + 32 * kb + c32, Sk, h, dv[kb], 1.0f,
+            fb_store_rows_f32<NDBO>(pv, G0.dks, p.dr, kw + 32 * kb + c32, Sk, h, dv[kb], 1.0f,
                                     32 * db0);
         }
         return;
     }
 #pragma unroll
     for (int kb = 0; kb < FbKv<D>::KB; ++kb) {
-        fb_store_rows<NDBO>(p.dK + G0.k_base, G0.ks, p.dr, kw + 32 * kb + c32, Sk, h, dk[kb], p.scale,
+        fb_store_rows<NDBO>(p.dK + G0.dk_base, G0.dks, p.dr, kw + 32 * kb + c32, Sk, h, dk[kb], p.scale,
                             32 * db0);
-        fb_store_rows<NDBO>(p.dV + G0.k_base, G0.ks, p.dr, kw + 32 * kb + c32, Sk, h, dv[kb], 1.0f,
+        fb_store_rows<NDBO>(p.dV + G0.dk_base, G0.dks, p.dr, kw + 32 * kb + c32, Sk, h, dv[kb], 1.0f,
                             32 * db0);
     }
 }
@@ -818,25 +843,39 @@ template <int D>
 void launch_bwd_d(BwdArgs a, int B, bool causal, hipStream_t stream) {
     a.nqb = ceil_div(a.Sq, FbGeom<D>::BLOCK_Q);
     const dim3 bq(FbGeom<D>::WQ * kWave), bk(FB_WAVES_KV * kWave);
-    const dim3 gq(B * a.H, a.cu_q ? varlen_grid_y(B, a.total_q, a.Sq, FbGeom<D>::BLOCK_Q) : a.nqb);
-    const dim3 gk(B * a.Hkv,
-                  a.cu_q ? varlen_grid_y(B, a.total_k, a.Sk, FbKv<D>::BLOCK)
-                         : ceil_div(a.Sk, FbKv<D>::BLOCK),
+    const bool order_q = a.cu_q && varlen_ordered((int64_t)B * a.H, a.nqb);
+    const int nkb = ceil_div(a.Sk, FbKv<D>::BLOCK);
+    const bool order_k = a.cu_q && varlen_ordered((int64_t)B * a.Hkv, nkb);
+    const dim3 gq(B * a.H, order_q ? varlen_grid_y(B, a.total_q, a.Sq, FbGeom<D>::BLOCK_Q) : a.nqb);
+    const dim3 gk(B * a.Hkv, order_k ? varlen_grid_y(B, a.total_k, a.Sk, FbKv<D>::BLOCK) : nkb,
                   FbKv<D>::DSPLIT * a.gsplit);
+    a.ordered = order_q;
+    a.grid_y = gq.y;
     // The dQ kernel writes the row statistics the dK/dV kernel reads: same stream, in order.
     // An empty side (no query or no key rows) launches nothing for it; with no query rows
     // the dK/dV kernel still runs and stores zeros.
     if (gq.x > 0 && gq.y > 0) {
-        if (causal)
-            hipLaunchKernelGGL((flash_bwd_dq_kernel<D, true>), gq, bq, 0, stream, a);
+        if (a.cu_q && causal)
+            hipLaunchKernelGGL((flash_bwd_dq_kernel<D, true, true>), gq, bq, 0, stream, a);
+        else if (a.cu_q)
+            hipLaunchKernelGGL((flash_bwd_dq_kernel<D, false, true>), gq, bq, 0, stream, a);
+        else if (causal)
+            hipLaunchKernelGGL((flash_bwd_dq_kernel<D, true, false>), gq, bq, 0, stream, a);
         else
-            hipLaunchKernelGGL((flash_bwd_dq_kernel<D, false>), gq, bq, 0, stream, a);
+            hipLaunchKernelGGL((flash_bwd_dq_kernel<D, false, false>), gq, bq, 0, stream, a);
     }
+    a.ordered = order_k;
+    a.grid_y = gk.y;
+    a.div_z = fast_div(gk.z);
     if (gk.x > 0 && gk.y > 0) {
-        if (causal)
-            hipLaunchKernelGGL((flash_bwd_dkdv_kernel<D, true>), gk, bk, 0, stream, a);
+        if (a.cu_q && causal)
+            hipLaunchKernelGGL((flash_bwd_dkdv_kernel<D, true, true>), gk, bk, 0, stream, a);
+        else if (a.cu_q)
+            hipLaunchKernelGGL((flash_bwd_dkdv_kernel<D, false, true>), gk, bk, 0, stream, a);
+        else if (causal)
+            hipLaunchKernelGGL((flash_bwd_dkdv_kernel<D, true, false>), gk, bk, 0, stream, a);
         else
-            hipLaunchKernelGGL((flash_bwd_dkdv_kernel<D, false>), gk, bk, 0, stream, a);
+            hipLaunchKernelGGL((flash_bwd_dkdv_kernel<D, false, false>), gk, bk, 0, stream, a);
         if (a.gsplit > 1 && a.kv_elems > 0) {
             const int grid = (int)std::min<int64_t>(ceil_div64(2 * (a.kv_elems / 4), 256), 8192);
             hipLaunchKernelGGL(flash_bwd_kv_sum_kernel, dim3(grid), dim3(256), 0, stream,
@@ -912,6 +951,17 @@ hipError_t launch_flash_bwd(const FlashBwdLaunch& f, hipStream_t stream) {
     a.Hkv = f.Hkv;
     a.total_q = f.total_q;
     a.total_k = f.total_k;
+    a.q = chunks_of(f.q);
+    a.k = chunks_of(f.k);
+    a.v = chunks_of(f.v);
+    a.dout = chunks_of(f.dout);
+    a.o = chunks_of(f.cu_q ? packed_strides(f.H, f.D) : dense_strides(f.H, f.Sq, f.D));
+    a.dkv = chunks_of(f.cu_q ? packed_strides(f.Hkv, f.D) : dense_strides(f.Hkv, f.Sk, f.D));
+    a.div_h = fast_div(f.H);
+    a.div_hkv = fast_div(f.Hkv);
+    a.div_group = fast_div(a.group);
+    a.div_bh = fast_div((uint32_t)f.B * f.H);
+    a.div_bhkv = fast_div((uint32_t)f.B * f.Hkv);
     a.gsplit = 1;
     a.gper = a.group;
     if (!f.cu_q && f.gsplit > 1 && f.kv_part) {

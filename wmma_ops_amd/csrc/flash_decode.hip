@@ -20,6 +20,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "flash_sched.hpp"
 #include "kernels.hpp"
 #include "plan.hpp"
 
@@ -37,7 +38,10 @@ struct DecodeArgs {
     f16* O;
     float* lse;
     int rows;         // query rows per key/value head
+    int heads;        // key/value heads per batch entry (a unit is one of them)
     int Sk, dr;
+    ChunkStrides q, k, v;  // k.row == v.row; O is contiguous
+    FastDiv div_heads;
     float scale_log2;
     int chunk;        // steps per workgroup
     float* o_part;    // [chunks][units * rows][dr], nullptr: one chunk, final output
@@ -88,21 +92,23 @@ flash_decode_kernel(DecodeArgs p) {
     const int q = lane >> 4, r16 = lane & 15;
     const int unit = blockIdx.x;
     const int Sk = p.Sk, dr = p.dr;
+    const int qs = p.q.row_elems(), ks = p.k.row_elems();
     const float c = p.scale_log2;
-    const f16* Kb = p.K + (int64_t)unit * Sk * dr;
-    const f16* Vb = p.V + (int64_t)unit * Sk * dr;
+    const int b = div_by(p.div_heads, unit), hk = unit - b * p.heads;
+    const f16* Kb = p.K + p.k.at(b, hk, 0);
+    const f16* Vb = p.V + p.v.at(b, hk, 0);
 
     // Query row 16 mb + lane%16, d = 32 u + 8 q + 0..7 (zeros past the rows and past dr).
     f16x8 qf[MB][C::KU];
     {
-        const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.Q + (int64_t)unit * p.rows * dr);
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.Q + p.q.at(b, hk, 0));
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
             for (int u = 0; u < C::KU; ++u) {
                 const int row = 16 * mb + r16, d = 32 * u + 8 * q;
                 qf[mb][u] = as_f16x8(
-                    buf_load16(rs, row < p.rows && d < dr ? (uint32_t)((row * dr + d) * 2) : kOobOffset));
+                    buf_load16(rs, row < p.rows && d < dr ? (uint32_t)((row * qs + d) * 2) : kOobOffset));
             }
     }
 
@@ -112,7 +118,7 @@ flash_decode_kernel(DecodeArgs p) {
     // Loads of a step past the range go out of bounds (zeros, no memory request), so the loop
     // has no branch around them.
     auto tile = [&](const f16* base, int s) {
-        return make_rsrc(base + (int64_t)min(s, nsteps - 1) * FD_KEYS * dr);
+        return make_rsrc(base + (int64_t)min(s, nsteps - 1) * FD_KEYS * ks);
     };
     auto load_k = [&](int s, FdK<D>& S) {
         const int left = s < s1 ? Sk - s * FD_KEYS : 0;
@@ -122,7 +128,7 @@ flash_decode_kernel(DecodeArgs p) {
 #pragma unroll
             for (int u = 0; u < C::KU; ++u) {
                 const int key = 16 * kb + r16, d = 32 * u + 8 * q;
-                S.x[kb][u] = buf_load16_nt(rk, key < left && d < dr ? (uint32_t)((key * dr + d) * 2)
+                S.x[kb][u] = buf_load16_nt(rk, key < left && d < dr ? (uint32_t)((key * ks + d) * 2)
                                                                    : kOobOffset);
             }
     };
@@ -135,7 +141,7 @@ flash_decode_kernel(DecodeArgs p) {
             for (int e = 0; e < 8; ++e) {
                 const int key = 16 * (e >> 2) + 4 * q + (e & 3);
                 const int d = 128 * vh + C::VC * r16;
-                const uint32_t off = key < left && d < dr ? (uint32_t)((key * dr + d) * 2) : kOobOffset;
+                const uint32_t off = key < left && d < dr ? (uint32_t)((key * ks + d) * 2) : kOobOffset;
                 if constexpr (C::VC == 8) {
                     S.x[vh][e] = buf_load16_nt(rv, off);
                 } else {
@@ -370,6 +376,11 @@ hipError_t launch_flash_decode(const FlashLaunch& f, hipStream_t stream) {
     a.O = static_cast<f16*>(f.O);
     a.lse = f.lse;
     a.rows = f.Sq;
+    a.heads = f.H;
+    a.q = chunks_of(f.q);
+    a.k = chunks_of(f.k);
+    a.v = chunks_of(f.v);
+    a.div_heads = fast_div(f.H);
     a.Sk = f.Sk;
     a.dr = f.D;
     a.scale_log2 = f.scale * 1.4426950408889634f;

@@ -46,6 +46,7 @@ struct FlashArgs {
     f16* O;
     int Sq, Sk;
     int nqb;           // query blocks
+    int grid_y;
     float scale_log2;  // scale * log2(e)
     int group;         // query heads per key/value head (1: multi-head attention)
     int dr;            // head dim of the tensors: a multiple of 8, at most the kernel's D
@@ -56,9 +57,12 @@ struct FlashArgs {
     // cannot send a load or store outside the tensors.
     const int* cu_q;
     const int* cu_k;
+    bool ordered;      // items in the order of flash_sched.hpp
     int B;             // sequences
     int H, Hkv;
     int total_q, total_k;
+    ChunkStrides q, k, v, o;  // k.row == v.row
+    FastDiv div_h, div_group, div_bh;  // by H, the group and B * H
     // Optional per-row log-sum-exp of the scaled scores (natural log; +inf for a row with
     // no key): [B*H][Sq] dense, [H][total_q] variable length.
     float* lse;
@@ -312,7 +316,9 @@ __device__ __forceinline__ void fa_iter(const WMMA_LDS unsigned char* __restrict
     }
 }
 
-template <int D, bool CAUSAL>
+// VARLEN is a kernel of its own: a dense workgroup then starts without a branch, its arguments
+// loaded together.
+template <int D, bool CAUSAL, bool VARLEN>
 __global__ void __launch_bounds__(FaCfg<D>::WAVES * kWave)
 __attribute__((amdgpu_waves_per_eu(FaCfg<D>::WAVES / 4, FaCfg<D>::WAVES / 4)))
 flash_fwd_kernel(FlashArgs p) {
@@ -325,17 +331,17 @@ flash_fwd_kernel(FlashArgs p) {
     const int h = lane >> 5, c32 = lane & 31;
     // Which query block of which (batch, head): see flash_sched.hpp.
     int bh = blockIdx.x, qb_idx = blockIdx.y;
-    if (p.cu_q) {
-        int b, head;
-        const int64_t item = flash_split_id(flash_linear_id(), p.H, &head);
+    if (VARLEN && p.ordered) {
+        int seq, head;
+        const int64_t item =
+            flash_split_id(flash_linear_id(p.div_bh.d, p.grid_y), p.div_h, &head);
         if (!varlen_item<false, CAUSAL, C::BQ>(p.cu_q, p.cu_k, p.B, p.total_q, p.total_k, p.Sq, p.Sk,
-                                               item, &b, &qb_idx))
+                                               item, &seq, &qb_idx))
             return;
-        bh = b * p.H + head;
-    } else if (CAUSAL && !p.kv_chunk) {
-        qb_idx = p.nqb - 1 - (int)flash_split_id(flash_linear_id(), gridDim.x, &bh);
+        bh = seq * p.H + head;
     } else if (CAUSAL) {
-        qb_idx = p.nqb - 1 - qb_idx;
+        qb_idx = p.nqb - 1 -
+                 (int)flash_split_id(flash_linear_id(p.div_bh.d, p.grid_y), p.div_bh, &bh);
     }
     const int q0 = qb_idx * C::BQ;
     const int qw = q0 + wave * FA_WQ;
@@ -344,34 +350,31 @@ flash_fwd_kernel(FlashArgs p) {
     // Rows of this (batch, head): base offsets and row strides (elements).  Grouped-query
     // attention: query heads of one batch entry come in runs of `group` that share one
     // key/value head (heads are the inner index of both layouts).
-    int Sq, Sk, qs, ks;
-    int64_t q_base, k_base, lse_base;
-    if (p.cu_q) {
-        const int b = bh / p.H, hq = bh % p.H;
+    int Sq, Sk;
+    const int qs = p.q.row_elems(), ks = p.k.row_elems(), os = p.o.row_elems();
+    const int b = div_by(p.div_h, bh), hq = bh - b * p.H, hk = div_by(p.div_group, hq);
+    int q_row = 0, k_row = 0;  // first query and key row
+    int64_t lse_base;
+    if constexpr (VARLEN) {
         const int qa = min(max(p.cu_q[b], 0), p.total_q);
         const int qe = min(max(p.cu_q[b + 1], qa), p.total_q);
         const int ka = min(max(p.cu_k[b], 0), p.total_k);
         const int ke = min(max(p.cu_k[b + 1], ka), p.total_k);
         Sq = min(qe - qa, p.Sq);
         Sk = min(ke - ka, p.Sk);
-        qs = p.H * p.dr;
-        ks = p.Hkv * p.dr;
-        q_base = (int64_t)qa * qs + (int64_t)hq * p.dr;
-        k_base = (int64_t)ka * ks + (int64_t)(hq / p.group) * p.dr;
+        q_row = qa;
+        k_row = ka;
         lse_base = (int64_t)hq * p.total_q + qa;
     } else {
         Sq = p.Sq;
         Sk = p.Sk;
-        qs = p.dr;
-        ks = p.dr;
-        q_base = (int64_t)bh * Sq * p.dr;
-        k_base = (int64_t)(bh / p.group) * Sk * p.dr;
         lse_base = (int64_t)bh * Sq;
     }
-    const f16* Qb = p.Q + q_base;
-    const f16* Kb = p.K + k_base;
-    const f16* Vb = p.V + k_base;
-    f16* Ob = p.O + q_base;
+    if (VARLEN && q0 >= Sq) return;  // a query block past this sequence: no work
+    const f16* Qb = p.Q + p.q.at(b, hq, q_row);
+    const f16* Kb = p.K + p.k.at(b, hk, k_row);
+    const f16* Vb = p.V + p.v.at(b, hk, k_row);
+    f16* Ob = p.O + p.o.at(b, hq, q_row);
 
     // Q fragments (B operand of S^T): query qw + 32 qb + lane%32, d = 16 ds + 8 h + 0..7
     // (zeros for d >= dr, so padded d columns add nothing to the scores).
@@ -524,7 +527,7 @@ flash_fwd_kernel(FlashArgs p) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[e] = (f16)(O[db][qb][4 * g + e] * inv);
                     const int d = 32 * db + 8 * g + 4 * h;
-                    if (d < p.dr) *reinterpret_cast<f16x4*>(Ob + (int64_t)q * qs + d) = v;
+                    if (d < p.dr) *reinterpret_cast<f16x4*>(Ob + (int64_t)q * os + d) = v;
                 }
             }
         }
@@ -591,13 +594,19 @@ flash_combine_kernel(const float* o_part, const float* ml_part, int split, int64
 template <int D>
 void launch_d(FlashArgs a, int BH, bool causal, hipStream_t stream) {
     a.nqb = ceil_div(a.Sq, FaCfg<D>::BQ);
-    const int rows = a.cu_q ? varlen_grid_y(a.B, a.total_q, a.Sq, FaCfg<D>::BQ) : a.nqb;
+    a.ordered = a.cu_q && varlen_ordered(BH, a.nqb);
+    const int rows = a.ordered ? varlen_grid_y(a.B, a.total_q, a.Sq, FaCfg<D>::BQ) : a.nqb;
     dim3 grid(BH, rows, a.kv_chunk ? ceil_div(a.Sk, a.kv_chunk) : 1);
     const dim3 block(FaCfg<D>::WAVES * kWave);
-    if (causal)
-        hipLaunchKernelGGL((flash_fwd_kernel<D, true>), grid, block, 0, stream, a);
+    a.grid_y = rows;
+    if (a.cu_q && causal)
+        hipLaunchKernelGGL((flash_fwd_kernel<D, true, true>), grid, block, 0, stream, a);
+    else if (a.cu_q)
+        hipLaunchKernelGGL((flash_fwd_kernel<D, false, true>), grid, block, 0, stream, a);
+    else if (causal)
+        hipLaunchKernelGGL((flash_fwd_kernel<D, true, false>), grid, block, 0, stream, a);
     else
-        hipLaunchKernelGGL((flash_fwd_kernel<D, false>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((flash_fwd_kernel<D, false, false>), grid, block, 0, stream, a);
 }
 
 }  // namespace
@@ -619,6 +628,13 @@ hipError_t launch_flash_fwd(const FlashLaunch& f, hipStream_t stream) {
     a.Hkv = f.Hkv;
     a.total_q = f.total_q;
     a.total_k = f.total_k;
+    a.q = chunks_of(f.q);
+    a.k = chunks_of(f.k);
+    a.v = chunks_of(f.v);
+    a.o = chunks_of(f.cu_q ? packed_strides(f.H, f.D) : dense_strides(f.H, f.Sq, f.D));
+    a.div_h = fast_div(f.H);
+    a.div_group = fast_div(a.group);
+    a.div_bh = fast_div((uint32_t)f.B * f.H);
     a.lse = f.lse;
     a.scale_log2 = f.scale * 1.4426950408889634f;
     const int BH = f.B * f.H;

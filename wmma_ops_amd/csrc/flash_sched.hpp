@@ -11,29 +11,63 @@
 #pragma once
 
 #include "common.hpp"
+#include "kernels.hpp"
 
 namespace wmma_amd {
 
-// The linear workgroup id with the engines of every other row of 32 ids mirrored (the XCD
-// is kept): where the weight falls along the ids, engine 0 is first in one row and last in
-// the next.  The ids of an incomplete last row stay.
-__device__ __forceinline__ int64_t flash_linear_id() {
-    const int64_t id = (int64_t)blockIdx.x +
-                       (int64_t)gridDim.x * ((int64_t)blockIdx.y + (int64_t)gridDim.y * blockIdx.z);
-    const int64_t total = (int64_t)gridDim.x * gridDim.y * gridDim.z;
-    return (id & 32) && (id | 31) < total ? id ^ 24 : id;
+// The linear workgroup id of an x by y grid (by z) with the engines of every other row of 32
+// ids mirrored (the XCD is kept): where the weight falls along the ids, engine 0 is first in
+// one row and last in the next.  The ids of an incomplete last row stay, and so do all where
+// x, the columns of equal weight, are whole rows of 32.
+__device__ __forceinline__ int64_t flash_linear_id(int64_t x, int64_t y, int64_t z = 1) {
+    const int64_t id = blockIdx.x + x * (blockIdx.y + y * (z > 1 ? blockIdx.z : 0));
+    return (x & 31) && (id & 32) && (id | 31) < x * y * z ? id ^ 24 : id;
 }
 
-// id = row * n + col.
-__device__ __forceinline__ int64_t flash_split_id(int64_t id, int64_t n, int* col) {
-    if ((id >> 31) == 0 && (n >> 31) == 0) {
-        const uint32_t r = (uint32_t)id / (uint32_t)n;
-        *col = (int)((uint32_t)id - r * (uint32_t)n);
+// Division of 0 <= n < 2^31 by a divisor known at the launch: a high product, an add and a
+// shift, all scalar (Granlund and Montgomery's invariant division), where the generic one is
+// a float reciprocal and its corrections.  A workgroup's prologue divides several times, and
+// every workgroup waits for it: with generic divisions, 64-bit strides and the variable-length
+// search behind a branch of the dense kernels, 4 x 16 heads of 2048 tokens, D = 64, causal,
+// took 3% longer than with none of them; as here 1.5%.
+struct FastDiv {
+    uint32_t d, mul, shift;
+};
+inline FastDiv fast_div(uint32_t d) {
+    uint32_t l = 0;
+    while ((uint64_t(1) << l) < d) ++l;
+    return {d, (uint32_t)(((uint64_t(1) << 32) * ((uint64_t(1) << l) - d)) / d + 1), l};
+}
+__device__ __forceinline__ int div_by(const FastDiv& f, int n) {
+    return (int)((__umulhi(f.mul, (uint32_t)n) + (uint32_t)n) >> f.shift);
+}
+
+// id = row * f.d + col.
+__device__ __forceinline__ int64_t flash_split_id(int64_t id, const FastDiv& f, int* col) {
+    if ((id >> 31) == 0) {
+        const int r = div_by(f, (int)id);
+        *col = (int)((uint32_t)id - (uint32_t)r * f.d);
         return r;
     }
-    const int64_t r = id / n;
-    *col = (int)(id - r * n);
+    const int64_t r = id / f.d;
+    *col = (int)(id - r * f.d);
     return r;
+}
+
+// Strides of an attention tensor in 16-byte chunks (they are multiples of 8 elements): head
+// and row fit 32 bits, so an address is a few scalar multiplies.
+struct ChunkStrides {
+    uint64_t batch;
+    uint32_t head, row;
+    // Elements to row `r` of head h of batch entry b.
+    __device__ __forceinline__ int64_t at(int b, int h, int r) const {
+        return (int64_t)((batch * (uint32_t)b + (uint64_t)head * (uint32_t)h +
+                          (uint64_t)row * (uint32_t)r) * 8);
+    }
+    __device__ __forceinline__ int row_elems() const { return (int)(row * 8); }
+};
+inline ChunkStrides chunks_of(const AttnStrides& s) {
+    return {(uint64_t)s.batch / 8, (uint32_t)(s.head / 8), (uint32_t)(s.row / 8)};
 }
 
 // Inclusive prefix sum over the 64 lanes (DPP: no LDS, no memory).
@@ -131,6 +165,14 @@ __device__ __forceinline__ bool varlen_item(const int* cu_q, const int* cu_k, in
         rank -= n;
     }
     return false;
+}
+
+// Whether a varlen grid of `columns` (sequences x heads) by `blocks` per longest sequence takes
+// its items in that order.  A few short sequences finish before an uneven engine matters,
+// and the search would be a visible part of them (five sequences of at most 322 tokens, 40
+// heads: 21.1 us in plain order, 21.8 searched).
+inline bool varlen_ordered(int64_t columns, int64_t blocks) {
+    return blocks > 2 || columns * blocks > 1024;
 }
 
 // Workgroups that a varlen grid needs for its items: no more than max_len / block per

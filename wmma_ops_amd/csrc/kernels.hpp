@@ -117,6 +117,12 @@ W4A16Plan w4a16_plan(int M, int N, int K, int G, int num_cus, bool aligned);
 // at this K: M <= 4 and its staged activations within its LDS budget.
 bool w4a16_fused_decode_ok(int M, int K);
 
+// Elements from one batch entry, head and row of an attention tensor to the next; the d
+// elements of a row are contiguous.  Packed (variable-length) tensors use head and row.
+using AttnStrides = wmma_attn_strides;
+inline AttnStrides dense_strides(int64_t H, int64_t S, int64_t D) { return {H * S * D, S * D, D}; }
+inline AttnStrides packed_strides(int64_t H, int64_t D) { return {0, D, H * D}; }
+
 struct FlashLaunch {
     const void* Q;
     const void* K;
@@ -139,6 +145,7 @@ struct FlashLaunch {
     // second kernel.
     int kv_split = 1;
     void* workspace = nullptr;
+    AttnStrides q, k, v;  // k.row == v.row; O is contiguous
 };
 hipError_t launch_flash_fwd(const FlashLaunch& f, hipStream_t stream);
 // Key-range split the forward uses for a dense shape on num_cus CUs (1: none): only when
@@ -184,6 +191,8 @@ struct FlashBwdLaunch {
     // (flash_bwd_split_bytes, 16-byte aligned), added by a second kernel.
     int gsplit = 1;
     float* kv_part = nullptr;
+    AttnStrides q, k, v, dout;  // q.row == dout.row, k.row == v.row; O and the gradients are
+                                // contiguous
 };
 int64_t flash_bwd_workspace_rows(const FlashBwdLaunch& f);
 // Grouped-query split of the dK/dV kernel for a dense shape on num_cus CUs (1: none): when

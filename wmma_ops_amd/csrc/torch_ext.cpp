@@ -20,6 +20,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <initializer_list>
 #include <string>
 
 #include "../../include/wmma_ops_amd.h"
@@ -280,6 +281,59 @@ torch::Tensor unpad_head(const torch::Tensor& t, int64_t D) {
     return t.size(-1) == D ? t : t.narrow(-1, 0, D).contiguous();
 }
 
+// An attention tensor as the kernels read it: `t` and its strides.  Dense tensors are
+// [B, heads, S, D], packed ones [rows, heads, D].
+struct AttnOperand {
+    torch::Tensor t;
+    wmma_attn_strides s;
+};
+
+wmma_attn_strides attn_strides(const torch::Tensor& t) {
+    if (t.dim() == 4) return {t.stride(0), t.stride(1), t.stride(2)};
+    return {0, t.stride(1), t.stride(0)};
+}
+
+// Whether the kernels can read t where it is: rows of whole 16-byte vectors at any batch, head
+// and row stride that 32-bit offsets hold over `rows` rows (one sequence of one head).
+bool attn_in_place(const torch::Tensor& t, int64_t rows) {
+    if (t.stride(-1) != 1 || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0) return false;
+    const wmma_attn_strides s = attn_strides(t);
+    return s.batch % 8 == 0 && s.head % 8 == 0 && s.row % 8 == 0 &&
+           s.head / 8 <= (int64_t)UINT32_MAX &&
+           std::max<int64_t>(rows, 64) * s.row * 2 <= INT32_MAX;
+}
+
+// One side of an attention call, Q (and dO) or K and V: contiguous tensors as they are, views
+// too where the kernels can read all of them in place with one row stride -- the heads of a
+// projection's [B, S, H, D] output need no copy -- and otherwise contiguous copies.
+void attn_operands(std::initializer_list<AttnOperand*> side, int64_t Dp, int64_t rows) {
+    bool as_is = true;
+    for (const AttnOperand* x : side)
+        as_is = as_is && x->t.size(-1) == Dp && x->t.numel() > 0 && attn_in_place(x->t, rows) &&
+                attn_strides(x->t).row == attn_strides((*side.begin())->t).row;
+    for (AttnOperand* x : side) {
+        if (as_is) {
+            x->s = attn_strides(x->t);
+            continue;
+        }
+        x->t = pad_head(x->t, Dp);
+        // not the tensor's own strides: dimensions of one element may have any
+        const bool dense = x->t.dim() == 4;
+        const int64_t h = x->t.size(1), n = dense ? x->t.size(2) : 1;
+        x->s = dense ? wmma_attn_strides{h * n * Dp, n * Dp, Dp} : wmma_attn_strides{0, Dp, h * Dp};
+    }
+}
+
+// Without a causal mask the query heads of a group run as one sequence of rows where they lie
+// one after the other (include/wmma_ops_amd.h); head views do not.  Q is copied for that
+// where 256-row blocks of single heads would be over 10% more blocks.
+bool pack_by_copy(const torch::Tensor& Q, const wmma_attn_strides& q, int64_t Hkv, bool causal) {
+    const int64_t H = Q.size(1), Sq = Q.size(2);
+    if (causal || H == Hkv || Sq <= 1 || q.head == Sq * q.row) return false;
+    const int64_t packed = (Sq * (H / Hkv) + 255) / 256 * Hkv, single = (Sq + 255) / 256 * H;
+    return 10 * single > 11 * packed;
+}
+
 float flash_scale(double scale, int64_t D) {
     return scale > 0.0 ? (float)scale : (float)(1.0 / std::sqrt((double)D));
 }
@@ -289,26 +343,30 @@ torch::Tensor flash_dense_fwd(torch::Tensor Q, torch::Tensor K, torch::Tensor V,
                               double scale, torch::Tensor* lse_out) {
     check_flash_dense(Q, K, V);
     const int64_t D = Q.size(3), Dp = padded_head_dim(D);
+    const int64_t B = Q.size(0), H = Q.size(1), Hkv = K.size(1), Sq = Q.size(2), Sk = K.size(2);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(Q.device());
-    Q = pad_head(Q, Dp);
-    K = pad_head(K, Dp);
-    V = pad_head(V, Dp);
-    auto O = torch::empty_like(Q);
+    AttnOperand q{Q, {}}, k{K, {}}, v{V, {}};
+    attn_operands({&q}, Dp, Sq);
+    if (pack_by_copy(q.t, q.s, Hkv, causal)) {
+        q.t = q.t.contiguous();
+        q.s = {H * Sq * Dp, Sq * Dp, Dp};
+    }
+    attn_operands({&k, &v}, Dp, Sk);
+    auto O = torch::empty({B, H, Sq, Dp}, Q.options());
     float* lse = nullptr;
     if (lse_out) {
-        *lse_out = torch::empty({Q.size(0), Q.size(1), Q.size(2)}, Q.options().dtype(torch::kFloat32));
+        *lse_out = torch::empty({B, H, Sq}, Q.options().dtype(torch::kFloat32));
         lse = lse_out->data_ptr<float>();
     }
     // decoding shapes split the key range; the partial sums come from the caching allocator
-    const size_t ws_bytes = wmma_flash_attn_fwd_workspace_size(
-        (int)Q.size(0), (int)Q.size(1), (int)K.size(1), (int)Q.size(2), (int)K.size(2), (int)Dp,
-        causal ? 1 : 0);
+    const size_t ws_bytes = wmma_flash_attn_fwd_strided_workspace_size(
+        q.s, (int)B, (int)H, (int)Hkv, (int)Sq, (int)Sk, (int)Dp, causal ? 1 : 0);
     torch::Tensor ws = workspace_for(ws_bytes, Q);
-    int rc = wmma_flash_attn_fwd_ws(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), lse,
-                                    (int)Q.size(0), (int)Q.size(1), (int)K.size(1),
-                                    (int)Q.size(2), (int)K.size(2), (int)Dp, flash_scale(scale, D),
-                                    causal ? 1 : 0, ws.defined() ? ws.data_ptr() : nullptr,
-                                    ws_bytes, current_stream(Q));
+    int rc = wmma_flash_attn_fwd_strided(q.t.data_ptr(), q.s, k.t.data_ptr(), k.s, v.t.data_ptr(),
+                                         v.s, O.data_ptr(), lse, (int)B, (int)H, (int)Hkv, (int)Sq,
+                                         (int)Sk, (int)Dp, flash_scale(scale, D), causal ? 1 : 0,
+                                         ws.defined() ? ws.data_ptr() : nullptr, ws_bytes,
+                                         current_stream(Q));
     check_status(rc, "wmma_flash_attn_fwd_ws");
     return unpad_head(O, D);
 }
@@ -344,24 +402,23 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> flash_attention_backward
     const int64_t Dp = padded_head_dim(D);
     TORCH_CHECK(Sq == 0 || K.size(2) > 0, "K must have keys when Q has queries");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(Q.device());
-    Q = pad_head(Q, Dp);
-    K = pad_head(K, Dp);
-    V = pad_head(V, Dp);
+    AttnOperand q{Q, {}}, k{K, {}}, v{V, {}}, g{dO, {}};
+    attn_operands({&q, &g}, Dp, Sq);
+    attn_operands({&k, &v}, Dp, K.size(2));
     O = pad_head(O, Dp);
-    dO = pad_head(dO, Dp);
     lse = lse.contiguous();
-    auto dQ = torch::empty_like(Q);
-    auto dK = torch::empty_like(K);
-    auto dV = torch::empty_like(V);
+    auto dQ = torch::empty({B, H, Sq, Dp}, Q.options());
+    auto dK = torch::empty({B, K.size(1), K.size(2), Dp}, K.options());
+    auto dV = torch::empty_like(dK);
     // row statistics, plus the grouped-query split's partial dK/dV where it applies
     const size_t ws_bytes = wmma_flash_attn_bwd_split_workspace_size(
         (int)B, (int)H, (int)K.size(1), (int)Sq, (int)K.size(2), (int)Dp, causal ? 1 : 0);
     auto ws = torch::empty({(int64_t)((ws_bytes + 3) / 4)}, Q.options().dtype(torch::kFloat32));
-    int rc = wmma_flash_attn_bwd(dO.data_ptr(), Q.data_ptr(), K.data_ptr(), V.data_ptr(),
-                                 O.data_ptr(), lse.data_ptr<float>(), dQ.data_ptr(), dK.data_ptr(),
-                                 dV.data_ptr(), ws.data_ptr(), ws_bytes, (int)B, (int)H,
-                                 (int)K.size(1), (int)Sq, (int)K.size(2), (int)Dp,
-                                 flash_scale(scale, D), causal ? 1 : 0, current_stream(Q));
+    int rc = wmma_flash_attn_bwd_strided(
+        g.t.data_ptr(), g.s, q.t.data_ptr(), q.s, k.t.data_ptr(), k.s, v.t.data_ptr(), v.s,
+        O.data_ptr(), lse.data_ptr<float>(), dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(),
+        ws.data_ptr(), ws_bytes, (int)B, (int)H, (int)K.size(1), (int)Sq, (int)K.size(2), (int)Dp,
+        flash_scale(scale, D), causal ? 1 : 0, current_stream(Q));
     check_status(rc, "wmma_flash_attn_bwd");
     return {unpad_head(dQ, D), unpad_head(dK, D), unpad_head(dV, D)};
 }
@@ -372,20 +429,20 @@ torch::Tensor flash_varlen_fwd(torch::Tensor q, torch::Tensor k, torch::Tensor v
     check_flash_varlen(q, k, v, cu_q, cu_k);
     const int64_t D = q.size(2), Dp = padded_head_dim(D);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
-    q = pad_head(q, Dp);
-    k = pad_head(k, Dp);
-    v = pad_head(v, Dp);
+    AttnOperand qo{q, {}}, ko{k, {}}, vo{v, {}};
+    attn_operands({&qo}, Dp, max_q);
+    attn_operands({&ko, &vo}, Dp, max_k);
     cu_q = cu_q.contiguous();
     cu_k = cu_k.contiguous();
-    auto O = torch::empty_like(q);
+    auto O = torch::empty({q.size(0), q.size(1), Dp}, q.options());
     float* lse = nullptr;
     if (lse_out) {
         *lse_out = torch::empty({q.size(1), q.size(0)}, q.options().dtype(torch::kFloat32));
         lse = lse_out->data_ptr<float>();
     }
-    int rc = wmma_flash_attn_varlen_fwd_lse(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), O.data_ptr(), lse, cu_q.data_ptr<int32_t>(),
-        cu_k.data_ptr<int32_t>(), (int)(cu_q.size(0) - 1), (int)q.size(1), (int)k.size(1),
+    int rc = wmma_flash_attn_varlen_fwd_strided(
+        qo.t.data_ptr(), qo.s, ko.t.data_ptr(), ko.s, vo.t.data_ptr(), vo.s, O.data_ptr(), lse,
+        cu_q.data_ptr<int32_t>(), cu_k.data_ptr<int32_t>(), (int)(cu_q.size(0) - 1), (int)q.size(1), (int)k.size(1),
         (int)q.size(0), (int)k.size(0), (int)max_q, (int)max_k, (int)Dp, flash_scale(scale, D),
         causal ? 1 : 0, current_stream(q));
     check_status(rc, "wmma_flash_attn_varlen_fwd_lse");
@@ -419,28 +476,27 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> flash_attention_varlen_b
     check_flash_grad_inputs(q, dO, O, lse, {q.size(1), q.size(0)});
     const int64_t H = q.size(1), D = q.size(2), Dp = padded_head_dim(D);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
-    q = pad_head(q, Dp);
-    k = pad_head(k, Dp);
-    v = pad_head(v, Dp);
+    AttnOperand qo{q, {}}, ko{k, {}}, vo{v, {}}, go{dO, {}};
+    attn_operands({&qo, &go}, Dp, max_q);
+    attn_operands({&ko, &vo}, Dp, max_k);
     O = pad_head(O, Dp);
-    dO = pad_head(dO, Dp);
     lse = lse.contiguous();
     cu_q = cu_q.contiguous();
     cu_k = cu_k.contiguous();
-    auto dq = torch::empty_like(q);
-    auto dk = torch::empty_like(k);
-    auto dv = torch::empty_like(v);
+    auto dq = torch::empty({q.size(0), q.size(1), Dp}, q.options());
+    auto dk = torch::empty({k.size(0), k.size(1), Dp}, k.options());
+    auto dv = torch::empty_like(dk);
     // rows outside every sequence are not written by the kernels: start from zeros
-    if (q.numel()) dq.zero_();
-    if (k.numel()) {
+    if (dq.numel()) dq.zero_();
+    if (dk.numel()) {
         dk.zero_();
         dv.zero_();
     }
     const size_t ws_bytes = wmma_flash_attn_bwd_workspace_size(1, (int)H, (int)q.size(0));
     auto ws = torch::empty({(int64_t)(ws_bytes / 4)}, q.options().dtype(torch::kFloat32));
-    int rc = wmma_flash_attn_varlen_bwd(
-        dO.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), O.data_ptr(),
-        lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+    int rc = wmma_flash_attn_varlen_bwd_strided(
+        go.t.data_ptr(), go.s, qo.t.data_ptr(), qo.s, ko.t.data_ptr(), ko.s, vo.t.data_ptr(), vo.s,
+        O.data_ptr(), lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
         cu_q.data_ptr<int32_t>(), cu_k.data_ptr<int32_t>(), ws.data_ptr(), ws_bytes,
         (int)(cu_q.size(0) - 1), (int)H, (int)k.size(1), (int)q.size(0), (int)k.size(0),
         (int)max_q, (int)max_k, (int)Dp, flash_scale(scale, D), causal ? 1 : 0, current_stream(q));
