@@ -332,28 +332,34 @@ void launch_decode_d(const DecodeArgs& a, dim3 grid, hipStream_t stream) {
 
 bool flash_decode_takes(int Sq, bool causal) { return !causal && Sq >= 1 && Sq <= FD_MAX_ROWS; }
 
-// Chunks of the key range.  The time of a split, read off a sweep of 1-64 chunks at 17 shapes
-// (2-512 units, 318-32768 keys, D = 64-256): the reads at 28 KB/us per busy CU and at most
-// 6.2 TB/s; past one wave of workgroups the busiest CU sets the pace (80 units, 5408 keys: 3
-// chunks 32 us, 4 chunks -- 320 workgroups -- 42 us); two chunks or more add the merge and
-// their partial sums.  Each wave of a chunk gets a step.
+// Chunks of the key range: 256 keys or more each, down to 96 while fewer than 64 workgroups
+// run.  The time of a split, read off a sweep of 1-64 chunks at 17 shapes (2-512 units,
+// 318-32768 keys, D = 64-256): the reads at 24.5 KB/us per busy CU and at most 6.2 TB/s; past
+// one wave of workgroups the busiest CU sets the pace (80 units, 5408 keys: 3 chunks 32 us, 4
+// chunks -- 320 workgroups -- 42 us); two chunks or more add the merge and their partial
+// sums.  The split that fills the CUs once stays unless another is 1% better.
 int flash_decode_split(int64_t units, int Sq, int Sk, int D, int num_cus) {
     const int steps = ceil_div(Sk, FD_KEYS);
     const double mb = (double)units * Sk * D * 4e-6;
-    int best = 1;
-    double best_t = 1e300;
-    for (int z = 1; z <= 64; z = z < 8 ? z + 1 : z + z / 8) {
-        if (z > 1 && ceil_div(steps, z) < FD_WAVES) break;
-        const int zz = ceil_div(steps, ceil_div(steps, z));
-        const int64_t wgs = units * zz;
-        const double rate = std::min(6.2, 0.028 * (double)std::min<int64_t>(wgs, num_cus));
+    const int few = (int)std::min<int64_t>(std::max<int64_t>(64 / units, 1), Sk / 96);
+    const int most = std::min(64, std::max({Sk / 256, few, 1}));
+    const int fill = (int)std::min<int64_t>(std::max<int64_t>(num_cus / units, 1), most);
+    auto time = [&](int z) {
+        const int64_t wgs = units * z;
+        const double rate = std::min(6.2, 0.0245 * (double)std::min<int64_t>(wgs, num_cus));
         const double uneven =
             wgs > num_cus ? (double)(ceil_div64(wgs, num_cus) * num_cus) / (double)wgs : 1.0;
-        double t = 2.5 + uneven * mb / rate;
-        if (zz > 1) t += 5.0 + 0.15 * zz + (double)zz * units * Sq * D * 8e-6 / 5.0;
+        const double t = 2.5 + uneven * mb / rate;
+        return z > 1 ? t + 5.0 + 0.15 * z + (double)z * units * Sq * D * 8e-6 / 5.0 : t;
+    };
+    auto chunks = [&](int z) { return ceil_div(steps, ceil_div(steps, z)); };
+    int best = chunks(fill);
+    double best_t = time(best);
+    for (int z = 1; z <= most; z = z < 8 ? z + 1 : z + z / 8) {
+        const double t = time(chunks(z));
         if (t < best_t * 0.99) {
             best_t = t;
-            best = zz;
+            best = chunks(z);
         }
     }
     return best;
