@@ -24,6 +24,7 @@ BATCHES = {
     "empty": [0, 300, 0, 0, 65, 0],
     "wave": [17] * 63 + [520],
     "past_wave": [(37 * i) % 90 for i in range(64)] + [400, 0, 3, 261],
+    "long": [700, 1500, 90, 0, 1000, 1281],
     "two_waves": [(11 * i) % 23 for i in range(130)] + [300],
 }
 

@@ -168,11 +168,12 @@ __device__ __forceinline__ bool varlen_item(const int* cu_q, const int* cu_k, in
 }
 
 // Whether a varlen grid of `columns` (sequences x heads) by `blocks` per longest sequence takes
-// its items in that order.  A few short sequences finish before an uneven engine matters,
-// and the search would be a visible part of them (five sequences of at most 322 tokens, 40
-// heads: 21.1 us in plain order, 21.8 searched).
+// its items in that order.  Where every workgroup has a CU at once, or a few short sequences
+// finish before an uneven engine matters, the search would be a visible part of them (eight
+// sequences of 33 to 966 tokens, 8 heads: 32.6 us in plain order, 33.2 searched; five of at
+// most 322, 40 heads: 21.1 and 21.8).
 inline bool varlen_ordered(int64_t columns, int64_t blocks) {
-    return blocks > 2 || columns * blocks > 1024;
+    return columns * blocks > (blocks > 2 ? 256 : 1024);
 }
 
 // Workgroups that a varlen grid needs for its items: no more than max_len / block per
