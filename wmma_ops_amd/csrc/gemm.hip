@@ -1058,12 +1058,20 @@ struct MfmaStages {
     int bk, ns;
 };
 constexpr MfmaStages kMfmaStages[WMMA_TILE_COUNT] = {
-    {64, 4}, {64, 4}, {64, 3}, {64, 4}, {64, 3}, {32, 4}};
+    {64, 4}, {64, 4}, {64, 3}, {64, 4}, {32, 4}, {32, 4}};
+// The 256 x 128 tile (8 waves of 64 x 64) takes 32-deep stages, except with both operands
+// K-major, whose 64-byte rows would halve the DMA's runs: 2048 x 4096 x 4096, NN / NT / TN,
+// 32 deep, 4 stages 72.3 / 75.2 / 71.1 us, 64 deep, 3 stages 73.4 / 70.7 / 75.6; four waves
+// of 128 x 64, 64 deep, as it was 75.3 / 73.4 / 78.0 (on half the CUs, 1024 x 4096 x 4096,
+// where power is no limit: 52.3 / 53.3 / 53.1 now, 58.8 / 59.8 / 62.9 then).
+constexpr MfmaStages mfma_stages(int cfg, bool tb) {
+    return cfg == WMMA_TILE_256x128 && tb ? MfmaStages{64, 3} : kMfmaStages[cfg];
+}
 
 template <int CFG, bool TA, bool TB>
 void launch_mfma(const GemmArgs& a, hipStream_t stream) {
     constexpr TileShape t = kTiles[CFG];
-    constexpr MfmaStages st = kMfmaStages[CFG];
+    constexpr MfmaStages st = mfma_stages(CFG, TB);
     dim3 grid(a.tiles_m * a.tiles_n, a.split);
     hipLaunchKernelGGL((gemm_mfma_kernel<t.bm, t.bn, st.bk, t.wm, t.wn, st.ns, TA, TB>), grid,
                        dim3(t.wm * t.wn * kWave), 0, stream, a);

@@ -5,11 +5,10 @@
 // (compute_config, wmma_xor_swizzle.hpp:293-332: target tiles = 4 x CUs, split capped at
 // 32 and at K/256, k_per_split = ceil(K/split)).  Here the choice is made against a
 // 256-CU device, in four tiers: exact shapes from the autotuned table; M <= 16 with
-// K > 1024 on the streaming kernel with its split rule; every other M <= 768 by a launch
-// model fitted to measured times of every plan (model_plan); larger M by whole waves of
-// workgroups, the tile that reuses the most bytes per LDS byte, a K split only when too
-// few output tiles exist to occupy the CUs, and bulk + edge plans.  The result never
-// depends on the plan beyond fp32 summation order.
+// K > 1024 on the streaming kernel with its split rule; every other M <= 256 and larger M
+// by two launch models fitted to measured times of every plan (model_plan, tiled_plan),
+// the latter with bulk + edge plans.  The result never depends on the plan beyond fp32
+// summation order.
 #include "plan.hpp"
 
 #include <algorithm>
@@ -39,19 +38,22 @@ static void fit_split(int M, int N, int K, size_t max_ws, wmma_gemm_plan* p) {
 double plan_time_us(const wmma_gemm_plan& p, int M, int N, int K, int num_cus) {
     if (M <= 0 || N <= 0 || K <= 0) return 0.0;
     if (num_cus <= 0) num_cus = 256;
-    const double hbm = (2.0 * M * K + 2.0 * K * N + 4.0 * M * N) / kHbmBytesPerUs;
     const int split = std::max(p.split_k, 1);
-    double t = hbm;
+    const double hbm_mb = (2.0 * M * K + 2.0 * K * N + 4.0 * M * N) / 1e6;
+    double t = hbm_mb / kHbmMBPerUs;
     if (p.kernel == WMMA_KERNEL_TILED) {
         const TileShape& ts = kTiles[p.tile_cfg];
-        const double area = (double)ts.bm * ts.bn / 65536.0;
+        const TileTime& tt = kTileTime[p.tile_cfg];
         const int64_t wgs = (int64_t)ceil_div(M, ts.bm) * ceil_div(N, ts.bn) * split;
-        const int kps = split > 1 ? p.k_per_split : K;
-        const double wave = area * (kEpiUs256 + kWaveUsPerK256 * kps / kWaveEff[p.tile_cfg]);
-        t = std::max((double)ceil_div64(wgs, num_cus) * wave, hbm);
+        const int64_t rounds = ceil_div64(wgs, num_cus);
+        const double stages = (split > 1 ? p.k_per_split : K) / (double)kBlockK;
+        const double last = (double)(wgs - (rounds - 1) * num_cus) / num_cus;
+        const double last_stage = tt.stage_lat_us + (tt.stage_us - tt.stage_lat_us) * last;
+        t = std::max(t, kLaunchUs + (rounds - 1) * (tt.fixed_us + stages * tt.stage_us) +
+                            tt.fixed_us + stages * last_stage);
     }
-    if (split > 1) t += (split + 1) * 4.0 * M * N / kHbmBytesPerUs + kReduceUs;
-    return t + kLaunchUs;
+    if (split > 1) t += kReduceUs + kReduceUsPerMB * (split + 1) * 4.0 * M * N / 1e6;
+    return t;
 }
 
 double model_time_us(const wmma_gemm_plan& p, int M, int N, int K, int num_cus) {
@@ -180,6 +182,32 @@ int make_custom_plan(int M, int N, int K, int kernel, int tile_cfg, int split,
     return WMMA_OK;
 }
 
+// The tiled plan with the shortest plan_time_us: every tile with K splits up to 16 (from
+// K = 2048, at least 256 of K per part, at most two rounds of the CUs).
+static wmma_gemm_plan tiled_plan(int M, int N, int K, int num_cus, size_t max_ws) {
+    wmma_gemm_plan best{};
+    double best_t = 1e300;
+    // larger tiles first: they win a tie
+    for (int cfg : {WMMA_TILE_256x256, WMMA_TILE_256x128, WMMA_TILE_128x128, WMMA_TILE_256x64,
+                    WMMA_TILE_128x64, WMMA_TILE_64x64}) {
+        const TileShape& ts = kTiles[cfg];
+        const int64_t tiles = (int64_t)ceil_div(M, ts.bm) * ceil_div(N, ts.bn);
+        for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
+            if (sp > 1 && (K < 2048 || K / sp < 256 || tiles * sp > 2 * (int64_t)num_cus)) break;
+            wmma_gemm_plan c{};
+            if (make_custom_plan(M, N, K, WMMA_KERNEL_TILED, cfg, sp, &c) != WMMA_OK ||
+                c.split_k != sp || c.workspace_bytes > max_ws)
+                continue;
+            const double t = plan_time_us(c, M, N, K, num_cus);
+            if (t < best_t * 0.999) {
+                best_t = t;
+                best = c;
+            }
+        }
+    }
+    return best;
+}
+
 // Bulk + edge: when the 256x256 tiles of the shape fill W >= 1 whole waves plus part of
 // another, the whole tile rows (or columns) that fit in W waves run as one launch and the
 // rest as a GEMM of its own, planned on its own (it is small, so it may take a smaller
@@ -203,8 +231,11 @@ static void two_part(int M, int N, int K, int num_cus, size_t max_ws, wmma_gemm_
             make_plan_within(em, en, K, WMMA_TILE_AUTO, num_cus, max_ws, &edge) != WMMA_OK ||
             edge.edge_dim != WMMA_EDGE_NONE)
             continue;
-        const double t = plan_time_us(bulk, bm, bn, K, num_cus) + plan_time_us(edge, em, en, K, num_cus);
-        if (t < best_t) {
+        const double t = plan_time_us(bulk, bm, bn, K, num_cus) +
+                         plan_time_us(edge, em, en, K, num_cus) + kSecondLaunchUs;
+        // columns only where they are 2% better than rows: each row of their edge is a short
+        // run of B and C (2560 x 14336 x 4096: 280 us by rows, 286 by columns, modelled level)
+        if (t < (p->edge_dim == WMMA_EDGE_ROWS ? 0.98 : 1.0) * best_t) {
             best_t = t;
             bulk.workspace_bytes = edge.workspace_bytes;
             bulk.edge_dim = dim;
@@ -286,40 +317,13 @@ int make_plan_within(int M, int N, int K, int tile_cfg, int num_cus, size_t max_
         return WMMA_OK;
     }
 
-    // Tiled MFMA kernel: the tile with the shortest estimated time (plan_time_us: waves of
-    // workgroups, one per CU, times the tile's wave time), the larger tile on a tie.
-    const int order[] = {WMMA_TILE_256x256, WMMA_TILE_256x128, WMMA_TILE_128x128,
-                         WMMA_TILE_256x64, WMMA_TILE_128x64, WMMA_TILE_64x64};
-    int best = WMMA_TILE_64x64;
-    double best_cost = 1e300;
-    for (int cfg : order) {
-        wmma_gemm_plan c{};
-        if (make_custom_plan(std::max(M, 1), std::max(N, 1), std::max(K, 1), WMMA_KERNEL_TILED, cfg,
-                             1, &c) != WMMA_OK)
-            continue;
-        const double cost = plan_time_us(c, std::max(M, 1), std::max(N, 1), std::max(K, 1), num_cus);
-        if (cost < best_cost * 0.999) {
-            best_cost = cost;
-            best = cfg;
-        }
+    // No output or an empty sum: any tile, the kernels write what there is to write.
+    if (M <= 0 || N <= 0 || K <= 0) {
+        make_custom_plan(M, N, K, WMMA_KERNEL_TILED, WMMA_TILE_64x64, 1, out);
+        return WMMA_OK;
     }
-    const TileShape& t = kTiles[best];
-    p.kernel = WMMA_KERNEL_TILED;
-    p.tile_cfg = best;
-    p.tile_m = t.bm;
-    p.tile_n = t.bn;
-    int tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn);
-    int split = 1;
-    // Split K only when the chip is under-filled and the GEMM is big enough (>= 2^30
-    // multiply-adds) for the extra reduction launch to pay for itself.
-    if (tiles > 0 && tiles * 2 <= num_cus && K >= 512 &&
-        (int64_t)M * N * K >= (int64_t(1) << 30)) {
-        split = std::min({num_cus / tiles, K / 256, kMaxSplitK});
-        split = std::max(split, 1);
-    }
-    finish_split(M, N, K, tiles, split, &p);
-    fit_split(M, N, K, max_ws, &p);
-    if (tile_cfg == WMMA_TILE_AUTO && p.split_k == 1) two_part(M, N, K, num_cus, max_ws, &p);
+    p = tiled_plan(M, N, K, num_cus, max_ws);
+    if (p.split_k == 1) two_part(M, N, K, num_cus, max_ws, &p);
     *out = p;
     return WMMA_OK;
 }

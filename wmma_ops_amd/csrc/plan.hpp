@@ -21,14 +21,14 @@ constexpr TileShape kTiles[WMMA_TILE_COUNT] = {
     {64, 64, 2, 2},    // 0: wave tile 32x32
     {128, 64, 4, 2},   // 1: wave tile 32x32 (8 waves; 5-9% faster than 4 waves of 64x32)
     {256, 64, 4, 1},   // 2: wave tile 64x64
-    {128, 128, 2, 2},  // 3: wave tile 64x64
-    {256, 128, 2, 2},  // 4: wave tile 128x64
+    {128, 128, 2, 4},  // 3: wave tile 64x32 (8 waves: 0-5% faster than 4 of 64x64)
+    {256, 128, 4, 2},  // 4: wave tile 64x64 (8 waves: 3-12% faster than 4 of 128x64)
     {256, 256, 2, 4},  // 5: wave tile 128x64 (8 waves, two per SIMD)
 };
 
 constexpr int kBlockK = 64;        // K depth of one LDS stage (fp16: 128-byte rows)
 constexpr int kSkinnyAutoMaxM = 16; // M at or below this (K > 1024): the streaming kernel's own rule
-constexpr int kModelMaxM = 768;     // M at or below this: the measured launch model picks the plan
+constexpr int kModelMaxM = 256;     // M at or below this: model_time_us picks the plan
 constexpr int kSkinnyMaxMWide = 64; // the streaming kernel's limit (four 16-row blocks)
 constexpr int kSkinnyBlockN = 128; // columns per skinny workgroup
 constexpr int kMaxSplitK = 32;     // cap from the reference's split-K config (wmma_xor_swizzle.hpp:318)
@@ -59,27 +59,36 @@ constexpr double kModelHbmMBPerUs = 8.0;   // operand bytes per microsecond at m
 // Modelled duration (microseconds) of a one-launch plan for M <= kModelMaxM.
 double model_time_us(const wmma_gemm_plan& p, int M, int N, int K, int num_cus);
 
-// Time model of the tiled kernel on full waves of workgroups (one workgroup per CU),
-// fitted on MI355X to full-wave launches of every tile (4096^3, 8192 x 8192 x 4096,
-// 4096 x 4096 x 1024, 4096 x 14336 x 4096, 8192 x 4096 x 8192; random fp16 operands):
-// one wave of 256x256 tiles takes kEpiUs256 + kWaveUsPerK256 * K microseconds (the
-// first term is the fp32 tile written out), and a wave of another tile the same scaled
-// by its area / 65536, with the K term divided by the tile's measured efficiency.
-constexpr double kWaveEff[WMMA_TILE_COUNT] = {0.45, 0.57, 0.55, 0.72, 0.81, 1.0};
-constexpr double kEpiUs256 = 13.2;
-constexpr double kWaveUsPerK256 = 0.0279;
-constexpr double kHbmBytesPerUs = 5.0e6;  // sustained HBM rate of the streaming kernels
-constexpr double kLaunchUs = 2.0;         // a launch behind another on the same stream
-constexpr double kReduceUs = 3.0;         // the split-K reduction's launch
+// Launch model for M > kModelMaxM, fitted on MI355X (256 CUs) to 320 shapes (M = 33-4096,
+// N, K = 256-14336 over their logarithms, up to 4096^3) x 6 tiles x splits 1-16, each plan
+// timed in a settled clock: 6% RMS error over the plans within twice the fastest.  A
+// workgroup takes a fixed time (prologue, epilogue) and a time per 64-deep stage, which
+// grows from its latency to what the chip's power and memory sustain with all CUs busy; the
+// launch takes that per round of workgroups, at least its operands' bytes at 4.4 TB/s, plus,
+// with a K split, the reduction launch and the partial sums' bytes.  Its choices take 2.0%
+// more time than the fastest plan of each shape; the rules before (the model above to
+// M = 768, full waves of tiles past it, a split only under half a wave) 5.3%, and up to 2.5
+// times at long K and few tiles (1665 x 384 x 12544: 50 us unsplit, 34 us split).
+struct TileTime {
+    double fixed_us, stage_us, stage_lat_us;
+};
+constexpr TileTime kTileTime[WMMA_TILE_COUNT] = {{2.51, 0.280, 0.220}, {2.88, 0.412, 0.258},
+                                                 {5.26, 0.766, 0.564}, {4.30, 0.635, 0.300},
+                                                 {5.03, 1.022, 0.626}, {8.14, 1.612, 1.001}};
+constexpr double kLaunchUs = 1.77;
+constexpr double kHbmMBPerUs = 4.4;
+constexpr double kReduceUs = 2.58;
+constexpr double kReduceUsPerMB = 0.217;   // per MB of (split + 1) x M x N x 4 bytes
+constexpr double kSecondLaunchUs = 3.0;    // a two-part plan's edge behind its bulk
 
-// Estimated duration (microseconds) of one launch of plan p on an M x N x K GEMM:
-// waves x wave time for the tiled kernel (at least the HBM time of its operands), the
-// operands' HBM time for the skinny kernel, plus the split-K reduction when there is one.
+// Modelled duration (microseconds) of one launch of tiled plan p.
 double plan_time_us(const wmma_gemm_plan& p, int M, int N, int K, int num_cus);
 
-// A two-part plan is taken when its estimate is below this fraction of the best
-// one-launch plan's (the estimates are within ~15% of measured times).
-constexpr double kEdgeGain = 0.93;
+// A two-part plan is taken when its estimate is below this fraction of the best one-launch
+// plan's.  Of 60 shapes timed both ways, those modelled below it ran 4-24% faster in two
+// parts (2106 x 8320 x 2552: 106 us against 138), those from there to 1 between 3% faster
+// and 4% slower.
+constexpr double kEdgeGain = 0.97;
 
 // Fill `out` for a GEMM of this shape; returns WMMA_OK or WMMA_ERR_INVALID_ARG.  With
 // tile_cfg == WMMA_TILE_AUTO on a 256-CU device, a shape found in the autotuned table
