@@ -339,24 +339,21 @@ static int gemm_run(const void* A, int64_t lda, const void* B, int64_t ldb, cons
         const hipStream_t st = static_cast<hipStream_t>(stream);
         unsigned char* dst = reinterpret_cast<unsigned char*>(
             round256(reinterpret_cast<uintptr_t>(workspace) + plan.workspace_bytes));
-        // The copy of an operand stored as n rows of `len`; its new leading dimension in *ld.
-        auto copy = [&](const void*& src, int64_t* ld, int n, int len, const char* what) -> int {
-            const int64_t len8 = ((int64_t)len + 7) & ~(int64_t)7;
-            if (int rc = hip_status(launch_gemm_repack(src, *ld, n, len, dst, st), what)) return rc;
-            src = dst;
-            *ld = len8;
-            dst += round256((size_t)n * (size_t)len8 * 2);
-            return WMMA_OK;
-        };
-        if (room && rows.a_copy) {
-            const bool ta = layout == GemmLayout::TN;
-            if (int rc = copy(A, &lda, ta ? K : M, ta ? M : K, "gemm repack A")) return rc;
-            rows.a_vec = true;
-        }
-        if (room && rows.b_copy) {
-            const bool tb = layout == GemmLayout::NT;
-            if (int rc = copy(B, &ldb, tb ? N : K, tb ? K : N, "gemm repack B")) return rc;
-            rows.b_vec = true;
+        if (room) {
+            const bool ta = layout == GemmLayout::TN, tb = layout == GemmLayout::NT;
+            GemmRepack ra, rb;
+            // An operand stored as n rows of `len`: its copy, which the GEMM reads instead.
+            auto copy = [&](GemmRepack* r, const void** src, int64_t* ld, int n, int len) {
+                *r = {*src, *ld, n, len, dst};
+                *ld = ((int64_t)len + 7) & ~(int64_t)7;
+                *src = dst;
+                dst += round256((size_t)n * (size_t)*ld * 2);
+            };
+            if (rows.a_copy) copy(&ra, &A, &lda, ta ? K : M, ta ? M : K);
+            if (rows.b_copy) copy(&rb, &B, &ldb, tb ? N : K, tb ? K : N);
+            rows.a_vec |= rows.a_copy;
+            rows.b_vec |= rows.b_copy;
+            if (int rc = hip_status(launch_gemm_repack(ra, rb, st), "gemm repack")) return rc;
         }
     }
     const bool vec = K > 0 && rows.a_vec && rows.b_vec;

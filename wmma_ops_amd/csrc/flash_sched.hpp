@@ -24,24 +24,6 @@ __device__ __forceinline__ int64_t flash_linear_id(int64_t x, int64_t y, int64_t
     return (x & 31) && (id & 32) && (id | 31) < x * y * z ? id ^ 24 : id;
 }
 
-// Division of 0 <= n < 2^31 by a divisor known at the launch: a high product, an add and a
-// shift, all scalar (Granlund and Montgomery's invariant division), where the generic one is
-// a float reciprocal and its corrections.  A workgroup's prologue divides several times, and
-// every workgroup waits for it: with generic divisions, 64-bit strides and the variable-length
-// search behind a branch of the dense kernels, 4 x 16 heads of 2048 tokens, D = 64, causal,
-// took 3% longer than with none of them; as here 1.5%.
-struct FastDiv {
-    uint32_t d, mul, shift;
-};
-inline FastDiv fast_div(uint32_t d) {
-    uint32_t l = 0;
-    while ((uint64_t(1) << l) < d) ++l;
-    return {d, (uint32_t)(((uint64_t(1) << 32) * ((uint64_t(1) << l) - d)) / d + 1), l};
-}
-__device__ __forceinline__ int div_by(const FastDiv& f, int n) {
-    return (int)((__umulhi(f.mul, (uint32_t)n) + (uint32_t)n) >> f.shift);
-}
-
 // id = row * f.d + col.
 __device__ __forceinline__ int64_t flash_split_id(int64_t id, const FastDiv& f, int* col) {
     if ((id >> 31) == 0) {

@@ -992,44 +992,65 @@ splitk_reduce_kernel(const float* ws, int split, const float* Cin, int64_t ldcin
 // ------------------------------------------------------------------------------------
 // Operand repack for rows that break 16-byte vectors: a [rows][cols] fp16 matrix with
 // leading dimension ld (any alignment) becomes a dense [rows][cols_p] copy, cols_p = cols
-// rounded up to 8, whose columns cols..cols_p-1 are zero.  One wave per row, one output
-// dword (two fp16) per lane and step; a row whose start is 4-byte aligned is read a dword
-// at a time, any other row in 16-bit halves.  Both sides are contiguous across the lanes
-// of a wave.
+// rounded up to 8, whose columns cols..cols_p-1 are zero.  Both operands of a GEMM in one
+// launch.  The copy is bound by its bytes, so a thread moves whole 16-byte chunks of the
+// output, the chunks of all rows in one run: a dword-aligned 16-byte load, where the row
+// starts on an odd element one from 2 bytes earlier plus the next dword, shifted together
+// by v_alignbyte; four chunks in flight per thread.  1001 x 4099 and 4099 x 4100: REPACKED.
 // ------------------------------------------------------------------------------------
-constexpr int RP_WAVES = 4;  // rows per workgroup
-constexpr int RP_STEPS = 4;  // dwords per lane and row (a workgroup covers 256 of a row)
+constexpr int RP_THREADS = 256;
+constexpr int RP_STEPS = 4;  // chunks per thread
 
-__global__ void __launch_bounds__(RP_WAVES * kWave)
-gemm_repack_kernel(const f16* src, int64_t ld, int rows, int cols, uint32_t* dst) {
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int dw_row = ((cols + 7) & ~7) >> 1;
-    const int w0 = blockIdx.x * (kWave * RP_STEPS) + lane;
-    for (int r = blockIdx.y * RP_WAVES + wave; r < rows; r += gridDim.y * RP_WAVES) {
-        const f16* s = src + (int64_t)r * ld;
-        const __amdgpu_buffer_rsrc_t rs = make_rsrc(s);
-        const bool al4 = (reinterpret_cast<uintptr_t>(s) & 3u) == 0;
-        uint32_t v[RP_STEPS];
+struct RepackArgs {
+    const f16* src;
+    int64_t ld;
+    int64_t chunks;  // of the copy
+    int cols;
+    FastDiv row_chunks;
+    u32x4* dst;
+};
+
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// Eight elements from s on, `left` of them valid (zeros past them).
+__device__ __forceinline__ u32x4 repack_chunk(const f16* s, int left) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(s);
+    u32x4 v{};
+    if (left >= 8) {
+        // both dwords that an odd start shares with a neighbour hold an element of the chunk
+        const uint32_t odd = (uint32_t)(at & 2);
+        const u32x4_a4 x = *reinterpret_cast<const u32x4_a4*>(at - odd);
+        const uint32_t y = odd ? *reinterpret_cast<const uint32_t*>(at + 14) : 0;
+        v = u32x4{__builtin_amdgcn_alignbyte(x[1], x[0], odd), __builtin_amdgcn_alignbyte(x[2], x[1], odd),
+                  __builtin_amdgcn_alignbyte(x[3], x[2], odd), __builtin_amdgcn_alignbyte(y, x[3], odd)};
+    } else {
+        const uint16_t* e = reinterpret_cast<const uint16_t*>(s);
 #pragma unroll
-        for (int u = 0; u < RP_STEPS; ++u) {
-            const int c = 2 * (w0 + u * kWave);  // first column of this dword
-            if (al4) {
-                v[u] = buf_load4(rs, c + 1 < cols ? (uint32_t)c * 2 : kOobOffset);
-                if (c + 1 == cols) v[u] = buf_load2(rs, (uint32_t)c * 2);  // odd cols: last one
-            } else {
-                const uint32_t lo = buf_load2(rs, c < cols ? (uint32_t)c * 2 : kOobOffset);
-                const uint32_t hi = buf_load2(rs, c + 1 < cols ? (uint32_t)(c + 1) * 2 : kOobOffset);
-                v[u] = lo | (hi << 16);
-            }
-        }
-        uint32_t* d = dst + (int64_t)r * dw_row;
+        for (int i = 0; i < 8; ++i)
+            if (i < left) v[i >> 1] |= (uint32_t)e[i] << (16 * (i & 1));
+    }
+    return v;
+}
+
+__global__ void __launch_bounds__(RP_THREADS)
+gemm_repack_kernel(RepackArgs a, RepackArgs b, int a_blocks) {
+    const bool first = (int)blockIdx.x < a_blocks;
+    const RepackArgs& p = first ? a : b;
+    const int64_t i0 = (int64_t)(first ? blockIdx.x : blockIdx.x - a_blocks) * (RP_THREADS * RP_STEPS) +
+                       threadIdx.x;
+    u32x4 v[RP_STEPS];
 #pragma unroll
-        for (int u = 0; u < RP_STEPS; ++u) {
-            const int w = w0 + u * kWave;
-            if (w < dw_row) d[w] = v[u];
+    for (int u = 0; u < RP_STEPS; ++u) {
+        const int64_t i = i0 + u * RP_THREADS;
+        if (i < p.chunks) {
+            const int64_t r = p.chunks <= INT32_MAX ? div_by(p.row_chunks, (int)i) : i / p.row_chunks.d;
+            const int c = (int)(i - r * p.row_chunks.d);
+            v[u] = repack_chunk(p.src + r * p.ld + 8 * c, p.cols - 8 * c);
         }
     }
+#pragma unroll
+    for (int u = 0; u < RP_STEPS; ++u)
+        if (i0 + u * RP_THREADS < p.chunks) p.dst[i0 + u * RP_THREADS] = v[u];
 }
 
 template <int CFG, bool VEC>
@@ -1124,13 +1145,21 @@ void launch_mfma_cfg(int cfg, const GemmArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-hipError_t launch_gemm_repack(const void* src, int64_t ld, int rows, int cols, void* dst,
-                              hipStream_t stream) {
-    if (rows <= 0 || cols <= 0) return hipSuccess;
-    const int dw_row = ((cols + 7) & ~7) >> 1;
-    const dim3 grid(ceil_div(dw_row, kWave * RP_STEPS), std::min(ceil_div(rows, RP_WAVES), 65535));
-    hipLaunchKernelGGL(gemm_repack_kernel, grid, dim3(RP_WAVES * kWave), 0, stream,
-                       static_cast<const f16*>(src), ld, rows, cols, static_cast<uint32_t*>(dst));
+hipError_t launch_gemm_repack(const GemmRepack& a, const GemmRepack& b, hipStream_t stream) {
+    int64_t blocks[2];
+    RepackArgs args[2];
+    const GemmRepack* ops[2] = {&a, &b};
+    for (int i = 0; i < 2; ++i) {
+        const GemmRepack& o = *ops[i];
+        const int row_chunks = std::max(ceil_div(o.cols, 8), 1);
+        const int64_t chunks = o.src && o.rows > 0 && o.cols > 0 ? (int64_t)o.rows * row_chunks : 0;
+        args[i] = {static_cast<const f16*>(o.src), o.ld, chunks, o.cols, fast_div(row_chunks),
+                   static_cast<u32x4*>(o.dst)};
+        blocks[i] = ceil_div64(chunks, RP_THREADS * RP_STEPS);
+    }
+    if (blocks[0] + blocks[1] == 0) return hipSuccess;
+    hipLaunchKernelGGL(gemm_repack_kernel, dim3((unsigned)(blocks[0] + blocks[1])), dim3(RP_THREADS),
+                       0, stream, args[0], args[1], (int)blocks[0]);
     return hipGetLastError();
 }
 

@@ -30,10 +30,16 @@ struct GemmLaunch {
     wmma_gemm_plan plan;
 };
 hipError_t launch_gemm(const GemmLaunch& g, hipStream_t stream);
-// Dense zero-padded copy of a [rows][cols] fp16 matrix (leading dimension ld, any
-// alignment) into dst [rows][cols rounded up to 8]; dst 4-byte aligned.
-hipError_t launch_gemm_repack(const void* src, int64_t ld, int rows, int cols, void* dst,
-                              hipStream_t stream);
+// Dense zero-padded copies of the operands whose stored rows break 16-byte vectors: [rows][cols]
+// fp16 (leading dimension ld, any alignment) into dst [rows][cols rounded up to 8], 16-byte
+// aligned.  src NULL: this operand needs none.
+struct GemmRepack {
+    const void* src = nullptr;
+    int64_t ld = 0;
+    int rows = 0, cols = 0;
+    void* dst = nullptr;
+};
+hipError_t launch_gemm_repack(const GemmRepack& a, const GemmRepack& b, hipStream_t stream);
 
 // INT4 weight layout conversions (w4a16.hip).
 hipError_t launch_int4_prepack(const int32_t* qweight, int K, int N, int32_t* packed,
