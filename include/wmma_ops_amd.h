@@ -424,8 +424,11 @@ int wmma_flash_attn_varlen_fwd_lse(const void* Q, const void* K, const void* V, 
  * to the next (`batch` is not used by the packed entry points); the D elements of a row are
  * contiguous.  All multiples of 8, K and V with equal row strides, and in the backward pass
  * Q and dO too; the rows of one head within 2^31 bytes.  O, lse and the gradients are
- * contiguous as in the entry points above, whose results these return.  No counterpart in
- * the reference.
+ * contiguous as in the entry points above and below, whose results these return, and
+ * wmma_flash_attn_varlen_bwd_strided also zeroes the gradient rows outside every sequence.
+ * Its workspace may be that of wmma_flash_attn_bwd_split_workspace_size(1, H, Hkv, total_q,
+ * total_k, D, causal), with which it splits grouped-query heads as the dense pass does.  No
+ * counterpart in the reference.
  */
 typedef struct wmma_attn_strides {
     int64_t batch, head, row;

@@ -47,3 +47,51 @@ def test_varlen_every_block_once(wo, name, h, hkv, d, causal):
     _close(o.detach(), oatt.sdpa_varlen_ref(q, k, v, cu, cu, causal))
     for got, ref in zip(grads, oatt.sdpa_varlen_bwd_ref(q, k, v, do, cu, cu, causal)):
         _close(got, ref)
+
+
+# Gradient rows outside every sequence are zero, wherever they lie: before the first, behind
+# the last, past the longest length, all of them (no sequence at all), and for offsets that
+# do not even increase.
+@pytest.mark.parametrize("cu,longest", [([40, 90, 90, 300], 210), ([0, 100, 400], 64), ([400, 400], 8),
+                                        ([0, 130, 60, 310], 400), ([0], 0)])
+def test_varlen_rows_outside_sequences(wo, cu, longest):
+    report("varlen_rows_outside_sequences", cu=cu, longest=longest)
+    total, h, hkv, d = 400, 4, 2, 64
+    g = torch.Generator().manual_seed(9)
+    q, do = (torch.randn(total, h, d, generator=g).half().cuda() for _ in range(2))
+    k, v = (torch.randn(total, hkv, d, generator=g).half().cuda() for _ in range(2))
+    c = torch.tensor(cu, dtype=torch.int32, device="cuda")
+    inside = torch.zeros(total, dtype=torch.bool)
+    for a, b in zip(cu[:-1], cu[1:]):
+        inside[a:min(b, a + longest)] = True
+    # two passes over caching-allocator memory that the first left full of NaN
+    for _ in range(2):
+        o, lse = wo.flash_attention_varlen_forward(q, k, v, c, c, longest, longest, True)
+        junk = [torch.full_like(x, float("nan")) for x in (q, k, v)]
+        del junk
+        grads = wo.flash_attention_varlen_backward(do, q, k, v, o, lse, c, c, longest, longest, True)
+        for x in grads:
+            assert torch.count_nonzero(x[~inside]) == 0
+            assert torch.isfinite(x[~inside]).all()
+            if bool(inside.any()):
+                assert torch.count_nonzero(x[inside]) > 0
+
+
+# Grouped heads over few key blocks: the group's query heads in parts, added per sequence.
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("lens,h,hkv,d", [([300, 0, 77], 8, 2, 64), ([129], 16, 1, 128), ([64, 200], 6, 2, 256)])
+def test_varlen_group_parts(wo, lens, h, hkv, d, causal):
+    report("varlen_group_parts", lens=lens, h=h, hkv=hkv, d=d, causal=causal)
+    g = torch.Generator().manual_seed(11)
+    total = sum(lens)
+    q, do = (torch.randn(total, h, d, generator=g).half() for _ in range(2))
+    k, v = (torch.randn(total, hkv, d, generator=g).half() for _ in range(2))
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    args = (cu.cuda(), cu.cuda(), max(lens), max(lens), causal)
+    x = [t.cuda() for t in (q, k, v)]
+    o, lse = wo.flash_attention_varlen_forward(*x, *args)
+    first = wo.flash_attention_varlen_backward(do.cuda(), *x, o, lse, *args)
+    for got, ref in zip(first, oatt.sdpa_varlen_bwd_ref(q, k, v, do, cu, cu, causal)):
+        _close(got, ref)
+    for got, again in zip(first, wo.flash_attention_varlen_backward(do.cuda(), *x, o, lse, *args)):
+        assert torch.equal(got, again)

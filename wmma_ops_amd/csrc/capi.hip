@@ -1046,13 +1046,14 @@ int flash_bwd_run(FlashBwdLaunch& f, void* workspace, size_t workspace_bytes, vo
             return fail(WMMA_ERR_WORKSPACE, "workspace of %zu bytes, %zu needed", workspace_bytes, need);
     }
     f.ws = static_cast<float*>(workspace);
-    // Dense grouped-query attention whose dK/dV workgroups would leave most CUs idle: the
-    // group's query heads are split over more workgroups when the workspace also holds their
-    // fp32 partial dK, dV (behind the row statistics, 256-byte aligned).
-    if (!f.cu_q && has_q && has_k) {
-        const int gs =
-            flash_bwd_group_split(f.B, f.H, f.Hkv, f.Sq, f.Sk, f.D, f.causal, current_cus());
-        const size_t part = flash_bwd_split_bytes(f.B, f.Hkv, f.Sk, f.D, gs);
+    // Grouped-query attention whose dK/dV workgroups would leave most CUs idle: the group's
+    // query heads are split over more workgroups when the workspace also holds their fp32
+    // partial dK, dV (behind the row statistics, 256-byte aligned).  Packed sequences count as
+    // one of all their rows.
+    if (has_q && has_k) {
+        const int B = f.cu_q ? 1 : f.B, Sq = f.cu_q ? f.total_q : f.Sq, Sk = f.cu_k ? f.total_k : f.Sk;
+        const int gs = flash_bwd_group_split(B, f.H, f.Hkv, Sq, Sk, f.D, f.causal, current_cus());
+        const size_t part = flash_bwd_split_bytes(B, f.Hkv, Sk, f.D, gs);
         if (gs > 1 && workspace_bytes >= round256(need) + part && aligned16(workspace)) {
             f.gsplit = gs;
             f.kv_part = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + round256(need));
@@ -1133,7 +1134,7 @@ static int flash_varlen_bwd_run(const void* dO, AttnStrides dout, const void* Q,
                                 const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
                                 void* workspace, size_t workspace_bytes, int B, int H, int Hkv,
                                 int total_q, int total_k, int max_seqlen_q, int max_seqlen_k,
-                                int D, float scale, int causal, void* stream) {
+                                int D, float scale, int causal, bool zero_gaps, void* stream) {
     if (int rc = flash_varlen_check(B, H, Hkv, total_q, total_k, max_seqlen_q, max_seqlen_k, D,
                                     scale, kFlashMaxDBwd))
         return rc;
@@ -1163,6 +1164,7 @@ static int flash_varlen_bwd_run(const void* dO, AttnStrides dout, const void* Q,
     f.k = k;
     f.v = v;
     f.dout = dout;
+    f.zero_gaps = zero_gaps;
     f.cu_q = cu_seqlens_q;
     f.cu_k = cu_seqlens_k;
     f.total_q = total_q;
@@ -1179,7 +1181,7 @@ int wmma_flash_attn_varlen_bwd(const void* dO, const void* Q, const void* K, con
     const AttnStrides q = packed_strides(H, D), kv = packed_strides(Hkv, D);
     return flash_varlen_bwd_run(dO, q, Q, q, K, kv, V, kv, O, lse, dQ, dK, dV, cu_seqlens_q,
                                 cu_seqlens_k, workspace, workspace_bytes, B, H, Hkv, total_q,
-                                total_k, max_seqlen_q, max_seqlen_k, D, scale, causal, stream);
+                                total_k, max_seqlen_q, max_seqlen_k, D, scale, causal, false, stream);
 }
 
 int wmma_flash_attn_varlen_bwd_strided(const void* dO, wmma_attn_strides dout, const void* Q,
@@ -1197,7 +1199,7 @@ int wmma_flash_attn_varlen_bwd_strided(const void* dO, wmma_attn_strides dout, c
     if (int rc = flash_stride_check(kv, 2, max_seqlen_k, "K and V")) return rc;
     return flash_varlen_bwd_run(dO, dout, Q, q, K, k, V, v, O, lse, dQ, dK, dV, cu_seqlens_q,
                                 cu_seqlens_k, workspace, workspace_bytes, B, H, Hkv, total_q,
-                                total_k, max_seqlen_q, max_seqlen_k, D, scale, causal, stream);
+                                total_k, max_seqlen_q, max_seqlen_k, D, scale, causal, true, stream);
 }
 
 }  // extern "C"

@@ -812,6 +812,24 @@ flash_bwd_dkdv_kernel(BwdArgs p) {
     }
 }
 
+// Four elements of a grouped-query split: the parts, n elements apart, added in part order.
+__device__ __forceinline__ void kv_sum4(const float* src, int gsplit, int64_t n, f16* dst) {
+    float4 a = *reinterpret_cast<const float4*>(src);
+    for (int g = 1; g < gsplit; ++g) {
+        const float4 b = *reinterpret_cast<const float4*>(src + (int64_t)g * n);
+        a.x += b.x;
+        a.y += b.y;
+        a.z += b.z;
+        a.w += b.w;
+    }
+    f16x4 o;
+    o[0] = (f16)a.x;
+    o[1] = (f16)a.y;
+    o[2] = (f16)a.z;
+    o[3] = (f16)a.w;
+    *reinterpret_cast<f16x4*>(dst) = o;
+}
+
 // dK, dV of a grouped-query split: the gsplit fp32 parts of each element added in part
 // order (deterministic) and rounded once to fp16.  Four elements per thread.
 __global__ void __launch_bounds__(256)
@@ -821,21 +839,45 @@ flash_bwd_kv_sum_kernel(const float* kv_part, int gsplit, int64_t n, f16* dK, f1
          i += (int64_t)gridDim.x * blockDim.x) {
         const bool v = i >= n4;
         const int64_t e = 4 * (v ? i - n4 : i);
-        const float* src = kv_part + (v ? (int64_t)gsplit * n : 0) + e;
-        float4 a = *reinterpret_cast<const float4*>(src);
-        for (int g = 1; g < gsplit; ++g) {
-            const float4 b = *reinterpret_cast<const float4*>(src + (int64_t)g * n);
-            a.x += b.x;
-            a.y += b.y;
-            a.z += b.z;
-            a.w += b.w;
-        }
-        f16x4 o;
-        o[0] = (f16)a.x;
-        o[1] = (f16)a.y;
-        o[2] = (f16)a.z;
-        o[3] = (f16)a.w;
-        *reinterpret_cast<f16x4*>((v ? dV : dK) + e) = o;
+        kv_sum4(kv_part + (v ? (int64_t)gsplit * n : 0) + e, gsplit, n, (v ? dV : dK) + e);
+    }
+}
+
+// The same for packed sequences: the rows of each sequence (blockIdx.y) that the dK/dV kernel
+// wrote, all heads of a row in one run.
+__global__ void __launch_bounds__(256)
+flash_bwd_kv_sum_varlen_kernel(const float* kv_part, int gsplit, int64_t n, const int* cu_k,
+                               int total_k, int max_k, int row, f16* dK, f16* dV) {
+    const int seq = blockIdx.y;
+    const int64_t first = (int64_t)min(max(cu_k[seq], 0), total_k) * row;
+    const int64_t n4 = (int64_t)varlen_len(cu_k, seq, total_k, max_k) * row / 4;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < 2 * n4;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        const bool v = i >= n4;
+        const int64_t e = first + 4 * (v ? i - n4 : i);
+        kv_sum4(kv_part + (v ? (int64_t)gsplit * n : 0) + e, gsplit, n, (v ? dV : dK) + e);
+    }
+}
+
+// Zeroes the rows of dQ (blockIdx.z = 0) or dK and dV (1) that belong to no sequence or lie past
+// the longest length: before sequence blockIdx.x, and behind the last.  The steps from one
+// sequence's processed end to the next one's start climb from row 0 to `total` together with
+// the sequences themselves, so whatever the offsets every row is in one of them.
+__global__ void __launch_bounds__(256)
+flash_bwd_gaps_kernel(const int* cu_q, const int* cu_k, int B, int total_q, int total_k, int max_q,
+                      int max_k, int row_q, int row_k, f16* dQ, f16* dK, f16* dV) {
+    const bool q = blockIdx.z == 0;
+    const int* cu = q ? cu_q : cu_k;
+    const int total = q ? total_q : total_k, b = blockIdx.x;
+    const int lo = b == 0 ? 0
+                          : min(max(cu[b - 1], 0), total) + varlen_len(cu, b - 1, total, q ? max_q : max_k);
+    const int hi = b == B ? total : min(max(cu[b], 0), total);
+    const int row = (q ? row_q : row_k) / 8;  // 16-byte chunks
+    const int64_t n = (int64_t)max(hi - lo, 0) * row, first = (int64_t)lo * row;
+    for (int64_t i = (int64_t)blockIdx.y * blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.y * blockDim.x) {
+        reinterpret_cast<u32x4*>(q ? dQ : dK)[first + i] = u32x4{};
+        if (!q) reinterpret_cast<u32x4*>(dV)[first + i] = u32x4{};
     }
 }
 
@@ -876,7 +918,13 @@ void launch_bwd_d(BwdArgs a, int B, bool causal, hipStream_t stream) {
             hipLaunchKernelGGL((flash_bwd_dkdv_kernel<D, true, false>), gk, bk, 0, stream, a);
         else
             hipLaunchKernelGGL((flash_bwd_dkdv_kernel<D, false, false>), gk, bk, 0, stream, a);
-        if (a.gsplit > 1 && a.kv_elems > 0) {
+        if (a.gsplit > 1 && a.cu_k) {
+            const int64_t longest = (int64_t)a.Sk * a.Hkv * a.dr;
+            const int grid = (int)std::min<int64_t>(ceil_div64(longest / 2, 256), 1024);
+            hipLaunchKernelGGL(flash_bwd_kv_sum_varlen_kernel, dim3(std::max(grid, 1), B), dim3(256), 0,
+                               stream, a.kv_part, a.gsplit, a.kv_elems, a.cu_k, a.total_k, a.Sk,
+                               a.Hkv * a.dr, a.dK, a.dV);
+        } else if (a.gsplit > 1 && a.kv_elems > 0) {
             const int grid = (int)std::min<int64_t>(ceil_div64(2 * (a.kv_elems / 4), 256), 8192);
             hipLaunchKernelGGL(flash_bwd_kv_sum_kernel, dim3(grid), dim3(256), 0, stream,
                                a.kv_part, a.gsplit, a.kv_elems, a.dK, a.dV);
@@ -964,11 +1012,19 @@ hipError_t launch_flash_bwd(const FlashBwdLaunch& f, hipStream_t stream) {
     a.div_bhkv = fast_div((uint32_t)f.B * f.Hkv);
     a.gsplit = 1;
     a.gper = a.group;
-    if (!f.cu_q && f.gsplit > 1 && f.kv_part) {
+    if (f.gsplit > 1 && f.kv_part) {
         a.gsplit = f.gsplit;
         a.gper = ceil_div(a.group, f.gsplit);
         a.kv_part = f.kv_part;
-        a.kv_elems = (int64_t)f.B * f.Hkv * f.Sk * f.D;
+        a.kv_elems = f.cu_q ? (int64_t)f.total_k * f.Hkv * f.D : (int64_t)f.B * f.Hkv * f.Sk * f.D;
+    }
+    if (f.cu_q && f.zero_gaps) {
+        // Only the rows outside every sequence: three fills of whole gradients took 18 us of a
+        // 1456 us step over 11091 tokens, and three launches of any step.
+        hipLaunchKernelGGL(flash_bwd_gaps_kernel, dim3(f.B + 1, 8, 2), dim3(256), 0, stream, f.cu_q,
+                           f.cu_k, f.B, f.total_q, f.total_k, f.Sq, f.Sk, f.H * f.D, f.Hkv * f.D,
+                           a.dQ, a.dK, a.dV);
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     }
     if (f.D > 128)
         launch_bwd_d<256>(a, f.B, f.causal, stream);

@@ -192,11 +192,12 @@ struct FlashBwdLaunch {
     const int* cu_q = nullptr;
     const int* cu_k = nullptr;
     int total_q = 0, total_k = 0;
-    // Dense grouped-query attention: split the dK/dV kernel's query heads of a group over
+    // Grouped-query attention: split the dK/dV kernel's query heads of a group over
     // gsplit workgroups (> 1) whose fp32 partial dK, dV go to kv_part
     // (flash_bwd_split_bytes, 16-byte aligned), added by a second kernel.
     int gsplit = 1;
     float* kv_part = nullptr;
+    bool zero_gaps = false;  // variable length: zero the gradient rows outside every sequence
     AttnStrides q, k, v, dout;  // q.row == dout.row, k.row == v.row; O and the gradients are
                                 // contiguous
 };

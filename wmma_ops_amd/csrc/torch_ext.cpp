@@ -486,14 +486,15 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> flash_attention_varlen_b
     auto dq = torch::empty({q.size(0), q.size(1), Dp}, q.options());
     auto dk = torch::empty({k.size(0), k.size(1), Dp}, k.options());
     auto dv = torch::empty_like(dk);
-    // rows outside every sequence are not written by the kernels: start from zeros
-    if (dq.numel()) dq.zero_();
-    if (dk.numel()) {
+    if (cu_q.size(0) == 1) {  // no sequence: every row lies outside
+        dq.zero_();
         dk.zero_();
         dv.zero_();
     }
-    const size_t ws_bytes = wmma_flash_attn_bwd_workspace_size(1, (int)H, (int)q.size(0));
-    auto ws = torch::empty({(int64_t)(ws_bytes / 4)}, q.options().dtype(torch::kFloat32));
+    // row statistics, plus the grouped-query split's partial dK/dV where it applies
+    const size_t ws_bytes = wmma_flash_attn_bwd_split_workspace_size(
+        1, (int)H, (int)k.size(1), (int)q.size(0), (int)k.size(0), (int)Dp, causal ? 1 : 0);
+    auto ws = torch::empty({(int64_t)((ws_bytes + 3) / 4)}, q.options().dtype(torch::kFloat32));
     int rc = wmma_flash_attn_varlen_bwd_strided(
         go.t.data_ptr(), go.s, qo.t.data_ptr(), qo.s, ko.t.data_ptr(), ko.s, vo.t.data_ptr(), vo.s,
         O.data_ptr(), lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
