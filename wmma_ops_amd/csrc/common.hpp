@@ -128,6 +128,14 @@ __device__ __forceinline__ void transpose8x8(const u32x4 in[8], u32x4 out[8]) {
 // conflict-free as well.
 __device__ __forceinline__ int swz8(int row) { return (row ^ (row >> 3)) & 7; }
 
+// Row pitch (elements) of an attention tile in LDS: the kernels' layouts and swizzles are those
+// of power-of-two rows, so head dims up to 96 keep the 128-wide layout and leave its last 32
+// columns out of the matrix work.
+template <int D>
+constexpr int attn_pitch() {
+    return D == 96 ? 128 : D;
+}
+
 // Division of 0 <= n < 2^31 by a divisor known at the launch: a high product, an add and a
 // shift, all scalar (Granlund and Montgomery's invariant division), where the generic one is
 // a float reciprocal and its corrections.  A workgroup's prologue divides several times, and

@@ -33,8 +33,8 @@
 //    only tiles crossing the diagonal are masked.  Heaviest workgroups are dispatched first.
 //  * Query rows past the end of a sequence load as zeros (dO = 0, Delta = 0), so they add
 //    nothing to dK, dV without a mask; key rows past the end are never stored.
-//  * Head dims: as in the forward, any multiple of 8 up to 128 runs on the D = 64 or D = 128
-//    kernels with the d columns past the head dim loaded as zeros and never stored.
+//  * Head dims: as in the forward, any multiple of 8 runs on the smallest kernel that holds it,
+//    with the d columns past the head dim loaded as zeros and never stored.
 #include <type_traits>
 
 #include "common.hpp"
@@ -79,8 +79,9 @@ constexpr float kLog2e = 1.4426950408889634f;
 
 template <int D>
 struct FbDim {
-    static constexpr int RB = D * 2;                    // bytes per row
-    static constexpr int DCH = D / 8;                   // 16-byte chunks per row
+    static constexpr int P = attn_pitch<D>();           // row pitch of a tile
+    static constexpr int RB = P * 2;                    // bytes per row
+    static constexpr int DCH = P / 8;                   // 16-byte chunks per row
     static constexpr int NDS = D / 16;                  // 16-wide d steps
     static constexpr int NDB = D / 32;                  // 32-wide d blocks of an accumulator
     static constexpr int TILE = FB_T * RB;              // bytes of one 64-row tile
@@ -108,7 +109,7 @@ struct FbCfg : FbDim<D> {
 // only, so offsets of 16 rows are plain additions.
 template <int D>
 __host__ __device__ constexpr int swz2(int row) {
-    return D >= 128 ? (((row & 3) << 2) | ((row >> 2) & 3))
+    return attn_pitch<D>() >= 128 ? (((row & 3) << 2) | ((row >> 2) & 3))
                     : ((((row >> 1) & 1) << 2) | ((row >> 2) & 3));
 }
 
@@ -273,7 +274,7 @@ __device__ __forceinline__ int fb_tr_addr(const FbLane<D, W>& L, int db, bool hi
 template <int D>
 constexpr bool tr_addr_identity() {
     // The XOR forms of fb_tr_addr equal the direct address for every lane and d block.
-    constexpr int RB = D * 2;
+    constexpr int RB = attn_pitch<D>() * 2;
     for (int lane = 0; lane < 64; ++lane) {
         const int g = lane >> 4, jj = (lane & 15) >> 2, aa = lane & 3;
         const int r0 = 4 * (g >> 1) + jj;
@@ -289,7 +290,8 @@ constexpr bool tr_addr_identity() {
     }
     return true;
 }
-static_assert(tr_addr_identity<256>() && tr_addr_identity<128>() && tr_addr_identity<64>(),
+static_assert(tr_addr_identity<256>() && tr_addr_identity<128>() && tr_addr_identity<96>() &&
+                  tr_addr_identity<64>(),
               "transposing-read addresses");
 
 // DMA of one 64-row tile (rows >= left load zeros).
@@ -1028,8 +1030,10 @@ hipError_t launch_flash_bwd(const FlashBwdLaunch& f, hipStream_t stream) {
     }
     if (f.D > 128)
         launch_bwd_d<256>(a, f.B, f.causal, stream);
-    else if (f.D > 64)
+    else if (f.D > 96)
         launch_bwd_d<128>(a, f.B, f.causal, stream);
+    else if (f.D > 64)
+        launch_bwd_d<96>(a, f.B, f.causal, stream);
     else
         launch_bwd_d<64>(a, f.B, f.causal, stream);
     return hipGetLastError();
