@@ -252,7 +252,9 @@ size_t wmma_w4a16_workspace_size(int M, int N, int K, int group_size);
 #define WMMA_W4_KERNEL_DECODE_MFMA 0  /* M <= 4: one workgroup per 16 columns, matrix pipe */
 #define WMMA_W4_KERNEL_DECODE 1       /* M <= 4, other group sizes: VALU dot products      */
 #define WMMA_W4_KERNEL_GEMV_SPLIT 2   /* M <= 4, narrow N: 32 columns per workgroup, split-K */
-#define WMMA_W4_KERNEL_MFMA 3         /* other shapes: tiled MFMA kernel                     */
+#define WMMA_W4_KERNEL_MFMA 3         /* other shapes: tiled MFMA kernel; group_size 32 and 64
+                                         with M <= 32: the skinny kernel, group parameters
+                                         loaded per lane                                   */
 #define WMMA_W4_KERNEL_SKINNY 4       /* 4 < M <= 32: 32/64 columns per workgroup, matrix pipe */
 #define WMMA_W4_KERNEL_GEMM 5         /* M > 32: LDS-DMA MFMA GEMM                           */
 #define WMMA_W4_KERNEL_ROWS 6         /* M > 4, short K or wide N: 16/32 rows x 16-64
@@ -278,17 +280,18 @@ int wmma_w4a16_plan_make(int M, int N, int K, int group_size, int num_cus, wmma_
  * zeros_format.  G = group_size, G % 32 == 0, K % G == 0.  With WMMA_W4_FUSED, packed is
  * the output of wmma_int4_prepack_fused and scales / zeros are not read (may be NULL).
  * Arithmetic by path (wmma_w4a16_plan_make reports the path of a shape).  The tiled
- * kernels (WMMA_W4_KERNEL_SKINNY, _GEMM, _ROWS, _MFMA, _GEMV_SPLIT) and the decode kernel at
- * M = 3, 4 form each weight exactly as written above before its fp32-accumulated product.
+ * kernels (WMMA_W4_KERNEL_SKINNY, _GEMM, _ROWS, _MFMA, _GEMV_SPLIT) and the matrix-pipe
+ * decode kernel at M = 3, 4 or group_size 32, 64 form each weight exactly as written above
+ * before its fp32-accumulated product.
  * Two decode paths form no per-weight fp16 value: WMMA_W4_KERNEL_DECODE_MFMA at M <= 2
- * and WMMA_W4_KERNEL_DECODE (M <= 4).  For each 128-deep (resp. 32-deep) K run inside a
- * group they accumulate the exact products a * (1024 + q) (a * (64 + q) at k % 8 in
- * {2,3,6,7}) and the activation sums in fp32 and add s * (D - P - z Q) once per run: the
- * same value up to fp32 rounding and the omitted fp16 rounding of each dequantised weight
- * (measured max relative error 2.2e-4 at K = 4096).  The bits of a row therefore depend
- * on the path M selects: row 0 of an M = 2 call can differ in the last bits from row 0 of
- * an M = 3 call (not batch-invariant across that boundary).  Every path is deterministic
- * (no atomics; a K split is summed in a fixed order).
+ * (group_size 128 * 2^j) and WMMA_W4_KERNEL_DECODE (M <= 4).  For each 128-deep (resp.
+ * 32-deep) K run inside a group they accumulate the exact products a * (1024 + q) (a * (64
+ * + q) at k % 8 in {2,3,6,7}) and the activation sums in fp32 and add s * (D - P - z Q)
+ * once per run: the same value up to fp32 rounding and the omitted fp16 rounding of each
+ * dequantised weight (measured max relative error 2.2e-4 at K = 4096).  The bits of a row
+ * therefore depend on the path M selects: row 0 of an M = 2 call can differ in the last
+ * bits from row 0 of an M = 3 call (not batch-invariant across that boundary).  Every path
+ * is deterministic (no atomics; a K split is summed in a fixed order).
  * No reference counterpart (BASELINE-defined W4A16 path).
  */
 int wmma_w4a16_gemm(const void* A, int64_t lda, const int32_t* packed, const void* scales,

@@ -1,4 +1,4 @@
-"""The VALU decode kernel (M <= 4, groups that are not 128 * 2^j) at activations that do not
+"""The VALU decode kernel (M <= 4, groups that are not 32 * 2^j) at activations that do not
 fill its staging rounds of 512 16-byte chunks."""
 import numpy as np
 import pytest
@@ -12,10 +12,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("zeros", ["packed", "bytes", "sliced"])
-@pytest.mark.parametrize("K", [128, 640, 1408, 4096, 5376])
+@pytest.mark.parametrize("K", [384, 1152, 1920, 4224, 5376])
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
 def test_w4a16_decode_partial_staging(wo, M, K, zeros):
-    N, G = 4096, 64
+    N, G = 4096, 96
     plan = wo.w4a16_plan(M, N, K, G)
     report("w4a16_decode_partial_staging", M=M, K=K, zeros=zeros, plan=plan)
     assert plan[0] == 1

@@ -361,8 +361,8 @@ struct W4Args {
     float* ws;            // partials [split][M][N]
     int split;
     int kc_per_split;     // 64-deep chunks per split
-    int pp_shift;         // decode-MFMA kernel: log2(G / 128)
-    int g_shift;          // LDS-DMA GEMM: log2(G) (G a power of two there)
+    int pp_shift;         // decode-MFMA, skinny and rows kernels, G >= 128: log2(G / 128)
+    int g_shift;          // LDS-DMA GEMM and the FINE forms: log2(G) (G a power of two there)
     int kg;               // K / G (groups)
     int y_half;           // Y is fp16 (each fp32 result rounded once), else fp32
 };
@@ -430,6 +430,10 @@ __device__ __forceinline__ void group_load(const W4Args& p, int g, int n, uint32
         *zraw = (uint32_t)static_cast<const int32_t*>(p.Z)[z_index<ZF>(p, g, n)];
     else
         *zraw = static_cast<const uint8_t*>(p.Z)[z_index<ZF>(p, g, n)];
+}
+// Group of K quarter `sub` (32 values) of the 128-deep pair-step pp, for G = 32 or 64.
+__device__ __forceinline__ int fine_group(const W4Args& p, int pp, int sub) {
+    return (4 * pp + sub) >> (p.g_shift - 5);
 }
 template <int ZF>
 __device__ __forceinline__ void group_decode(uint32_t sraw, uint32_t zraw, int n, uint32_t* zs,
@@ -765,7 +769,7 @@ w4a16_decode_kernel(W4Args p) {
 //   fp32, so the result differs from the fp16-rounded dequantised weights of the definition
 //   by at most their rounding (2^-11 of each weight).
 // The eight waves' partials meet in LDS at the end.  Requires G = 128 * 2^j (a pair-step
-// never straddles two groups).
+// never straddles two groups), or 32 or 64 in the FINE form below.
 // D layout: lane l holds column n = l%16 and rows m = 4*(l/16) + r; rows 0..3 live in
 // lanes 0..15.
 constexpr int DM_NW = 8;
@@ -789,11 +793,13 @@ __device__ __forceinline__ float row16_sum(float v) {
     return v;
 }
 
-template <int MM>
+template <int MM, bool FINE>
 struct DecodeMRound {
     u32x4 a[MM];    // activations: row m, pair-step l/16 of the round, chunk l%16
     u32x4 w[DM_U];  // weights of pair-steps u
-    uint32_t s, z;  // raw scale / zero of (pair-step l/16 of the round, column l%16)
+    // raw scale / zero of column l%16 and pair-step l/16 of the round; FINE: of column l%16
+    // and this lane's 32 K values of pair-step u
+    uint32_t s[FINE ? DM_U : 1], z[FINE ? DM_U : 1];
 };
 
 // Staging buffers per wave: one when a single round covers K, else two (rounds alternate).
@@ -805,7 +811,11 @@ size_t decode_mfma_lds_bytes(int M, int K) {
 
 // ONE: K <= DM_NW * DM_U * 128 -- a single round per wave, no second register set, so
 // the kernel fits 64 VGPRs and eight waves per SIMD stay resident.
-template <int ZF, bool ONE, int MM>
+// FINE: G = 32 or 64.  A lane dequantises 32 consecutive K values, so it stays inside one
+// group all the same; it loads that group's scale and zero for every pair-step itself and
+// takes the per-weight form at every M (a pair-step's sum holds more than one group, so
+// nothing can be put off to it).
+template <int ZF, bool ONE, int MM, bool FINE>
 __global__ void __launch_bounds__(DM_NW * kWave)
 __attribute__((amdgpu_waves_per_eu(ONE ? 8 : 4)))
 w4a16_decode_mfma_kernel(W4Args p) {
@@ -834,7 +844,7 @@ w4a16_decode_mfma_kernel(W4Args p) {
         reinterpret_cast<const unsigned char*>(p.W) + (int64_t)slice * fused_slice_bytes(K);
     const unsigned char* fw = fslice + fused_hdr_bytes(K);
     auto frec = [&](int pp) { return fslice + (int64_t)(pp >> 2) * kFusedBlock; };
-    auto load_round = [&](int r, DecodeMRound<MM>& R) {
+    auto load_round = [&](int r, DecodeMRound<MM, FINE>& R) {
         // this lane's activation chunk / group parameters: pair-step `sub` of the round
         const int ppl = min(pstep(r, sub), KP - 1);
         const int ka = 128 * ppl + 8 * col;
@@ -843,15 +853,14 @@ w4a16_decode_mfma_kernel(W4Args p) {
             R.a[m] = *reinterpret_cast<const u32x4*>(p.A + (int64_t)m * p.lda + ka);
         if constexpr (ZF == WMMA_W4_FUSED) {
             const unsigned char* rec = frec(ppl);
-            R.s = *reinterpret_cast<const uint16_t*>(rec + 2 * (16 * (ppl & 3) + col));
-            R.z = rec[128 + 8 * (ppl & 3) + (col >> 1)];
+            R.s[0] = *reinterpret_cast<const uint16_t*>(rec + 2 * (16 * (ppl & 3) + col));
+            R.z[0] = rec[128 + 8 * (ppl & 3) + (col >> 1)];
+        } else if constexpr (FINE) {
+#pragma unroll
+            for (int u = 0; u < DM_U; ++u)
+                group_load<ZF>(p, fine_group(p, min(pstep(r, u), KP - 1), sub), n, &R.s[u], &R.z[u]);
         } else {
-            const int g = ppl >> p.pp_shift;  // G = 128 << pp_shift
-            R.s = __builtin_bit_cast(uint16_t, p.S[s_index<ZF>(p, g, n)]);
-            if constexpr (ZF != WMMA_ZEROS_U8)
-                R.z = (uint32_t)static_cast<const int32_t*>(p.Z)[z_index<ZF>(p, g, n)];
-            else
-                R.z = static_cast<const uint8_t*>(p.Z)[z_index<ZF>(p, g, n)];
+            group_load<ZF>(p, ppl >> p.pp_shift, n, &R.s[0], &R.z[0]);  // G = 128 << pp_shift
         }
 #pragma unroll
         for (int u = 0; u < DM_U; ++u) {
@@ -868,14 +877,14 @@ w4a16_decode_mfma_kernel(W4Args p) {
     asm volatile("" : "+v"(magic), "+v"(magic_hi));  // constants in VGPRs: one v_and_or per pair
     // DEFER: scale and zero applied per pair-step (fewer VALU operations for one or two
     // rows; from three rows on the per-row sums cost as much as they save).
-    constexpr bool DEFER = MM <= 2;
+    constexpr bool DEFER = MM <= 2 && !FINE;
     f32x4 d{};              // exact path: accumulator over all pair-steps
     float y[MM], corr[MM];  // deferred path: sum of s D_t (lanes 0..15); this lane's corrections
 #pragma unroll
     for (int m = 0; m < MM; ++m) y[m] = corr[m] = 0.0f;
     const int am = col < MM ? col : 0;  // A-operand row (rows >= M repeat row 0, unused)
     const f16x2 ones = {(f16)1.0f, (f16)1.0f};
-    auto compute_round = [&](int r, const DecodeMRound<MM>& R, f16* buf) {
+    auto compute_round = [&](int r, const DecodeMRound<MM, FINE>& R, f16* buf) {
         // This lane's pair-step: its activation chunk, scale and zero.
         const bool lane_live = pstep(r, sub) < KP;
         float P[MM], Q[MM];
@@ -895,15 +904,17 @@ w4a16_decode_mfma_kernel(W4Args p) {
             // stage this lane's chunk of row m
             *reinterpret_cast<u32x4*>(buf + m * DM_ROW + 128 * sub + 8 * col) = R.a[m];
         }
-        uint32_t rs = R.s, rz = R.z;
+        auto zero_of = [&](uint32_t raw) -> uint32_t {
+            if constexpr (ZF == WMMA_W4_FUSED)
+                return (raw >> (4 * (col & 1))) & 0xFu;
+            else if constexpr (ZF != WMMA_ZEROS_U8)
+                return (raw >> (4 * (n & 7))) & 0xFu;
+            else
+                return raw & 0xFu;
+        };
+        uint32_t rs = R.s[0], rz = R.z[0];
         asm volatile("" : "+v"(rs), "+v"(rz));  // no work on them hoisted up to their load
-        uint32_t z;
-        if constexpr (ZF == WMMA_W4_FUSED)
-            z = (rz >> (4 * (col & 1))) & 0xFu;
-        else if constexpr (ZF != WMMA_ZEROS_U8)
-            z = (rz >> (4 * (n & 7))) & 0xFu;
-        else
-            z = rz & 0xFu;
+        const uint32_t z = zero_of(rz);
         if constexpr (DEFER) {
             const float sf = lane_live ? (float)__builtin_bit_cast(f16, (uint16_t)rs) : 0.0f;
             const float zf = (float)z;
@@ -915,7 +926,11 @@ w4a16_decode_mfma_kernel(W4Args p) {
         const f16* arow = buf + am * DM_ROW + 32 * sub;
 #pragma unroll
         for (int u = 0; u < DM_U; ++u) {
-            const uint32_t v = (uint32_t)__shfl(DEFER ? (int)rs : sz, 16 * u + col);
+            uint32_t v;
+            if constexpr (FINE)
+                v = R.s[u] | (zero_of(R.z[u]) << 16);
+            else
+                v = (uint32_t)__shfl(DEFER ? (int)rs : sz, 16 * u + col);
             const int pp = pstep(r, u);
             if (pp < KP) {
                 const uint32_t zz = v >> 16, s = v & 0xFFFFu;
@@ -952,7 +967,7 @@ w4a16_decode_mfma_kernel(W4Args p) {
     };
 
     if constexpr (ONE) {
-        DecodeMRound<MM> R0;
+        DecodeMRound<MM, FINE> R0;
         load_round(0, R0);
         compute_round(0, R0, sbuf);
     } else {
@@ -960,7 +975,7 @@ w4a16_decode_mfma_kernel(W4Args p) {
         // past the last round are clamped re-loads of it).  Staging buffers alternate, so
         // a wave's LDS writes for round r+1 never race its reads of round r.
         const int rounds = (KP - DM_U * wave + DM_NW * DM_U - 1) / (DM_NW * DM_U);
-        DecodeMRound<MM> R0, R1;
+        DecodeMRound<MM, FINE> R0, R1;
         load_round(0, R0);
         load_round(1, R1);
         for (int r = 0; r < rounds; r += 2) {
@@ -993,25 +1008,25 @@ w4a16_decode_mfma_kernel(W4Args p) {
     }
 }
 
-template <int ZF, bool ONE, int MM>
+template <int ZF, bool ONE, int MM, bool FINE>
 void launch_decode_mfma_m(const W4Args& a, dim3 grid, dim3 block, size_t lds, hipStream_t stream) {
     // Above 64 KB of dynamic LDS (M = 4 past one round) the kernel's launch limit is raised
     // first.
     if (lds > 64 * 1024 &&
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&w4a16_decode_mfma_kernel<ZF, ONE, MM>),
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&w4a16_decode_mfma_kernel<ZF, ONE, MM, FINE>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return;  // the error stays for the caller's hipGetLastError
-    hipLaunchKernelGGL((w4a16_decode_mfma_kernel<ZF, ONE, MM>), grid, block, lds, stream, a);
+    hipLaunchKernelGGL((w4a16_decode_mfma_kernel<ZF, ONE, MM, FINE>), grid, block, lds, stream, a);
 }
 
-template <int ZF, bool ONE>
+template <int ZF, bool ONE, bool FINE>
 void launch_decode_mfma(const W4Args& a, int M, dim3 grid, dim3 block, size_t lds,
                         hipStream_t stream) {
     switch (M) {
-        case 1: launch_decode_mfma_m<ZF, ONE, 1>(a, grid, block, lds, stream); break;
-        case 2: launch_decode_mfma_m<ZF, ONE, 2>(a, grid, block, lds, stream); break;
-        case 3: launch_decode_mfma_m<ZF, ONE, 3>(a, grid, block, lds, stream); break;
-        default: launch_decode_mfma_m<ZF, ONE, 4>(a, grid, block, lds, stream); break;
+        case 1: launch_decode_mfma_m<ZF, ONE, 1, FINE>(a, grid, block, lds, stream); break;
+        case 2: launch_decode_mfma_m<ZF, ONE, 2, FINE>(a, grid, block, lds, stream); break;
+        case 3: launch_decode_mfma_m<ZF, ONE, 3, FINE>(a, grid, block, lds, stream); break;
+        default: launch_decode_mfma_m<ZF, ONE, 4, FINE>(a, grid, block, lds, stream); break;
     }
 }
 
@@ -1035,9 +1050,11 @@ void launch_decode_mfma(const W4Args& a, int M, dim3 grid, dim3 block, size_t ld
 //    twice the workgroups of NH = 2 where 32-column tiles would leave CUs idle.
 // D layout per 16-row block b and slice sc (0 .. NH-1): lane l holds column
 // 16*NH*wg + 16*sc + l%16 and rows 16*b + 4*(l/16) + r.
+// FINE: G = 32 or 64; every lane loads the scale and zero of its own 32 K values of each
+// pair-step.
 constexpr int SK_NW = 8;
 
-template <int ZF, int MB, int U, int NH>
+template <int ZF, int MB, int U, int NH, bool FINE>
 __global__ void __launch_bounds__(SK_NW * kWave)
 w4a16_skinny_kernel(W4Args p) {
     constexpr int NC = 16 * NH;  // columns per workgroup
@@ -1052,19 +1069,15 @@ w4a16_skinny_kernel(W4Args p) {
 
     // Group parameters: lane l fetches pair-step min(l/16, U-1) of this wave for every
     // 16-column half; a lane shuffle later hands each lane its own.
-    uint32_t sraw[NH], zraw[NH];
-    {
-        const int ppl = min(kp0 + wave + SK_NW * min(sub, U - 1), KP - 1);
-        const int g = ppl >> p.pp_shift;  // G = 128 << pp_shift
+    constexpr int NP = FINE ? U : 1;
+    uint32_t sraw[NP][NH], zraw[NP][NH];
 #pragma unroll
-        for (int sc = 0; sc < NH; ++sc) {
-            const int n = n0 + 16 * sc + col;
-            sraw[sc] = __builtin_bit_cast(uint16_t, p.S[s_index<ZF>(p, g, n)]);
-            if constexpr (ZF != WMMA_ZEROS_U8)
-                zraw[sc] = (uint32_t)static_cast<const int32_t*>(p.Z)[z_index<ZF>(p, g, n)];
-            else
-                zraw[sc] = static_cast<const uint8_t*>(p.Z)[z_index<ZF>(p, g, n)];
-        }
+    for (int j = 0; j < NP; ++j) {
+        const int pp = min(kp0 + wave + SK_NW * (FINE ? j : min(sub, U - 1)), KP - 1);
+        const int g = FINE ? fine_group(p, pp, sub) : pp >> p.pp_shift;  // G = 128 << pp_shift
+#pragma unroll
+        for (int sc = 0; sc < NH; ++sc)
+            group_load<ZF>(p, g, n0 + 16 * sc + col, &sraw[j][sc], &zraw[j][sc]);
     }
     // Activations and weights, pair-step by pair-step (clamped: every load is issued).
     u32x4 av[U][MB][4], wv[U][NH];
@@ -1084,18 +1097,19 @@ w4a16_skinny_kernel(W4Args p) {
             wv[u][sc] = __builtin_nontemporal_load(wbase + (int64_t)sc * KC * 32 + (int64_t)(2 * pp + dc) * 32);
     }
 
+    int sz[NP][NH];
 #pragma unroll
-    for (int sc = 0; sc < NH; ++sc) asm volatile("" : "+v"(sraw[sc]), "+v"(zraw[sc]));
-    int sz[NH];
+    for (int j = 0; j < NP; ++j)
 #pragma unroll
-    for (int sc = 0; sc < NH; ++sc) {
-        uint32_t z;
-        if constexpr (ZF != WMMA_ZEROS_U8)
-            z = (zraw[sc] >> (4 * ((n0 + 16 * sc + col) & 7))) & 0xFu;
-        else
-            z = zraw[sc] & 0xFu;
-        sz[sc] = (int)(sraw[sc] | (z << 16));
-    }
+        for (int sc = 0; sc < NH; ++sc) {
+            asm volatile("" : "+v"(sraw[j][sc]), "+v"(zraw[j][sc]));
+            uint32_t z;
+            if constexpr (ZF != WMMA_ZEROS_U8)
+                z = (zraw[j][sc] >> (4 * ((n0 + 16 * sc + col) & 7))) & 0xFu;
+            else
+                z = zraw[j][sc] & 0xFu;
+            sz[j][sc] = (int)(sraw[j][sc] | (z << 16));
+        }
     uint32_t magic = 0x64006400u, magic_hi = 0x54005400u;
     asm volatile("" : "+v"(magic), "+v"(magic_hi));
     f32x4 d[MB][NH];
@@ -1107,7 +1121,8 @@ w4a16_skinny_kernel(W4Args p) {
     for (int u = 0; u < U; ++u) {
         uint32_t v[NH];
 #pragma unroll
-        for (int sc = 0; sc < NH; ++sc) v[sc] = (uint32_t)__shfl(sz[sc], 16 * u + col);
+        for (int sc = 0; sc < NH; ++sc)
+            v[sc] = (uint32_t)(FINE ? sz[FINE ? u : 0][sc] : __shfl(sz[0][sc], 16 * u + col));
         if (kp0 + wave + SK_NW * u < KP) {  // uniform
             f16x8 a[MB][4];
 #pragma unroll
@@ -1212,15 +1227,34 @@ void skinny_config(int M, int N, int K, int num_cus, int* nh_out, int* u_out) {
     *u_out = u;
 }
 
-template <int ZF, int MB, int NH>
+template <int ZF, int MB, int NH, bool FINE>
 void launch_skinny_mb(const W4Args& a, int U, dim3 grid, hipStream_t stream) {
     const dim3 block(SK_NW * kWave);
     if (U == 4)
-        hipLaunchKernelGGL((w4a16_skinny_kernel<ZF, MB, (MB == 1 ? 4 : 2), NH>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((w4a16_skinny_kernel<ZF, MB, (MB == 1 ? 4 : 2), NH, FINE>), grid, block, 0, stream, a);
     else if (U == 2)
-        hipLaunchKernelGGL((w4a16_skinny_kernel<ZF, MB, 2, NH>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((w4a16_skinny_kernel<ZF, MB, 2, NH, FINE>), grid, block, 0, stream, a);
     else
-        hipLaunchKernelGGL((w4a16_skinny_kernel<ZF, MB, 1, NH>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((w4a16_skinny_kernel<ZF, MB, 1, NH, FINE>), grid, block, 0, stream, a);
+}
+
+template <int ZF, bool FINE>
+void launch_skinny(const W4Args& a, const W4A16Plan& pl, hipStream_t stream) {
+    const int U = pl.k_per_split / (SK_NW * 128);
+    const dim3 grid(a.N / (16 * pl.big), pl.split);
+    if (a.M <= 16) {
+        if (pl.big == 4)
+            launch_skinny_mb<ZF, 1, 4, FINE>(a, U, grid, stream);
+        else if (pl.big == 2)
+            launch_skinny_mb<ZF, 1, 2, FINE>(a, U, grid, stream);
+        else
+            launch_skinny_mb<ZF, 1, 1, FINE>(a, U, grid, stream);
+    } else {
+        if (pl.big == 4)
+            launch_skinny_mb<ZF, 2, 4, FINE>(a, U, grid, stream);
+        else
+            launch_skinny_mb<ZF, 2, 2, FINE>(a, U, grid, stream);
+    }
 }
 
 // --------------------------------------------- rows (M > 4) on the matrix pipe, no LDS ring --
@@ -1243,6 +1277,7 @@ void launch_skinny_mb(const W4Args& a, int U, dim3 grid, hipStream_t stream) {
 // zeros without a memory request, so the loop body stays straight-line.
 // B operand: the skinny kernel's W = fp16((q - z) s), one rounding.  D layout per block b,
 // slice sc: lane l holds column 16*NH*wg + 16*sc + l%16, rows 16*MB*z + 16*b + 4*(l/16) + r.
+// FINE: G = 32 or 64; the group of a lane's scale and zero is that of its own 32 K values.
 constexpr int RW_NW = 8;
 
 template <int MB, int NH>
@@ -1252,7 +1287,7 @@ struct RowsRound {
     uint32_t s[NH], z[NH];
 };
 
-template <int ZF, int MB, int NH>
+template <int ZF, int MB, int NH, bool FINE>
 __global__ void __launch_bounds__(RW_NW * kWave)
 w4a16_rows_kernel(W4Args p) {
     constexpr int NC = 16 * NH, MR = 16 * MB;
@@ -1305,7 +1340,8 @@ w4a16_rows_kernel(W4Args p) {
     auto load_ap = [&](int r, RowsRound<MB, NH>& R) {
         const int pp = kb + wave + RW_NW * r;
         const uint32_t oob = r < rounds ? 0u : kOobOffset;
-        const uint32_t g = (uint32_t)(min(pp, KP - 1) >> p.pp_shift);  // G = 128 << pp_shift
+        const int ppc = min(pp, KP - 1);
+        const uint32_t g = FINE ? fine_group(p, ppc, sub) : ppc >> p.pp_shift;  // G = 128 << pp_shift
 #pragma unroll
         for (int sc = 0; sc < NH; ++sc) {
             R.s[sc] = buf_load2(sr, (s_lane + sc * s_sc + g * s_g) | oob);
@@ -1406,7 +1442,10 @@ w4a16_rows_kernel(W4Args p) {
 
 template <int ZF, int MB, int NH>
 void launch_rows(const W4Args& a, dim3 grid, hipStream_t stream) {
-    hipLaunchKernelGGL((w4a16_rows_kernel<ZF, MB, NH>), grid, dim3(RW_NW * kWave), 0, stream, a);
+    if (a.G < 128)
+        hipLaunchKernelGGL((w4a16_rows_kernel<ZF, MB, NH, true>), grid, dim3(RW_NW * kWave), 0, stream, a);
+    else
+        hipLaunchKernelGGL((w4a16_rows_kernel<ZF, MB, NH, false>), grid, dim3(RW_NW * kWave), 0, stream, a);
 }
 
 // ------------------------------------------------------ W4A16 GEMM (M > 32), LDS-DMA --
@@ -2047,11 +2086,14 @@ constexpr double kRowsKbPerUs = 45;
 constexpr int kRowsCfg[3][2] = {{1, 2}, {1, 4}, {2, 4}};  // {mb, nh}
 constexpr double kRowsWgFixedUs[3] = {0.75, 1.0, 2.0};
 
-// Shapes the rows kernel takes: whole 128-deep pair-steps inside one group, and weights
+// Group sizes a lane's 32 K values of a 128-deep pair-step always lie inside one group of
+// and a shift finds: 32, 64 (the kernels' FINE forms) and 128 * 2^j.
+bool w4a16_pow2_group(int G) { return G >= 32 && (G & (G - 1)) == 0; }
+
+// Shapes the rows kernel takes: whole 128-deep pair-steps, such a group size, and weights
 // addressable with 32-bit byte offsets.
 bool rows_shape_ok(int N, int K, int G) {
-    return K % 128 == 0 && G % 128 == 0 && ((G / 128) & (G / 128 - 1)) == 0 &&
-           (int64_t)N * K < ((int64_t)1 << 32);
+    return K % 128 == 0 && w4a16_pow2_group(G) && (int64_t)N * K < ((int64_t)1 << 32);
 }
 
 // Tile config and split of the LDS-DMA GEMM, or (rows_mb > 0) the rows kernel's shape.
@@ -2081,7 +2123,7 @@ void w4g_model_plan(int M, int N, int K, int G, int num_cus, int* cfg_out, int* 
             }
         }
     }
-    if (!rows_shape_ok(N, K, G)) return;
+    if (G < 128 || !rows_shape_ok(N, K, G)) return;
     for (int c = 0; c < 3; ++c) {
         const int mb = kRowsCfg[c][0], nh = kRowsCfg[c][1];
         if (N % (16 * nh) != 0) continue;
@@ -2158,7 +2200,7 @@ bool w4a16_narrow_skinny(int M, int N, int K, int num_cus) {
 }
 
 // Host-only: choose the kernel and K split.
-//   decode-mfma  M <= 4, G = 128 * 2^j, K % 128 == 0 and the staged activations fit LDS, at
+//   decode-mfma  M <= 4, G = 32 * 2^j, K % 128 == 0 and the staged activations fit LDS, at
 //                any N (narrow N included: at N = 256..1536, K = 1024..14336 it runs
 //                1.2-2.5x faster than the split GEMV), except the narrow, long-K shapes
 //                above, which take the skinny kernel.
@@ -2166,14 +2208,19 @@ bool w4a16_narrow_skinny(int M, int N, int K, int num_cus) {
 //                other group sizes.
 //   gemv-split   other M <= 4 shapes: one workgroup per 32 columns, K split (plus a reduce
 //                pass) only when fewer than 2*CUs workgroups would exist.
-//   skinny       4 < M <= 32 (and the narrow, long-K M <= 4 shapes) with G = 128 * 2^j: 16,
+//   skinny       4 < M <= 32 (and the narrow, long-K M <= 4 shapes) with G = 32 * 2^j: 16,
 //                32 or 64 columns per workgroup, K split (plus a reduce pass) only when the
-//                tiles alone give under half a workgroup per CU.
+//                tiles alone give under half a workgroup per CU.  G = 32 and 64 report
+//                W4_MFMA (slices in `big`).
+//   G = 32 and 64 on these two and on rows (M <= 32), us at G = 64, the kernels below in
+//   their place -> these: M = 1, N = 14336, K = 4096 8.9 -> 7.7; M = 4, N = 4096, K = 14336
+//   26.6 -> 9.1; M = 16, N = 14336, K = 4096 27.2 -> 10.1; M = 32, N = K = 4096 13.6 -> 6.7.
+//   What bounds them at M <= 2 is the per-weight dequantisation (G = 128: 5.9).
 //   gemm         M > 32 with G a power of two: LDS-DMA MFMA GEMM (tile below), K split
 //                (plus a reduce pass) only when the tiles cannot fill the chip.
-//   rows         4 < M <= 1024 with G = 128 * 2^j where the launch model prefers it to
-//                the skinny plan (M <= 32) or to every LDS-DMA plan (short K, few
-//                columns): no ring, no split.
+//   rows         4 < M <= 1024 with G = 128 * 2^j (M <= 32: 32 * 2^j) where the launch
+//                model prefers it to the skinny plan (M <= 32) or to every LDS-DMA plan
+//                (short K, few columns): no ring, no split.
 //   mfma         everything else (the shapes the kernels above do not take).
 W4A16Plan w4a16_plan(int M, int N, int K, int G, int num_cus, bool aligned) {
     if (num_cus <= 0) num_cus = 256;
@@ -2181,7 +2228,7 @@ W4A16Plan w4a16_plan(int M, int N, int K, int G, int num_cus, bool aligned) {
     pl.split = 1;
     pl.k_per_split = K;
     (void)aligned;
-    const bool g_ok = G % 128 == 0 && ((G / 128) & (G / 128 - 1)) == 0;
+    const bool g_ok = w4a16_pow2_group(G);
     const bool narrow_skinny = K % 128 == 0 && g_ok && w4a16_narrow_skinny(M, N, K, num_cus);
     if (M >= 1 && M <= DM_MAXM && K % 128 == 0 && g_ok && !narrow_skinny &&
         decode_mfma_lds_bytes(M, K) <= kDecodeMfmaLdsMax) {
@@ -2204,7 +2251,7 @@ W4A16Plan w4a16_plan(int M, int N, int K, int G, int num_cus, bool aligned) {
             return pl;
         }
         pl.big = nh;
-        pl.kind = W4_SKINNY;
+        pl.kind = G >= 128 ? W4_SKINNY : W4_MFMA;
         pl.k_per_split = SK_NW * u * 128;
         pl.split = ceil_div(K, pl.k_per_split);
         return pl;
@@ -2282,10 +2329,15 @@ hipError_t launch_w4a16_zf(const W4Args& a, const W4A16Launch& w, hipStream_t st
     if (pl.kind == W4_DECODE_MFMA) {
         const size_t lds = decode_mfma_lds_bytes(w.M, w.K);
         const dim3 grid(w.N / 16), block(DM_NW * kWave);
-        if (decode_mfma_one(w.K))
-            launch_decode_mfma<ZF, true>(a, w.M, grid, block, lds, stream);
+        const bool one = decode_mfma_one(w.K);
+        if (w.G < 128 && one)
+            launch_decode_mfma<ZF, true, true>(a, w.M, grid, block, lds, stream);
+        else if (w.G < 128)
+            launch_decode_mfma<ZF, false, true>(a, w.M, grid, block, lds, stream);
+        else if (one)
+            launch_decode_mfma<ZF, true, false>(a, w.M, grid, block, lds, stream);
         else
-            launch_decode_mfma<ZF, false>(a, w.M, grid, block, lds, stream);
+            launch_decode_mfma<ZF, false, false>(a, w.M, grid, block, lds, stream);
         return hipGetLastError();
     }
     if (pl.kind == W4_DECODE) {
@@ -2323,21 +2375,9 @@ hipError_t launch_w4a16_zf(const W4Args& a, const W4A16Launch& w, hipStream_t st
         else
             launch_rows<ZF, 2, 4>(a, grid, stream);
     } else if (pl.kind == W4_SKINNY) {
-        const int U = pl.k_per_split / (SK_NW * 128);
-        const dim3 grid(w.N / (16 * pl.big), pl.split);
-        if (w.M <= 16) {
-            if (pl.big == 4)
-                launch_skinny_mb<ZF, 1, 4>(a, U, grid, stream);
-            else if (pl.big == 2)
-                launch_skinny_mb<ZF, 1, 2>(a, U, grid, stream);
-            else
-                launch_skinny_mb<ZF, 1, 1>(a, U, grid, stream);
-        } else {
-            if (pl.big == 4)
-                launch_skinny_mb<ZF, 2, 4>(a, U, grid, stream);
-            else
-                launch_skinny_mb<ZF, 2, 2>(a, U, grid, stream);
-        }
+        launch_skinny<ZF, false>(a, pl, stream);
+    } else if (pl.kind == W4_MFMA && pl.big > 0) {
+        launch_skinny<ZF, true>(a, pl, stream);
     } else if (pl.kind == W4_GEMV_SPLIT) {
         hipLaunchKernelGGL((w4a16_gemv_kernel<ZF>), dim3(ntiles, pl.split), dim3(GV_NW * kWave), 0,
                            stream, a);
@@ -2399,9 +2439,9 @@ hipError_t launch_w4a16(const W4A16Launch& w, hipStream_t stream) {
         const size_t lds = decode_mfma_lds_bytes(w.M, w.K);
         const dim3 grid(w.N / 16), block(DM_NW * kWave);
         if (decode_mfma_one(w.K))
-            launch_decode_mfma<WMMA_W4_FUSED, true>(a, w.M, grid, block, lds, stream);
+            launch_decode_mfma<WMMA_W4_FUSED, true, false>(a, w.M, grid, block, lds, stream);
         else
-            launch_decode_mfma<WMMA_W4_FUSED, false>(a, w.M, grid, block, lds, stream);
+            launch_decode_mfma<WMMA_W4_FUSED, false, false>(a, w.M, grid, block, lds, stream);
         return hipGetLastError();
     }
     if (w.zeros_format == WMMA_ZEROS_PACKED) return launch_w4a16_zf<WMMA_ZEROS_PACKED>(a, w, stream);
