@@ -996,11 +996,13 @@ splitk_reduce_kernel(const float* ws, int split, const float* Cin, int64_t ldcin
 // launch.  The copy is bound by its bytes, so a thread moves whole 16-byte chunks of the
 // output, the chunks of all rows in one run: a dword-aligned 16-byte load, where the row
 // starts on an odd element one from 2 bytes earlier plus the next dword, shifted together
-// by v_alignbyte; four chunks in flight per thread.  1001 x 4099 and 4099 x
-// 4100: 14.6 us, 5.7 TB/s (a launch each of a dword per lane and step: 6.3 + 19.3 us).
+// by v_alignbyte; one chunk per thread.  1001 x 4099 and 4099 x 4100: 14.0 us, 5.9 TB/s (a
+// launch each of a dword per lane and step: 6.3 + 12.8 us); 9 x 5995 2.4 us (3.0).  Four
+// chunks per thread took 14.1 and 3.6 us, 513 x 4099 and 4099 x 1025 9.2 for 7.3: the
+// copies that fit the caches are bound by the chain of one thread, not by the loads in
+// flight.
 // ------------------------------------------------------------------------------------
 constexpr int RP_THREADS = 256;
-constexpr int RP_STEPS = 4;  // chunks per thread
 
 struct RepackArgs {
     const f16* src;
@@ -1025,10 +1027,13 @@ __device__ __forceinline__ u32x4 repack_chunk(const f16* s, int left) {
         v = u32x4{__builtin_amdgcn_alignbyte(x[1], x[0], odd), __builtin_amdgcn_alignbyte(x[2], x[1], odd),
                   __builtin_amdgcn_alignbyte(x[3], x[2], odd), __builtin_amdgcn_alignbyte(y, x[3], odd)};
     } else {
+        // every load issued (past the row: its last element again), then the masks
         const uint16_t* e = reinterpret_cast<const uint16_t*>(s);
+        uint32_t x[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (i < left) v[i >> 1] |= (uint32_t)e[i] << (16 * (i & 1));
+        for (int i = 0; i < 8; ++i) x[i] = e[min(i, left - 1)];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i >> 1] |= (i < left ? x[i] : 0u) << (16 * (i & 1));
     }
     return v;
 }
@@ -1037,21 +1042,11 @@ __global__ void __launch_bounds__(RP_THREADS)
 gemm_repack_kernel(RepackArgs a, RepackArgs b, int a_blocks) {
     const bool first = (int)blockIdx.x < a_blocks;
     const RepackArgs& p = first ? a : b;
-    const int64_t i0 = (int64_t)(first ? blockIdx.x : blockIdx.x - a_blocks) * (RP_THREADS * RP_STEPS) +
-                       threadIdx.x;
-    u32x4 v[RP_STEPS];
-#pragma unroll
-    for (int u = 0; u < RP_STEPS; ++u) {
-        const int64_t i = i0 + u * RP_THREADS;
-        if (i < p.chunks) {
-            const int64_t r = p.chunks <= INT32_MAX ? div_by(p.row_chunks, (int)i) : i / p.row_chunks.d;
-            const int c = (int)(i - r * p.row_chunks.d);
-            v[u] = repack_chunk(p.src + r * p.ld + 8 * c, p.cols - 8 * c);
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < RP_STEPS; ++u)
-        if (i0 + u * RP_THREADS < p.chunks) p.dst[i0 + u * RP_THREADS] = v[u];
+    const int64_t i = (int64_t)(first ? blockIdx.x : blockIdx.x - a_blocks) * RP_THREADS + threadIdx.x;
+    if (i >= p.chunks) return;
+    const int64_t r = p.chunks <= INT32_MAX ? div_by(p.row_chunks, (int)i) : i / p.row_chunks.d;
+    const int c = (int)(i - r * p.row_chunks.d);
+    p.dst[i] = repack_chunk(p.src + r * p.ld + 8 * c, p.cols - 8 * c);
 }
 
 template <int CFG, bool VEC>
@@ -1156,7 +1151,7 @@ hipError_t launch_gemm_repack(const GemmRepack& a, const GemmRepack& b, hipStrea
         const int64_t chunks = o.src && o.rows > 0 && o.cols > 0 ? (int64_t)o.rows * row_chunks : 0;
         args[i] = {static_cast<const f16*>(o.src), o.ld, chunks, o.cols, fast_div(row_chunks),
                    static_cast<u32x4*>(o.dst)};
-        blocks[i] = ceil_div64(chunks, RP_THREADS * RP_STEPS);
+        blocks[i] = ceil_div64(chunks, RP_THREADS);
     }
     if (blocks[0] + blocks[1] == 0) return hipSuccess;
     hipLaunchKernelGGL(gemm_repack_kernel, dim3((unsigned)(blocks[0] + blocks[1])), dim3(RP_THREADS),
