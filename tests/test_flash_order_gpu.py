@@ -95,3 +95,11 @@ def test_varlen_group_parts(wo, lens, h, hkv, d, causal):
         _close(got, ref)
     for got, again in zip(first, wo.flash_attention_varlen_backward(do.cuda(), *x, o, lse, *args)):
         assert torch.equal(got, again)
+
+
+# The order's rule: a group's parts count towards the grid (16 / 2 heads), and whole rows of 32
+# heads keep their plain order without a causal mask.
+@pytest.mark.parametrize("lens,h,hkv,d", [([700, 1300, 40, 300], 16, 2, 128), ([600, 1100, 70], 32, 32, 64)])
+def test_varlen_order_rule(wo, lens, h, hkv, d):
+    report("varlen_order_rule", lens=lens, h=h, hkv=hkv, d=d)
+    test_varlen_group_parts(wo, lens, h, hkv, d, False)

@@ -887,12 +887,13 @@ template <int D>
 void launch_bwd_d(BwdArgs a, int B, bool causal, hipStream_t stream) {
     a.nqb = ceil_div(a.Sq, FbGeom<D>::BLOCK_Q);
     const dim3 bq(FbGeom<D>::WQ * kWave), bk(FB_WAVES_KV * kWave);
-    const bool order_q = a.cu_q && varlen_ordered((int64_t)B * a.H, a.nqb);
+    const bool order_q = a.cu_q && varlen_ordered(B, a.H, a.nqb, 1, causal);
     const int nkb = ceil_div(a.Sk, FbKv<D>::BLOCK);
-    const bool order_k = a.cu_q && varlen_ordered((int64_t)B * a.Hkv, nkb);
+    const int parts = FbKv<D>::DSPLIT * a.gsplit;
+    const bool order_k = a.cu_q && varlen_ordered(B, a.Hkv, nkb, parts, causal);
     const dim3 gq(B * a.H, order_q ? varlen_grid_y(B, a.total_q, a.Sq, FbGeom<D>::BLOCK_Q) : a.nqb);
     const dim3 gk(B * a.Hkv, order_k ? varlen_grid_y(B, a.total_k, a.Sk, FbKv<D>::BLOCK) : nkb,
-                  FbKv<D>::DSPLIT * a.gsplit);
+                  parts);
     a.ordered = order_q;
     a.grid_y = gq.y;
     // The dQ kernel writes the row statistics the dK/dV kernel reads: same stream, in order.

@@ -595,7 +595,7 @@ flash_combine_kernel(const float* o_part, const float* ml_part, int split, int64
 template <int D>
 void launch_d(FlashArgs a, int BH, bool causal, hipStream_t stream) {
     a.nqb = ceil_div(a.Sq, FaCfg<D>::BQ);
-    a.ordered = a.cu_q && varlen_ordered(BH, a.nqb);
+    a.ordered = a.cu_q && varlen_ordered(a.B, a.H, a.nqb, 1, causal);
     const int rows = a.ordered ? varlen_grid_y(a.B, a.total_q, a.Sq, FaCfg<D>::BQ) : a.nqb;
     dim3 grid(BH, rows, a.kv_chunk ? ceil_div(a.Sk, a.kv_chunk) : 1);
     const dim3 block(FaCfg<D>::WAVES * kWave);

@@ -149,13 +149,19 @@ __device__ __forceinline__ bool varlen_item(const int* cu_q, const int* cu_k, in
     return false;
 }
 
-// Whether a varlen grid of `columns` (sequences x heads) by `blocks` per longest sequence takes
-// its items in that order.  Where every workgroup has a CU at once, or a few short sequences
-// finish before an uneven engine matters, the search would be a visible part of them (eight
-// sequences of 33 to 966 tokens, 8 heads: 32.6 us in plain order, 33.2 searched; five of at
-// most 322, 40 heads: 21.1 and 21.8).
-inline bool varlen_ordered(int64_t columns, int64_t blocks) {
-    return columns * blocks > (blocks > 2 ? 256 : 1024);
+// Whether a varlen grid of B sequences by `heads`, `blocks` per longest sequence and `parts`
+// workgroups per block takes its items in that order.  Where every workgroup has a CU at once,
+// or a few short sequences finish before an uneven engine matters, the search would be a
+// visible part of them (eight sequences of 33 to 966 tokens, 8 heads: 32.6 us in plain order,
+// 33.2 searched; five of at most 322, 40 heads: 21.1 and 21.8).  The parts count: 16 / 2 heads,
+// 1885, 2714, 371 and 949 tokens in 3 parts are 528 ids, the longest sequence's on one XCD
+// (dK/dV 584 us in plain order, 246 in this one).  Without a causal mask, whole rows of 32
+// heads load the engines evenly as they are, and ran faster mixed than heaviest first (32 heads,
+// forward / dQ / dK/dV: 1945 and 276 tokens, D = 64, 61 / 75 / 90 us against 67 / 81 / 93; 1500,
+// 1500, 900 and 300, D = 128, 123 / 161 / 216 against 119 / 155 / 239).
+inline bool varlen_ordered(int64_t B, int64_t heads, int64_t blocks, int64_t parts, bool causal) {
+    if (!causal && heads % 32 == 0) return false;
+    return B * heads * blocks * parts > (blocks > 2 ? 256 : 1024);
 }
 
 // Workgroups that a varlen grid needs for its items: no more than max_len / block per
