@@ -94,3 +94,24 @@ def test_other_strides_are_copied(wo):
     far.copy_(A[:2])
     _close(wo.matmul(far, B.cuda()), ref[:2])
     _close(wo.matmul(B.cuda().t(), far.t()), og.gemm_ref(B.t(), A[:2].t()))
+
+
+# Two-part plans of each layout: an edge of the transposed B's streaming kernel with a K split
+# (its workspace is not that of the plain layout's edge) and without one, of the tiled kernel,
+# of rows and of columns.
+@pytest.mark.parametrize("m,n,k", [(1300, 11008, 4096), (2840, 11008, 4096), (4100, 4096, 1024),
+                                   (2848, 11008, 4096), (4096, 4104, 1024), (785, 18944, 3584)])
+def test_transposed_two_part(wo, m, n, k):
+    report("transposed_two_part", m=m, n=n, k=k)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    a = torch.randn(m, k, generator=g, device="cuda").half()
+    w = torch.randn(n, k, generator=g, device="cuda").half()
+    C = torch.randn(m, n, generator=g, device="cuda")
+    ref = a.float() @ w.float().t()
+    at = a.t().contiguous().t()
+    for x, y in ((a, w.t()), (at, w.t().contiguous())):
+        _close(wo.matmul(x, y), ref.cpu())
+        _close(wo.gemm(x, y, 2.0, 0.5, C), (2.0 * ref + 0.5 * C).cpu())
+        out = C.clone()
+        wo.gemm_inplace(x, y, out, 2.0, 0.5)
+        _close(out, (2.0 * ref + 0.5 * C).cpu())

@@ -213,8 +213,11 @@ static wmma_gemm_plan tiled_plan(int M, int N, int K, int num_cus, size_t max_ws
 // rest as a GEMM of its own, planned on its own (it is small, so it may take a smaller
 // tile or a K split and spread over the chip).  Measured on MI355X (N = K = 4096): M = 4352
 // one launch of 128x128 tiles 193 us, 4096 + 256 rows 148 us; M = 5000: 209 vs 171 us;
-// M = 9192: 347 vs 295 us.  Taken when plan_time_us says it gains more than 7%.
-static void two_part(int M, int N, int K, int num_cus, size_t max_ws, wmma_gemm_plan* p) {
+// M = 9192: 347 vs 295 us.  Taken when the modelled time gains more than kEdgeGain asks for.
+// The edge is planned and priced for the layout it runs in, as the launch plans it: the
+// streaming kernels of the layouts differ in their K splits, hence in their workspaces.
+static void two_part(GemmLayout layout, int M, int N, int K, int num_cus, size_t max_ws,
+                     wmma_gemm_plan* p) {
     const int64_t tm = ceil_div(M, 256), tn = ceil_div(N, 256);
     const int64_t whole = tm * tn / num_cus * num_cus;  // 256x256 tiles in whole waves
     if (whole == 0) return;
@@ -228,11 +231,13 @@ static void two_part(int M, int N, int K, int num_cus, size_t max_ws, wmma_gemm_
         const int em = dim == WMMA_EDGE_ROWS ? M - at : M, en = dim == WMMA_EDGE_ROWS ? N : N - at;
         wmma_gemm_plan bulk{}, edge{};
         if (make_custom_plan(bm, bn, K, WMMA_KERNEL_TILED, WMMA_TILE_256x256, 1, &bulk) != WMMA_OK ||
-            make_plan_within(em, en, K, WMMA_TILE_AUTO, num_cus, max_ws, &edge) != WMMA_OK ||
+            make_layout_plan(layout, em, en, K, WMMA_TILE_AUTO, num_cus, max_ws, &edge) != WMMA_OK ||
             edge.edge_dim != WMMA_EDGE_NONE)
             continue;
-        const double t = plan_time_us(bulk, bm, bn, K, num_cus) +
-                         plan_time_us(edge, em, en, K, num_cus) + kSecondLaunchUs;
+        const bool skinny_nt = layout == GemmLayout::NT && edge.kernel == WMMA_KERNEL_SKINNY;
+        const double t = plan_time_us(bulk, bm, bn, K, num_cus) + kSecondLaunchUs +
+                         (skinny_nt ? skinny_nt_time_us(edge, em, en, K, num_cus)
+                                    : plan_time_us(edge, em, en, K, num_cus));
         // columns only where they are 2% better than rows: each row of their edge is a short
         // run of B and C (2560 x 14336 x 4096: 280 us by rows, 286 by columns, modelled level)
         if (t < (p->edge_dim == WMMA_EDGE_ROWS ? 0.98 : 1.0) * best_t) {
@@ -251,6 +256,13 @@ int make_plan(int M, int N, int K, int tile_cfg, int num_cus, wmma_gemm_plan* ou
 
 int make_plan_within(int M, int N, int K, int tile_cfg, int num_cus, size_t max_ws,
                      wmma_gemm_plan* out) {
+    return make_layout_plan(GemmLayout::NN, M, N, K, tile_cfg, num_cus, max_ws, out);
+}
+
+// The plan of the kernels that take every layout, and of the plain layout's streaming kernel;
+// `layout` is that of a two-part plan's edge.
+static int plain_plan(GemmLayout layout, int M, int N, int K, int tile_cfg, int num_cus,
+                      size_t max_ws, wmma_gemm_plan* out) {
     if (!out || M < 0 || N < 0 || K < 0) return WMMA_ERR_INVALID_ARG;
     if (tile_cfg < WMMA_TILE_AUTO || tile_cfg >= WMMA_TILE_COUNT) return WMMA_ERR_INVALID_ARG;
     if (num_cus <= 0) num_cus = 256;
@@ -323,7 +335,7 @@ int make_plan_within(int M, int N, int K, int tile_cfg, int num_cus, size_t max_
         return WMMA_OK;
     }
     p = tiled_plan(M, N, K, num_cus, max_ws);
-    if (p.split_k == 1) two_part(M, N, K, num_cus, max_ws, &p);
+    if (p.split_k == 1) two_part(layout, M, N, K, num_cus, max_ws, &p);
     *out = p;
     return WMMA_OK;
 }
@@ -362,7 +374,7 @@ int make_layout_plan(GemmLayout layout, int M, int N, int K, int tile_cfg, int n
         *out = skinny_nt_plan(M, N, K, num_cus, max_ws);
         return WMMA_OK;
     }
-    int rc = make_plan_within(M, N, K, tile_cfg, num_cus, max_ws, out);
+    int rc = plain_plan(layout, M, N, K, tile_cfg, num_cus, max_ws, out);
     if (rc == WMMA_OK && layout != GemmLayout::NN && out->kernel == WMMA_KERNEL_SKINNY)
         *out = model_plan(M, N, K, num_cus, max_ws, /*skinny=*/false);
     return rc;

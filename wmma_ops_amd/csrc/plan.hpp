@@ -108,7 +108,8 @@ constexpr int kSkinnyNtRound = 1024;
 // either layout and keeps the plan of the plain layout (its tiles read whole 64-byte or
 // longer runs of every operand in each of them); the streaming kernel reads B row-major
 // only: TN takes a tiled plan instead, NT at M <= kSkinnyNtMaxM a plan of its own kernel
-// (tile_m 16 or 32, tile_n 16, 32 or 64 columns per workgroup).
+// (tile_m 16 or 32, tile_n 16, 32 or 64 columns per workgroup).  The same holds for the edge
+// of a two-part plan, whose workspace_bytes is what this function's plan of the edge needs.
 int make_layout_plan(GemmLayout layout, int M, int N, int K, int tile_cfg, int num_cus,
                      size_t max_ws, wmma_gemm_plan* out);
 
