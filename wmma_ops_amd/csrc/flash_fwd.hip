@@ -567,10 +567,12 @@ flash_combine_kernel(const float* o_part, const float* ml_part, int split, int64
             }
 #pragma unroll
             for (int j = 0; j < FA_ZB; ++j) {
-                if (mz[j] == kNegInf) continue;  // a chunk with no live key
+                // A chunk with no live key has max -inf, sum 0 and O = 0.  One whose scores
+                // are all NaN has max -inf too, but a NaN sum and O: weight 0, not skipped,
+                // so that the row ends as one pass over its keys leaves it.
                 const float mn = fmaxf(m, mz[j]);
-                const float a = __builtin_amdgcn_exp2f(m - mn);  // 0 while m is -inf
-                const float w = __builtin_amdgcn_exp2f(mz[j] - mn);
+                const float a = m == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
+                const float w = mz[j] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(mz[j] - mn);
                 l = l * a + w * lz[j];
                 acc.x = acc.x * a + w * oz[j].x;
                 acc.y = acc.y * a + w * oz[j].y;
