@@ -115,3 +115,36 @@ def test_transposed_two_part(wo, m, n, k):
         out = C.clone()
         wo.gemm_inplace(x, y, out, 2.0, 0.5)
         _close(out, (2.0 * ref + 0.5 * C).cpu())
+
+
+def test_one_row_at_any_stride(wo):
+    # A contiguous tensor of one row may carry any row stride: the transpose of a column has 1.
+    g = torch.Generator().manual_seed(8)
+    B, W = torch.randn(96, 200, generator=g).half(), torch.randn(200, 1, generator=g).half()
+    col, C = torch.randn(96, 1, generator=g).half(), torch.randn(200, 1, generator=g)
+    x = torch.randn(50, 1, generator=g).half()
+    ref = og.gemm_ref(col.t(), B)
+    report("one_row_at_any_stride", strides=col.t().stride())
+    _close(wo.matmul(col.cuda().t(), B.cuda()), ref)
+    far = torch.empty(96, dtype=torch.half, device="cuda").as_strided((1, 96), (1 << 40, 1))
+    far.copy_(col.t())
+    _close(wo.matmul(far, B.cuda()), ref)
+    _close(wo.matmul(x.cuda(), W.cuda().t()), og.gemm_ref(x, W.t()))           # B [1, N]
+    _close(wo.matmul_tiled(x.cuda(), W.cuda().t(), 0), og.gemm_ref(x, W.t()))
+    ref = og.gemm_ref(col.t(), B, 2.0, 0.5, C.t())
+    _close(wo.gemm(col.cuda().t(), B.cuda(), 2.0, 0.5, C.cuda().t()), ref)
+    out = C.cuda().t()
+    wo.gemm_inplace(col.cuda().t(), B.cuda(), out, 2.0, 0.5)
+    _close(out, ref)
+
+
+def test_int4_one_row_at_any_stride(wo):
+    g = torch.Generator().manual_seed(9)
+    q = torch.randint(-2 ** 31, 2 ** 31, (32, 64), generator=g, dtype=torch.int64).int().cuda()
+    s = (torch.rand(2, 64, generator=g) * 0.01).half().cuda()
+    z = torch.randint(0, 16, (2, 64), generator=g, dtype=torch.uint8).cuda()
+    a = torch.randn(256, 1, generator=g).half().cuda()
+    row = a.reshape(1, 256).clone()
+    p, f = wo.prepack_int4(q), wo.prepack_int4_fused(q, s, z, 128)
+    assert torch.equal(wo.matmul_int4(a.t(), p, s, z, 128), wo.matmul_int4(row, p, s, z, 128))
+    assert torch.equal(wo.matmul_int4_fused(a.t(), f, 128), wo.matmul_int4_fused(row, f, 128))

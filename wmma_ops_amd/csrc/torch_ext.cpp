@@ -70,16 +70,16 @@ constexpr int64_t kMaxViewStride = 4000000;
 
 // A tensor that is not contiguous but keeps whole rows (a slice of columns) or whole columns
 // (a transpose) in order is read where it is; anything else (steps, expanded or overlapping
-// rows, longer strides) as a contiguous copy.
+// rows, longer strides) as a contiguous copy.  The row stride of a contiguous tensor is its row
+// length: a single row may carry any stride (1 for the transpose of a column).
 GemmOperand gemm_operand(const torch::Tensor& t) {
     const int64_t r = t.size(0), c = t.size(1);
-    if (t.is_contiguous()) return {t, t.stride(0), false};
+    if (t.is_contiguous()) return {t, c, false};
     if (r > 1 && c > 1 && std::max(t.stride(0), t.stride(1)) <= kMaxViewStride) {
         if (t.stride(1) == 1 && t.stride(0) >= c) return {t, t.stride(0), false};
         if (t.stride(0) == 1 && t.stride(1) >= r) return {t, t.stride(1), true};
     }
-    torch::Tensor copy = t.contiguous();
-    return {copy, copy.stride(0), false};
+    return {t.contiguous(), c, false};
 }
 
 // A and B as the GEMM reads them; of two transposed ones the smaller is copied.
@@ -89,12 +89,12 @@ void gemm_operands(const torch::Tensor& A, const torch::Tensor& B, GemmOperand* 
     if (a->trans && b->trans) {
         GemmOperand* x = A.numel() <= B.numel() ? a : b;
         x->t = x->t.contiguous();
-        x->ld = x->t.stride(0);
+        x->ld = x->t.size(1);
         x->trans = false;
     }
 }
 
-// One GEMM through the C-ABI.  C_in may be undefined; C_out preallocated.
+// One GEMM through the C-ABI.  C_in may be undefined; C_out preallocated; both contiguous.
 void run_gemm(const GemmOperand& A, const GemmOperand& B, const torch::Tensor& C_in,
               torch::Tensor& C_out, double alpha, double beta, int tile_cfg) {
     TORCH_CHECK(A.t.size(0) <= INT32_MAX && A.t.size(1) <= INT32_MAX && B.t.size(1) <= INT32_MAX,
@@ -105,9 +105,8 @@ void run_gemm(const GemmOperand& A, const GemmOperand& B, const torch::Tensor& C
                                       M, N, K, tile_cfg);
     torch::Tensor ws = workspace_for(ws_bytes, A.t);
     const float* cin = C_in.defined() ? C_in.data_ptr<float>() : nullptr;
-    const int64_t ldcin = C_in.defined() ? C_in.stride(0) : N;
     int rc = wmma_gemm_f16f32_view(A.t.data_ptr(), A.ld, A.trans, B.t.data_ptr(), B.ld, B.trans, cin,
-                                   ldcin, C_out.data_ptr<float>(), C_out.stride(0), M, N, K,
+                                   N, C_out.data_ptr<float>(), N, M, N, K,
                                    static_cast<float>(alpha), static_cast<float>(beta), tile_cfg,
                                    ws.defined() ? ws.data_ptr() : nullptr, ws_bytes,
                                    current_stream(A.t));
@@ -793,11 +792,11 @@ torch::Tensor matmul_int4_fused(torch::Tensor A, torch::Tensor fused, int64_t gr
                           torch::dtype(half_out ? torch::kFloat16 : torch::kFloat32).device(A.device()));
     int rc;
     if (half_out)
-        rc = wmma_w4a16_gemm_f16out(A.data_ptr(), A.stride(0), fused.data_ptr<int32_t>(), nullptr,
+        rc = wmma_w4a16_gemm_f16out(A.data_ptr(), K, fused.data_ptr<int32_t>(), nullptr,
                                     nullptr, WMMA_W4_FUSED, M, (int)N, (int)K, (int)group_size,
                                     Y.data_ptr(), Y.stride(0), nullptr, 0, current_stream(A));
     else
-        rc = wmma_w4a16_gemm(A.data_ptr(), A.stride(0), fused.data_ptr<int32_t>(), nullptr, nullptr,
+        rc = wmma_w4a16_gemm(A.data_ptr(), K, fused.data_ptr<int32_t>(), nullptr, nullptr,
                              WMMA_W4_FUSED, M, (int)N, (int)K, (int)group_size, Y.data_ptr<float>(),
                              Y.stride(0), nullptr, 0, current_stream(A));
     check_status(rc, "wmma_w4a16_gemm");
@@ -868,13 +867,13 @@ torch::Tensor matmul_int4(torch::Tensor A, torch::Tensor packed, torch::Tensor s
     torch::Tensor ws = workspace_for(ws_bytes, A);
     int rc;
     if (half_out)
-        rc = wmma_w4a16_gemm_f16out(A.data_ptr(), A.stride(0), packed.data_ptr<int32_t>(),
+        rc = wmma_w4a16_gemm_f16out(A.data_ptr(), K, packed.data_ptr<int32_t>(),
                                     scales.data_ptr(), zeros.data_ptr(), zfmt, M, (int)N, (int)K,
                                     (int)group_size, Y.data_ptr(), Y.stride(0),
                                     ws.defined() ? ws.data_ptr() : nullptr, ws_bytes,
                                     current_stream(A));
     else
-        rc = wmma_w4a16_gemm(A.data_ptr(), A.stride(0), packed.data_ptr<int32_t>(),
+        rc = wmma_w4a16_gemm(A.data_ptr(), K, packed.data_ptr<int32_t>(),
                              scales.data_ptr(), zeros.data_ptr(), zfmt, M, (int)N, (int)K,
                              (int)group_size, Y.data_ptr<float>(), Y.stride(0),
                              ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, current_stream(A));
