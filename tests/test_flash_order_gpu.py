@@ -77,6 +77,32 @@ def test_varlen_rows_outside_sequences(wo, cu, longest):
                 assert torch.count_nonzero(x[inside]) > 0
 
 
+# Many gaps (three times the 64 that one workgroup looks at), and one that is most of a tensor
+# larger than one sweep of every workgroup.
+@pytest.mark.parametrize("starts,length,total", [(range(3, 3000, 16), 8, 3010), ((5,), 40, 30000)])
+def test_varlen_many_and_large_gaps(wo, starts, length, total):
+    report("varlen_many_and_large_gaps", total=total)
+    h, hkv, d = 4, 2, 64
+    cu, longest = list(starts) + [starts[-1] + length], length  # 16 apart, 8 rows of each taken
+    g = torch.Generator(device="cuda").manual_seed(13)
+    q, do = (torch.randn(total, h, d, generator=g, device="cuda").half() for _ in range(2))
+    k, v = (torch.randn(total, hkv, d, generator=g, device="cuda").half() for _ in range(2))
+    c = torch.tensor(cu, dtype=torch.int32, device="cuda")
+    rows = torch.cat([torch.arange(s, s + length) for s in starts]).cuda()
+    near = torch.arange(len(starts) + 1, dtype=torch.int32, device="cuda") * length
+    o, lse = wo.flash_attention_varlen_forward(q, k, v, c, c, longest, longest, True)
+    on, lsen = wo.flash_attention_varlen_forward(q[rows], k[rows], v[rows], near, near, longest, longest, True)
+    junk = [torch.full_like(x, float("nan")) for x in (q, k, v)]
+    del junk
+    got = wo.flash_attention_varlen_backward(do, q, k, v, o, lse, c, c, longest, longest, True)
+    ref = wo.flash_attention_varlen_backward(do[rows], q[rows], k[rows], v[rows], on, lsen, near, near,
+                                             longest, longest, True)
+    for x, y in zip(got, ref):
+        want = torch.zeros_like(x)
+        want[rows] = y
+        assert torch.equal(x, want)
+
+
 # Grouped heads over few key blocks: the group's query heads in parts, added per sequence.
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("lens,h,hkv,d", [([300, 0, 77], 8, 2, 64), ([129], 16, 1, 128), ([64, 200], 6, 2, 256)])
