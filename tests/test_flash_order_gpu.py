@@ -24,6 +24,7 @@ BATCHES = {
     "empty": [0, 300, 0, 0, 65, 0],
     "wave": [17] * 63 + [520],
     "past_wave": [(37 * i) % 90 for i in range(64)] + [400, 0, 3, 261],
+    "past_wave_long": [(37 * i) % 90 for i in range(64)] + [1100, 0, 3, 261],
     "long": [700, 1500, 90, 0, 1000, 1281],
     "two_waves": [(11 * i) % 23 for i in range(130)] + [300],
 }
@@ -123,9 +124,11 @@ def test_varlen_group_parts(wo, lens, h, hkv, d, causal):
         assert torch.equal(got, again)
 
 
-# The order's rule: a group's parts count towards the grid (16 / 2 heads), and whole rows of 32
-# heads keep their plain order without a causal mask.
-@pytest.mark.parametrize("lens,h,hkv,d", [([700, 1300, 40, 300], 16, 2, 128), ([600, 1100, 70], 32, 32, 64)])
-def test_varlen_order_rule(wo, lens, h, hkv, d):
-    report("varlen_order_rule", lens=lens, h=h, hkv=hkv, d=d)
-    test_varlen_group_parts(wo, lens, h, hkv, d, False)
+# The same at batches on both sides of the order's rule (its lines: test_flash_sched.py): the
+# parts of a group, whole rows of 32 heads.
+@pytest.mark.parametrize("lens,h,hkv,d", [([700, 1300, 40, 300], 16, 2, 128), ([600, 1100, 70], 32, 32, 64),
+                                          ([600, 1100, 70, 300], 32, 32, 64)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_varlen_parts_and_head_rows(wo, lens, h, hkv, d, causal):
+    report("varlen_parts_and_head_rows", lens=lens, h=h, hkv=hkv, d=d, causal=causal)
+    test_varlen_group_parts(wo, lens, h, hkv, d, causal)

@@ -75,7 +75,7 @@ __device__ __forceinline__ int varlen_len(const int* cu, int b, int total, int l
 // the blocks of one weight are a run: [nb - at_least(t), nb - at_least(t + 1)) of the query
 // blocks, [at_least(t + 1), at_least(t)) of the key blocks.
 template <bool KV, bool CAUSAL, int BLOCK>
-__device__ __forceinline__ int varlen_at_least(int owned, int other, int t) {
+__host__ __device__ __forceinline__ int varlen_at_least(int owned, int other, int t) {
     const int nb = (owned + BLOCK - 1) / BLOCK, w = (other + BLOCK - 1) / BLOCK;
     if (t <= 0) return nb;
     if (t > w) return 0;
@@ -150,18 +150,27 @@ __device__ __forceinline__ bool varlen_item(const int* cu_q, const int* cu_k, in
 }
 
 // Whether a varlen grid of B sequences by `heads`, `blocks` per longest sequence and `parts`
-// workgroups per block takes its items in that order.  Where every workgroup has a CU at once,
-// or a few short sequences finish before an uneven engine matters, the search would be a
-// visible part of them (eight sequences of 33 to 966 tokens, 8 heads: 32.6 us in plain order,
-// 33.2 searched; five of at most 322, 40 heads: 21.1 and 21.8).  The parts count: 16 / 2 heads,
-// 1885, 2714, 371 and 949 tokens in 3 parts are 528 ids, the longest sequence's on one XCD
-// (dK/dV 584 us in plain order, 246 in this one).  Without a causal mask, whole rows of 32
-// heads load the engines evenly as they are, and ran faster mixed than heaviest first (32 heads,
-// forward / dQ / dK/dV: 1945 and 276 tokens, D = 64, 61 / 75 / 90 us against 67 / 81 / 93; 1500,
-// 1500, 900 and 300, D = 128, 123 / 161 / 216 against 119 / 155 / 239).
+// workgroups per block takes its items in that order.  Where every workgroup has a CU at once
+// the search would be a visible part of them (eight sequences of 33 to 966 tokens, 8 heads: 32.6
+// us in plain order, 33.2 searched; five of at most 322, 40 heads: 21.1 and 21.8).  The parts
+// count: 16 / 2 heads, 1885, 2714, 371 and 949 tokens in 3 parts are 528 ids, the longest
+// sequence's on one XCD (dK/dV 584 us in plain order, 246 in this one).
+// The search takes about 0.5 us for 64 sequences and 0.4 for every 64 more, of every workgroup:
+// only where the longest sequence has blocks enough for it.  40 heads, D = 64, forward in plain
+// order and searched: 100 sequences of 16 to 200 tokens 83 and 101 us, 256 of 100 to 520 694 and
+// 841, 600 of at most 371 667 and 1406; on this side of the line 64 of 300 to 760 398 and 399, 65
+// of 200 to 1500 637 and 624, 16 of 400 to 3000 566 and 502 (backward 1888 and 1421).
+// Whole rows of 32 heads load the engines evenly as they are.  With a causal mask, where the
+// plain grid goes heaviest block first too, the search then only costs: 32 and 64 heads, D = 64
+// and 128, 20 batches of 3 to 40 sequences, forward 2% and backward 1% slower searched (six of
+// 100 to 2000 tokens: 56.9 and 59.1 us), none more than 3% faster.  Without one it pays but for the
+// fewest sequences (32 heads, D = 64, 1945 and 276 tokens: forward 61 us in plain order, 67
+// searched; three of 500 to 4000 109 and 111): over eleven batches of 4 to 24 the forward took 0
+// to 15% less searched.
 inline bool varlen_ordered(int64_t B, int64_t heads, int64_t blocks, int64_t parts, bool causal) {
-    if (!causal && heads % 32 == 0) return false;
-    return B * heads * blocks * parts > (blocks > 2 ? 256 : 1024);
+    if (heads % 32 == 0 && (causal || B < 4)) return false;
+    const int64_t passes = (B + 63) / 64;  // 64 sequences each
+    return blocks >= (passes == 1 ? 3 : 2 * passes) && B * heads * blocks * parts > 256;
 }
 
 // Workgroups that a varlen grid needs for its items: no more than max_len / block per
