@@ -78,6 +78,28 @@ def test_varlen_rows_outside_sequences(wo, cu, longest):
                 assert torch.count_nonzero(x[inside]) > 0
 
 
+# No query head, or no query row, attends to the keys: their gradients are zero.
+@pytest.mark.parametrize("h,total_q", [(0, 30), (4, 0)])
+def test_gradients_without_queries(wo, h, total_q):
+    report("gradients_without_queries", h=h, total_q=total_q)
+    half = dict(dtype=torch.half, device="cuda")
+    q, k = torch.zeros(total_q, h, 64, **half), torch.ones(30, 2, 64, **half)
+    cq = torch.tensor([0, total_q], dtype=torch.int32, device="cuda")
+    ck = torch.tensor([0, 30], dtype=torch.int32, device="cuda")
+    for dense in (False, True):
+        junk = [torch.full_like(k, float("nan")) for _ in range(8)]
+        del junk
+        if dense:
+            Q, K = q.transpose(0, 1)[None], k.transpose(0, 1)[None]
+            O, lse = wo.flash_attention_forward(Q, K, K)
+            grads = wo.flash_attention_backward(Q, Q, K, K, O, lse)
+        else:
+            O, lse = wo.flash_attention_varlen_forward(q, k, k, cq, ck, total_q, 30)
+            grads = wo.flash_attention_varlen_backward(q, q, k, k, O, lse, cq, ck, total_q, 30)
+        for x in grads:
+            assert torch.equal(x, torch.zeros_like(x))
+
+
 # Many gaps (three times the 64 that one workgroup looks at), and one that is most of a tensor
 # larger than one sweep of every workgroup.
 @pytest.mark.parametrize("starts,length,total", [(range(3, 3000, 16), 8, 3010), ((5,), 40, 30000)])

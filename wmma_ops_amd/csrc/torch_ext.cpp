@@ -409,6 +409,10 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> flash_attention_backward
     auto dQ = torch::empty({B, H, Sq, Dp}, Q.options());
     auto dK = torch::empty({B, K.size(1), K.size(2), Dp}, K.options());
     auto dV = torch::empty_like(dK);
+    if (H == 0) {  // no query heads: the kernels have nothing to run
+        dK.zero_();
+        dV.zero_();
+    }
     // row statistics, plus the grouped-query split's partial dK/dV where it applies
     const size_t ws_bytes = wmma_flash_attn_bwd_split_workspace_size(
         (int)B, (int)H, (int)K.size(1), (int)Sq, (int)K.size(2), (int)Dp, causal ? 1 : 0);
@@ -485,7 +489,7 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> flash_attention_varlen_b
     auto dq = torch::empty({q.size(0), q.size(1), Dp}, q.options());
     auto dk = torch::empty({k.size(0), k.size(1), Dp}, k.options());
     auto dv = torch::empty_like(dk);
-    if (cu_q.size(0) == 1) {  // no sequence: every row lies outside
+    if (cu_q.size(0) == 1 || H == 0) {  // no sequence: every row lies outside; no query heads
         dq.zero_();
         dk.zero_();
         dv.zero_();
