@@ -148,3 +148,24 @@ def test_int4_one_row_at_any_stride(wo):
     p, f = wo.prepack_int4(q), wo.prepack_int4_fused(q, s, z, 128)
     assert torch.equal(wo.matmul_int4(a.t(), p, s, z, 128), wo.matmul_int4(row, p, s, z, 128))
     assert torch.equal(wo.matmul_int4_fused(a.t(), f, 128), wo.matmul_int4_fused(row, f, 128))
+
+
+def test_inplace_on_a_view_of_c(wo):
+    # A strided fp16 view of C's own memory is read before C is written: more tiles than run at
+    # once, each row of tiles writing over the A of the next.
+    report("inplace_on_a_view_of_c")
+    m, n, k = 4096, 5120, 4096
+    g = torch.Generator(device="cuda").manual_seed(10)
+    halves = torch.randn(m, 2 * n, generator=g, device="cuda").half()
+    b = torch.randn(k, n, generator=g, device="cuda").half()
+    a, c = halves[:, 512:512 + k], halves.view(torch.float32)
+    assert c.shape == (m, n) and c.isfinite().all()
+    ref = wo.gemm(a.contiguous(), b, 2.0, 0.5, c.clone())
+    wo.gemm_inplace(a, b, c, 2.0, 0.5)
+    assert torch.equal(c, ref)
+    bt = torch.randn(n, 2 * m, generator=g, device="cuda").half()  # C^T: B a view of it
+    c, b = bt.view(torch.float32), bt[:, :m]
+    a = torch.randn(n, n, generator=g, device="cuda").half()
+    ref = wo.gemm(a, b.contiguous(), 2.0, 0.5, c.clone())
+    wo.gemm_inplace(a, b, c, 2.0, 0.5)
+    assert torch.equal(c, ref)

@@ -94,6 +94,16 @@ void gemm_operands(const torch::Tensor& A, const torch::Tensor& B, GemmOperand* 
     }
 }
 
+// A view of the memory that the GEMM writes is read from a copy.  (A contiguous operand there is
+// read where it is, as the reference does.)
+void copy_if_written(GemmOperand* x, const torch::Tensor& C) {
+    if (x->t.is_contiguous() || x->t.numel() == 0) return;
+    const int64_t last = (x->t.size(0) - 1) * x->t.stride(0) + (x->t.size(1) - 1) * x->t.stride(1);
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(x->t.data_ptr()), x1 = x0 + 2 * (last + 1);
+    const uintptr_t c0 = reinterpret_cast<uintptr_t>(C.data_ptr()), c1 = c0 + 4 * C.numel();
+    if (x0 < c1 && c0 < x1) *x = {x->t.contiguous(), x->t.size(1), false};
+}
+
 // One GEMM through the C-ABI.  C_in may be undefined; C_out preallocated; both contiguous.
 void run_gemm(const GemmOperand& A, const GemmOperand& B, const torch::Tensor& C_in,
               torch::Tensor& C_out, double alpha, double beta, int tile_cfg) {
@@ -210,6 +220,8 @@ void gemm_inplace(torch::Tensor A, torch::Tensor B, torch::Tensor C, double alph
     check_aligned(B, "B must be 16-byte aligned");
     GemmOperand a, b;
     gemm_operands(A, B, &a, &b);
+    copy_if_written(&a, C);
+    copy_if_written(&b, C);
     run_gemm(a, b, C, C, alpha, beta, WMMA_TILE_AUTO);
 }
 
