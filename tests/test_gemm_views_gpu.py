@@ -169,3 +169,22 @@ def test_inplace_on_a_view_of_c(wo):
     ref = wo.gemm(a, b.contiguous(), 2.0, 0.5, c.clone())
     wo.gemm_inplace(a, b, c, 2.0, 0.5)
     assert torch.equal(c, ref)
+
+
+def test_repack_past_one_launch(wo):
+    # Rows off 16 bytes whose copy is more 16-byte chunks than one grid has threads (2^32).
+    m, k = 8300, 4177973
+    if torch.cuda.mem_get_info()[0] < 180 << 30:
+        pytest.skip("needs 180 GiB of GPU memory")
+    report("repack_past_one_launch", m=m, k=k)
+    a = torch.ones(m, k, dtype=torch.half, device="cuda")
+    a[m // 2] = 2
+    a[-1, 1::2] = 3
+    b = torch.ones(k, 8, dtype=torch.half, device="cuda")
+    got = wo.matmul(a, b)
+    ref = torch.full((m, 8), float(k), device="cuda")  # whole numbers below 2^24
+    ref[m // 2] = 2 * k
+    ref[-1] = k + 2 * (k // 2)
+    assert torch.equal(got, ref)
+    del a, b
+    torch.cuda.empty_cache()

@@ -1141,6 +1141,9 @@ void launch_mfma_cfg(int cfg, const GemmArgs& a, hipStream_t stream) {
 
 }  // namespace
 
+// Workgroups of one repack launch: a grid holds fewer than 2^32 threads.
+constexpr int64_t RP_MAX_BLOCKS = ((int64_t)1 << 32) / RP_THREADS - 1;
+
 hipError_t launch_gemm_repack(const GemmRepack& a, const GemmRepack& b, hipStream_t stream) {
     int64_t blocks[2];
     RepackArgs args[2];
@@ -1154,6 +1157,19 @@ hipError_t launch_gemm_repack(const GemmRepack& a, const GemmRepack& b, hipStrea
         blocks[i] = ceil_div64(chunks, RP_THREADS);
     }
     if (blocks[0] + blocks[1] == 0) return hipSuccess;
+    if (blocks[0] + blocks[1] > RP_MAX_BLOCKS) {  // 64 GiB of copies: in parts
+        GemmRepack part[2] = {a, b};
+        if (blocks[0] == 0 || blocks[1] == 0) {  // one operand: half of its rows (one row fits)
+            const GemmRepack& o = blocks[0] ? a : b;
+            part[0] = part[1] = o;
+            part[0].rows = o.rows / 2;
+            part[1].rows -= part[0].rows;
+            part[1].src = static_cast<const f16*>(o.src) + (int64_t)part[0].rows * o.ld;
+            part[1].dst = static_cast<u32x4*>(o.dst) + (int64_t)part[0].rows * ceil_div(o.cols, 8);
+        }
+        const hipError_t e = launch_gemm_repack(part[0], GemmRepack{}, stream);
+        return e != hipSuccess ? e : launch_gemm_repack(part[1], GemmRepack{}, stream);
+    }
     hipLaunchKernelGGL(gemm_repack_kernel, dim3((unsigned)(blocks[0] + blocks[1])), dim3(RP_THREADS),
                        0, stream, args[0], args[1], (int)blocks[0]);
     return hipGetLastError();
