@@ -252,10 +252,8 @@ size_t wmma_w4a16_workspace_size(int M, int N, int K, int group_size);
 #define WMMA_W4_KERNEL_DECODE_MFMA 0  /* M <= 4: one workgroup per 16 columns, matrix pipe */
 #define WMMA_W4_KERNEL_DECODE 1       /* M <= 4, other group sizes: VALU dot products      */
 #define WMMA_W4_KERNEL_GEMV_SPLIT 2   /* M <= 4, narrow N: 32 columns per workgroup, split-K */
-#define WMMA_W4_KERNEL_MFMA 3         /* other shapes: tiled MFMA kernel; group_size 32 and 64
-                                         with M <= 32: the skinny kernel, group parameters
-                                         loaded per lane                                   */
-#define WMMA_W4_KERNEL_SKINNY 4       /* 4 < M <= 32: 32/64 columns per workgroup, matrix pipe */
+#define WMMA_W4_KERNEL_MFMA 3         /* other shapes: tiled MFMA kernel                     */
+#define WMMA_W4_KERNEL_SKINNY 4       /* M <= 32: 16-64 columns per workgroup, matrix pipe   */
 #define WMMA_W4_KERNEL_GEMM 5         /* M > 32: LDS-DMA MFMA GEMM                           */
 #define WMMA_W4_KERNEL_ROWS 6         /* M > 4, short K or wide N: 16/32 rows x 16-64
                                          columns per workgroup over all of K, no LDS ring,

@@ -342,8 +342,10 @@ def test_w4a16_plan_make(lib):
     assert plan(33, 14336, 4096)[0] == 5               # LDS-DMA GEMM beyond 32 rows ...
     assert plan(64, 4096, 4608, 384)[0] == 3           # ... for group sizes 2^j only
     assert plan(2048, 14336, 4096)[:2] == (5, 1)
-    assert plan(16, 14336, 4096, 64)[0] == 3           # G not 128 * 2^j: older tiled kernel
-    assert plan(16, 14336, 4608, 384)[0] == 3
+    assert plan(16, 14336, 4096, 64)[0] == 4           # G = 32, 64: the skinny kernel too
+    assert plan(2, 512, 11008, 32)[0] == 4
+    assert plan(4, 4096, 14336, 32)[0] == 0            # ... and the decode kernel
+    assert plan(16, 14336, 4608, 384)[0] == 3          # G not 32 * 2^j: older tiled kernel
     for M, N, K, G in [(5, 1024, 4224, 128), (17, 352, 1536, 256), (2048, 14336, 4096, 128)]:
         k, s, kps, ws = plan(M, N, K, G)
         assert kps * (s - 1) < K <= kps * s

@@ -87,9 +87,8 @@ enum W4A16Kind {
     W4_DECODE_MFMA = 0,  // M <= 4, G = 32 * 2^j: one workgroup per 16 columns, matrix-pipe dots
     W4_DECODE = 1,       // M <= 4: one workgroup per 16 columns, VALU dots
     W4_GEMV_SPLIT = 2,   // M <= 4, other shapes: 32 columns per workgroup, K split + reduce
-    W4_MFMA = 3,         // larger M, other shapes: tiled MFMA kernel, K split + reduce when few
-                         // tiles; G = 32 and 64 at M <= 32: the skinny kernel's FINE form
-    W4_SKINNY = 4,       // M <= 32, G = 128 * 2^j: 16-64 columns per workgroup, K split + reduce when few tiles
+    W4_MFMA = 3,         // larger M, other shapes: tiled MFMA kernel, K split + reduce when few tiles
+    W4_SKINNY = 4,       // M <= 32, G = 32 * 2^j: 16-64 columns per workgroup, K split + reduce when few tiles
     W4_GEMM = 5,         // M > 32: LDS-DMA MFMA GEMM, K split + reduce when few tiles
     W4_ROWS = 6,         // M > 4: row groups x column groups, register-staged, no LDS ring
 };
@@ -98,8 +97,7 @@ struct W4A16Plan {
     int kind;         // W4A16Kind
     int split;        // K partitions (1: no workspace)
     int k_per_split;  // multiple of 64 (and of G when split > 1)
-    int big = 0;      // W4_GEMM: tile (W4G_TILE_*); W4_SKINNY, W4_ROWS and the FINE form
-                      // under W4_MFMA: 16-column slices per workgroup (W4_MFMA: 0, the tiles)
+    int big = 0;      // W4_GEMM: tile (W4G_TILE_*); W4_SKINNY, W4_ROWS: 16-column slices per workgroup
     int mb = 0;       // W4_ROWS: 16-row blocks per workgroup
 };
 

@@ -2210,12 +2210,14 @@ bool w4a16_narrow_skinny(int M, int N, int K, int num_cus) {
 //                pass) only when fewer than 2*CUs workgroups would exist.
 //   skinny       4 < M <= 32 (and the narrow, long-K M <= 4 shapes) with G = 32 * 2^j: 16,
 //                32 or 64 columns per workgroup, K split (plus a reduce pass) only when the
-//                tiles alone give under half a workgroup per CU.  G = 32 and 64 report
-//                W4_MFMA (slices in `big`).
+//                tiles alone give under half a workgroup per CU.
 //   G = 32 and 64 on these two and on rows (M <= 32), us at G = 64, the kernels below in
 //   their place -> these: M = 1, N = 14336, K = 4096 8.9 -> 7.7; M = 4, N = 4096, K = 14336
 //   26.6 -> 9.1; M = 16, N = 14336, K = 4096 27.2 -> 10.1; M = 32, N = K = 4096 13.6 -> 6.7.
-//   What bounds them at M <= 2 is the per-weight dequantisation (G = 128: 5.9).
+//   What bounds them at M <= 2 is the per-weight dequantisation (G = 128: 5.9).  Forming the
+//   weight as the definition rounds it takes the error against 64 bits at M <= 4 from 2.0e-4
+//   (VALU decode) to 1.6e-7 at K = 4096; where the split GEMV ran, which rounds it too, from
+//   1.1e-7 to 1.5e-7 at K = 1024 and 2.0e-7 to 2.8e-7 at 14336, the order of the fp32 sum.
 //   gemm         M > 32 with G a power of two: LDS-DMA MFMA GEMM (tile below), K split
 //                (plus a reduce pass) only when the tiles cannot fill the chip.
 //   rows         4 < M <= 1024 with G = 128 * 2^j (M <= 32: 32 * 2^j) where the launch
@@ -2251,7 +2253,7 @@ W4A16Plan w4a16_plan(int M, int N, int K, int G, int num_cus, bool aligned) {
             return pl;
         }
         pl.big = nh;
-        pl.kind = G >= 128 ? W4_SKINNY : W4_MFMA;
+        pl.kind = W4_SKINNY;
         pl.k_per_split = SK_NW * u * 128;
         pl.split = ceil_div(K, pl.k_per_split);
         return pl;
@@ -2375,9 +2377,10 @@ hipError_t launch_w4a16_zf(const W4Args& a, const W4A16Launch& w, hipStream_t st
         else
             launch_rows<ZF, 2, 4>(a, grid, stream);
     } else if (pl.kind == W4_SKINNY) {
-        launch_skinny<ZF, false>(a, pl, stream);
-    } else if (pl.kind == W4_MFMA && pl.big > 0) {
-        launch_skinny<ZF, true>(a, pl, stream);
+        if (a.G < 128)
+            launch_skinny<ZF, true>(a, pl, stream);
+        else
+            launch_skinny<ZF, false>(a, pl, stream);
     } else if (pl.kind == W4_GEMV_SPLIT) {
         hipLaunchKernelGGL((w4a16_gemv_kernel<ZF>), dim3(ntiles, pl.split), dim3(GV_NW * kWave), 0,
                            stream, a);
