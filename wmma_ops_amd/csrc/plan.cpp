@@ -105,8 +105,9 @@ static double skinny_nt_time_us(const wmma_gemm_plan& p, int M, int N, int K, in
 // The plan with the shortest modelled time: every tile with K splits 1, 2, 4, 8, 16 (a
 // split only from K = 2048, at least 256 of K per part, and only while the workgroups fit
 // one wave of the CUs), and for M <= 32 the streaming kernel with splits up to K / 256.
-// Over the fitted shapes the choice costs 0.65% more time than the fastest plan of each
-// shape (the previous heuristics: 14%), and 0.8% on a second sweep of 63 shapes.
+// Over the fitted shapes the choice cost 0.65% more time than the fastest plan of each
+// shape (the previous heuristics: 14%), and 0.8% on a second sweep of 63 shapes, with four-wave
+// 128x128 and 256x128 tiles; with those of now 1.5% over 80 random shapes of 17 to 256 rows.
 static wmma_gemm_plan model_plan(int M, int N, int K, int num_cus, size_t max_ws,
                                  bool skinny = true) {
     wmma_gemm_plan best{};

@@ -21,7 +21,8 @@ constexpr TileShape kTiles[WMMA_TILE_COUNT] = {
     {64, 64, 2, 2},    // 0: wave tile 32x32
     {128, 64, 4, 2},   // 1: wave tile 32x32 (8 waves; 5-9% faster than 4 waves of 64x32)
     {256, 64, 4, 1},   // 2: wave tile 64x64
-    {128, 128, 2, 4},  // 3: wave tile 64x32 (8 waves: 0-5% faster than 4 of 64x64)
+    {128, 128, 2, 4},  // 3: wave tile 64x32 (8 waves: 0-5% faster than 4 of 64x64 at K to 8192,
+                       //    128 rows at K = 14336 unsplit or in two parts 1-4% slower)
     {256, 128, 4, 2},  // 4: wave tile 64x64 (8 waves: 3-12% faster than 4 of 128x64)
     {256, 256, 2, 4},  // 5: wave tile 128x64 (8 waves, two per SIMD)
 };
@@ -38,7 +39,10 @@ inline int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Launch model for M <= kModelMaxM, fitted on MI355X (256 CUs) to the autotuner's timings
 // of every plan (6 tiles x splits 1-16, the streaming kernel with splits 1-32) at 819
-// shapes, M = 1-768, N = 512-14336, K = 512-14336.  A workgroup streams its operand bytes
+// shapes, M = 1-768, N = 512-14336, K = 512-14336, when the 128x128 and 256x128 tiles ran four
+// waves; it has served M to 256 since the model below.  With the tiles of now its choices take
+// 1.5% more than the fastest plan of each of 80 random shapes (M = 17-256), at worst 1.2 times
+// (80 x 768 x 1664 unsplit, 12.4 us; 64x64 in seven parts 10.3).  A workgroup streams its operand bytes
 // (the rows of A that exist plus the tile's columns of B, over its K range) at a per-CU
 // rate, or is held by its MFMA work, whichever is longer, plus a fixed cost; the launch
 // takes as many such times as it has waves of workgroups (one per CU), at least the HBM
