@@ -25,8 +25,9 @@ def _case(wo, B, H, Hkv, Sq, Sk, D, scale=-1.0, spread=1.0):
 
 # Keys: one, around a step (32), around one step per wave (128) and a split; rows per
 # key/value head: 1, both sides of a 16-row block, the most (32) and one more (the general
-# kernel); every head-dim kernel and head dims that do not fill it.
-@pytest.mark.parametrize("Sk", [1, 31, 33, 127, 129, 260, 1025, 5000])
+# kernel, which also takes over 16 rows against at most 128 keys at D > 64); every head-dim
+# kernel and head dims that do not fill it.
+@pytest.mark.parametrize("Sk", [1, 31, 33, 127, 128, 129, 260, 1025, 5000])
 @pytest.mark.parametrize("H,Hkv,Sq", [(2, 2, 1), (15, 1, 1), (8, 1, 2), (17, 1, 1), (8, 1, 4), (33, 1, 1)])
 def test_decode_rows_and_keys(wo, H, Hkv, Sq, Sk):
     report("decode_rows_and_keys", H=H, Hkv=Hkv, Sq=Sq, Sk=Sk)

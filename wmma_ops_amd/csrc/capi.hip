@@ -861,7 +861,7 @@ static int flash_fwd_run(const void* Q, AttnStrides q, const void* K, AttnStride
     f.k = k;
     f.v = v;
     flash_pack_groups(causal, &f.H, f.Hkv, &f.Sq, &f.q);
-    const bool decode = f.H == f.Hkv && flash_decode_takes(f.Sq, causal != 0);
+    const bool decode = f.H == f.Hkv && flash_decode_takes(f.Sq, Sk, D, causal != 0);
     if (workspace) {
         int split;
         const size_t need = flash_fwd_split(B, f.H, Hkv, f.Sq, Sk, D, decode, &split);
@@ -896,8 +896,8 @@ static size_t flash_fwd_strided_workspace(AttnStrides q, int B, int H, int Hkv, 
                                           int causal) {
     flash_pack_groups(causal, &H, Hkv, &Sq, &q);
     int split;
-    return flash_fwd_split(B, H, Hkv, Sq, Sk, D, H == Hkv && flash_decode_takes(Sq, causal != 0),
-                           &split);
+    return flash_fwd_split(B, H, Hkv, Sq, Sk, D,
+                           H == Hkv && flash_decode_takes(Sq, Sk, D, causal != 0), &split);
 }
 
 size_t wmma_flash_attn_fwd_workspace_size(int B, int H, int Hkv, int Sq, int Sk, int D,

@@ -166,9 +166,10 @@ hipError_t launch_flash_combine(const float* o_part, const float* ml_part, int s
                                 int D, void* O, float* lse, hipStream_t stream);
 
 // Decoding shapes (flash_decode.hip): dense, not causal, at most 32 query rows per key/value
-// head after the query heads of a group are packed (f.H key/value heads of f.Sq rows).
+// head after the query heads of a group are packed (f.H key/value heads of f.Sq rows), but for
+// the shortest keys under more than 16.
 // kv_split / workspace as for launch_flash_fwd, sized by flash_decode_workspace_bytes.
-bool flash_decode_takes(int Sq, bool causal);
+bool flash_decode_takes(int Sq, int Sk, int D, bool causal);
 int flash_decode_split(int64_t units, int Sq, int Sk, int D, int num_cus);
 size_t flash_decode_workspace_bytes(int64_t units, int Sq, int Sk, int D, int split);
 hipError_t launch_flash_decode(const FlashLaunch& f, hipStream_t stream);
